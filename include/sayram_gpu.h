@@ -110,9 +110,11 @@ typedef struct {
                            levels (9-point operators); 0 selects the defaults
                            16, 160, 16, 768. */
   int fuse_cells;       /* the V-cycle levels of an instance from its first level
-                           of at most fuse_cells cells down run in one fused
-                           launch per instance (post-smoothing schedules);
-                           0 selects 1024, the maximum (a level is kept in
+                           of at most fuse_cells cells and sides of at most 64
+                           down run in one fused launch per instance (post-
+                           smoothing schedules, with or without an x-line
+                           pre-sweep); 0 selects 1024, the maximum with FP64
+                           V-cycles (4096 with FP32 ones; levels are kept in
                            LDS); -1 disables. Like line_tiles it changes the
                            rounding of those line solves. */
   int streams;          /* 2: the tile shapes of one finest-level line sweep

@@ -660,7 +660,8 @@ int Batch::fuse_level(const InstDev &I) const {
   // the fused cycle runs post-smoothing, optionally after an x-line pre-sweep
   if (opts.fuse_cells < 0 || ((opts.smoother | opts.coarse_smoother) & 2)) return I.nlev;
   for (int l = 0; l < I.nlev; ++l)
-    if ((long long)I.lev[l].nx * I.lev[l].ny <= opts.fuse_cells) return l;
+    if (std::max(I.lev[l].nx, I.lev[l].ny) <= kFuseSide && I.lev[l].nx * I.lev[l].ny <= opts.fuse_cells)
+      return l;
   return I.nlev;
 }
 

@@ -179,11 +179,11 @@ struct LineGrp { int inst; int first; int count; int step; };   // lines first +
 struct FuseMap { int inst; int lev; };    // an instance whose levels from lev down run fused
 
 // The coarse end of a V-cycle runs in one workgroup per instance from the
-// first level with at most fuse_cells cells (the fused coarse cycle; default
-// kFuseCells).
-constexpr int kFuseCells = 1024;
-// the largest fused level an FP32 V-cycle can keep in LDS
-constexpr int kFuseCells32 = 4096;
+// first level with at most fuse_cells cells and no side above kFuseSide (a
+// line is then solved by the lanes of one wave): the fused coarse cycle.
+constexpr int kFuseCells = 1024;     // default, and the largest with FP64 V-cycles
+constexpr int kFuseCells32 = 4096;   // the largest with FP32 V-cycles
+constexpr int kFuseSide = 64;
 // Threads of the per-instance finish kernels (sums of the partials).
 constexpr int kFinThreads = 1024;
 constexpr int kFuseThreads = 1024;

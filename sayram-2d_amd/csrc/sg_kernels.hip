@@ -10,6 +10,7 @@
 // streams over the device cell order of sg_internal.hpp (rows split into their
 // even and odd columns). A cell kernel's work-item K is a storage slot; it
 // decodes (i, j) with cell_ij and finds its x-neighbours with xslot.
+#include "sg_device.hpp"
 #include "sg_kernels.hpp"
 #include "sayram_gpu.h"   // sg_precision values of InstDev::prec
 
@@ -20,27 +21,6 @@ namespace sg {
 
 static constexpr double kEps = DBL_EPSILON;   // gEPS, source/common.h:38
 
-template <typename T> __device__ __forceinline__ T *ptr(void *p) { return static_cast<T *>(p); }
-
-// Element `slot` of an array whose base is uniform across the workgroup, through
-// a 32-bit byte offset in the global address space. The pointers of an
-// instance are read from its table, so without the cast the compiler must use
-// flat accesses, which also count against the LDS counter: every LDS wait would
-// then wait for the global loads in flight too. Cast, the access is
-// base + zext(offset), the scalar-base form of the global loads and stores, and
-// one offset register serves every array of the same element type. Instances
-// hold at most kMaxCells cells, so the offsets of FP64 arrays stay below 2^31.
-template <typename T> __device__ __forceinline__ T ld32(const T *base, uint32_t slot) {
-  using GC = const __attribute__((address_space(1))) char;
-  using GT = const __attribute__((address_space(1))) T;
-  return *(GT *)((GC *)base + slot * (uint32_t)sizeof(T));
-}
-template <typename T> __device__ __forceinline__ void st32(T *base, uint32_t slot, T v) {
-  using GC = __attribute__((address_space(1))) char;
-  using GT = __attribute__((address_space(1))) T;
-  *(GT *)((GC *)base + slot * (uint32_t)sizeof(T)) = v;
-}
-
 // LDS slot of step u of line k in a tile of S steps. A line's steps are stored
 // step-mod-4 major, so when the solve threads, each owning 4 consecutive steps,
 // read their e-th step, consecutive lanes read consecutive words: no bank
@@ -50,38 +30,6 @@ template <typename T> __device__ __forceinline__ void st32(T *base, uint32_t slo
 template <int S> __device__ __forceinline__ int tslot(int k, int u) {
   return k * (S + 4) + (u & 3) * (S / 4 + 1) + (u >> 2);
 }
-
-// Global-address-space view of an array pointer read from the instance table
-// (plain indexing of such a pointer compiles to flat accesses).
-template <typename T> __device__ __forceinline__ __attribute__((address_space(1))) T *gbl(T *p) {
-  return (__attribute__((address_space(1))) T *)p;
-}
-
-// Workgroup barrier for LDS data only: it waits for this thread's LDS
-// accesses but not for its global loads, so tiles prefetched into registers
-// stay in flight across it. Valid where threads exchange data through LDS
-// only (a thread that reloads a global element is the one that stored it).
-__device__ __forceinline__ void lds_barrier() {
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
-  __builtin_amdgcn_s_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
-}
-
-// (i, j) of storage slot K of a level with nx columns (hx = half_x(nx))
-__device__ __forceinline__ void cell_ij(int K, int nx, int hx, int &i, int &j) {
-  j = K / nx;
-  i = xcol(K - j * nx, hx);
-}
-template <typename T> __device__ __forceinline__ const T *cptr(const void *p) {
-  return static_cast<const T *>(p);
-}
-
-// Read-only view of an instance's scalars, for the kernels that do not write
-// them (only the begin and finish kernels do). Through the constant address
-// space the compiler reads these workgroup-uniform values with scalar loads
-// instead of per-lane loads that every later load waits behind.
-typedef const __attribute__((address_space(4))) KScal ConstKScal;
-__device__ __forceinline__ ConstKScal *rsc(const InstDev &I) { return (ConstKScal *)I.sc; }
 
 // ---------------------------------------------------------------------------
 // workgroup reduction of NT threads: wave64 shuffles, then LDS across the
@@ -614,18 +562,6 @@ __global__ void __launch_bounds__(kBlock) k_rap(const InstDev *__restrict__ inst
 // ---------------------------------------------------------------------------
 // multigrid cycle kernels (precision T)
 // ---------------------------------------------------------------------------
-// level-0 vector by id: a Krylov slot (Vec) or an FP32 V-cycle vector (PcVec)
-__device__ __forceinline__ void *vec(const InstDev &I, int id) {
-  return id < kNumVec ? I.kv[id] : (void *)I.pv[id - kNumVec];
-}
-
-template <typename T>
-__device__ __forceinline__ void level_xb(const InstDev &I, int l, int xid, int bid, T *&x,
-                                         const T *&b) {
-  if (l == 0) { x = ptr<T>(vec(I, xid)); b = cptr<T>(vec(I, bid)); }
-  else { x = ptr<T>(I.lev[l].x); b = cptr<T>(I.lev[l].b); }
-}
-
 // LU factors of every line matrix of a level (rows: DIR 0, columns: DIR 1),
 // once per step: lup_t = upper_t / pivot_t, linv_t = 1 / pivot_t with
 // pivot_t = diag_t - lower_t lup_{t-1} (Thomas elimination without pivoting;
@@ -1260,63 +1196,6 @@ template <int ROWS> __device__ __forceinline__ int prolong_count(const Lev &F) {
   return ROWS == 1 ? F.nx * (F.ny >> 1) : ROWS == 2 ? (F.nx - half_x(F.nx)) * F.ny : F.nx * F.ny;
 }
 
-template <typename T, bool ZERO, int ROWS>
-__device__ __forceinline__ void prolong_point(const InstDev &I, int l, int xid, int idx) {
-  const Lev &F = I.lev[l];
-  const Lev &Cl = I.lev[l + 1];
-  const int hx = half_x(F.nx);
-  int K, i, j;
-  if (ROWS == 1) {            // rows 1, 3, ..: nx cells each
-    if (idx >= F.nx * (F.ny >> 1)) return;
-    const int r = idx / F.nx, p = idx - r * F.nx;
-    j = 2 * r + 1; i = xcol(p, hx); K = j * F.nx + p;
-  } else if (ROWS == 2) {     // columns 1, 3, ..: the second half of each row
-    const int no = F.nx - hx;
-    if (idx >= no * F.ny) return;
-    j = idx / no;
-    const int p = hx + (idx - j * no);
-    i = xcol(p, hx); K = j * F.nx + p;
-  } else {
-    K = idx;
-    if (K >= F.nx * F.ny) return;
-    cell_ij(K, F.nx, hx, i, j);
-  }
-  const int I0 = i >> 1, J0 = j >> 1;
-  const int I1 = I0 + 1 < Cl.nx ? I0 + 1 : I0, J1 = J0 + 1 < Cl.ny ? J0 + 1 : J0;
-  const auto xc = gbl(cptr<T>(Cl.x));
-  const int hxc = half_x(Cl.nx);
-  const size_t r0 = (size_t)J0 * Cl.nx, r1 = (size_t)J1 * Cl.nx;
-  const int s0 = xslot(I0, hxc), s1 = xslot(I1, hxc);
-  // Weights of parents outside the coarse grid are zero, and so are the
-  // weights to the parents at I0 + 1 of an even i and at J0 + 1 of an even j
-  // (k_pweights writes exact zeros there): those terms are skipped, so half
-  // of each row's weight runs is not read. Each parity case issues all its
-  // loads before it adds (i's parity is uniform over each half-row).
-  const auto w0 = gbl(cptr<T>(F.pw[0])), w1 = gbl(cptr<T>(F.pw[1]));
-  const auto w2 = gbl(cptr<T>(F.pw[2])), w3 = gbl(cptr<T>(F.pw[3]));
-  T e;
-  if ((i & 1) && (j & 1)) {
-    const T a0 = w0[K], a1 = w1[K], a2 = w2[K], a3 = w3[K];
-    const T c0 = xc[r0 + s0], c1 = xc[r0 + s1], c2 = xc[r1 + s0], c3 = xc[r1 + s1];
-    e = a0 * c0;
-    e += a1 * c1;
-    e += a2 * c2;
-    e += a3 * c3;
-  } else if (i & 1) {
-    const T a0 = w0[K], a1 = w1[K], c0 = xc[r0 + s0], c1 = xc[r0 + s1];
-    e = a0 * c0;
-    e += a1 * c1;
-  } else if (j & 1) {
-    const T a0 = w0[K], a2 = w2[K], c0 = xc[r0 + s0], c2 = xc[r1 + s0];
-    e = a0 * c0;
-    e += a2 * c2;
-  } else {
-    e = xc[r0 + s0];   // injection: the even-even weight is exactly 1
-  }
-  const auto x = gbl(l == 0 ? ptr<T>(vec(I, xid)) : ptr<T>(F.x));
-  x[K] = ZERO ? e : x[K] + e;
-}
-
 // A workgroup takes kEnt map entries. Each entry's chain of dependent reads
 // (map entry, instance, its status, its level's pointers) and then its loads
 // are issued before any entry is computed or stored, so a workgroup has
@@ -1389,294 +1268,6 @@ __global__ void __launch_bounds__(kBlock) k_prolong(const InstDev *__restrict__ 
   }
 }
 
-// ---------------------------------------------------------------------------
-// Fused coarse cycle: the levels of one instance from `lev` (its first level
-// with at most kFuseCells cells) down to its coarsest and back, in one
-// workgroup with barriers between the phases, instead of several launches per
-// level. The cycle is the per-level one: per level on the way down an
-// optional pre-smoothing sweep of x-lines and the restriction of the
-// residual (of b itself without pre-smoothing), the exact line solve of the
-// coarsest level, then per level the prolongation of the lines the first
-// post-sweep reads and the zebra post-sweeps.
-//
-// A level being smoothed lives in LDS (x, and per sweep the line right-hand
-// sides and factors), so only the parallel phases touch global memory: every
-// thread forms the right-hand sides of some cells (b minus the couplings to
-// the other colour's lines) and copies their factors, then one thread per line
-// runs the two Thomas recurrences out of LDS (lines are short here). The line
-// solves are the per-level ones rounded in another order.
-// ---------------------------------------------------------------------------
-template <typename T, int CAP>
-struct FuseLds {
-  T x[CAP];     // x of the level being smoothed
-  T r[CAP];     // line right-hand sides, then d of the forward pass
-  T lo[CAP];    // coupling to the previous cell of the line (0 at t = 0)
-  T inv[CAP];   // 1 / pivot
-  T up[CAP];    // upper / pivot
-};
-
-// Levels of at most SCAP cells are staged into LDS whole (b, the off-diagonal
-// bands and the line factors of both directions) once per level, so that the
-// four sweeps read no global memory; larger levels (up to CAP cells) and FP64
-// levels read them from global memory in each sweep's parallel phase. The
-// variants keep a workgroup's LDS within 80 KB, two workgroups per CU:
-//   FP32: CAP 1024 with SCAP 1024 (72 KB), CAP 2048 with SCAP 512 (66 KB),
-//         CAP 4096 without staging (80 KB);  FP64: CAP 1024 (40 KB).
-enum FuseStageArr { FS_B, FS_W, FS_E, FS_S, FS_N, FS_SW, FS_SE, FS_NW, FS_NE, FS_I0, FS_U0, FS_I1,
-                    FS_U1, FS_COUNT };
-template <typename T, int SCAP> struct FuseStage { T a[FS_COUNT][SCAP > 0 ? SCAP : 1]; };
-
-template <typename T, int NB, int SCAP>
-__device__ void fused_stage(const InstDev &I, int l, int bid, FuseStage<T, SCAP> &G) {
-  const Lev &Lv = I.lev[l];
-  const int nc = Lv.nx * Lv.ny;
-  const auto b = gbl(l == 0 ? cptr<T>(vec(I, bid)) : cptr<T>(Lv.b));
-  for (int K = threadIdx.x; K < nc; K += blockDim.x) {
-    G.a[FS_B][K] = b[K];
-    G.a[FS_W][K] = gbl(cptr<T>(Lv.band[BW]))[K];
-    G.a[FS_E][K] = gbl(cptr<T>(Lv.band[BE]))[K];
-    G.a[FS_S][K] = gbl(cptr<T>(Lv.band[BS]))[K];
-    G.a[FS_N][K] = gbl(cptr<T>(Lv.band[BN]))[K];
-    if (NB == 9) {
-      G.a[FS_SW][K] = gbl(cptr<T>(Lv.band[BSW]))[K];
-      G.a[FS_SE][K] = gbl(cptr<T>(Lv.band[BSE]))[K];
-      G.a[FS_NW][K] = gbl(cptr<T>(Lv.band[BNW]))[K];
-      G.a[FS_NE][K] = gbl(cptr<T>(Lv.band[BNE]))[K];
-    }
-    G.a[FS_I0][K] = gbl(cptr<T>(Lv.linv[0]))[K];
-    G.a[FS_U0][K] = gbl(cptr<T>(Lv.lup[0]))[K];
-    G.a[FS_I1][K] = gbl(cptr<T>(Lv.linv[1]))[K];
-    G.a[FS_U1][K] = gbl(cptr<T>(Lv.lup[1]))[K];
-  }
-}
-
-// One zebra sweep (lines of one colour) of level l. STG: the level's inputs
-// are in G (LDS); otherwise they are read from global memory and the line
-// factors copied to S.lo, S.inv, S.up. Both read the same values and do the
-// same operations.
-template <typename T, int NB, int DIR, bool STG, int CAP, int SCAP>
-__device__ void fused_sweep(const InstDev &I, int l, int bid, int colour, bool zero,
-                            FuseLds<T, CAP> &S, FuseStage<T, SCAP> &G) {
-  const Lev &Lv = I.lev[l];
-  const int nx = Lv.nx, ny = Lv.ny, hx = half_x(nx);
-  const T *b = l == 0 ? cptr<T>(vec(I, bid)) : cptr<T>(Lv.b);
-  const T *lo = cptr<T>(Lv.band[DIR == 0 ? BW : BS]);
-  const T *om = cptr<T>(Lv.band[DIR == 0 ? BS : BW]);
-  const T *op = cptr<T>(Lv.band[DIR == 0 ? BN : BE]);
-  const T *omm = nullptr, *omp = nullptr, *opm = nullptr, *opp = nullptr;
-  if (NB == 9) {
-    omm = cptr<T>(Lv.band[BSW]);
-    omp = cptr<T>(Lv.band[DIR == 0 ? BSE : BNW]);
-    opm = cptr<T>(Lv.band[DIR == 0 ? BNW : BSE]);
-    opp = cptr<T>(Lv.band[BNE]);
-  }
-  const T *inv = cptr<T>(Lv.linv[DIR]);
-  const T *cu = cptr<T>(Lv.lup[DIR]);
-  // staged copies of the same arrays
-  constexpr int gLo = DIR == 0 ? FS_W : FS_S, gOm = DIR == 0 ? FS_S : FS_W;
-  constexpr int gOp = DIR == 0 ? FS_N : FS_E, gOmm = FS_SW, gOmp = DIR == 0 ? FS_SE : FS_NW;
-  constexpr int gOpm = DIR == 0 ? FS_NW : FS_SE, gOpp = FS_NE;
-  constexpr int gInv = DIR == 0 ? FS_I0 : FS_I1, gUp = DIR == 0 ? FS_U0 : FS_U1;
-  auto val = [&](const T *p, int g, uint32_t K) -> T {
-    if constexpr (STG) return G.a[g][K];
-    else return ld32(p, K);
-  };
-  const int n = DIR == 0 ? nx : ny, nperp = DIR == 0 ? ny : nx;
-  const int nl = (nperp - colour + 1) >> 1;   // lines colour, colour + 2, ..
-  auto at = [&](int li, int t) -> uint32_t {
-    return DIR == 0 ? (uint32_t)(li * nx + xslot(t, hx)) : (uint32_t)(t * nx + xslot(li, hx));
-  };
-  for (int idx = threadIdx.x; idx < nl * n; idx += blockDim.x) {
-    const int q = idx / n, t = idx - q * n, li = colour + 2 * q;
-    const uint32_t K = at(li, t);
-    T r = val(b, FS_B, K);
-    if (!zero) {
-      if (li > 0) {
-        r -= val(om, gOm, K) * S.x[at(li - 1, t)];
-        if (NB == 9) {
-          if (t > 0) r -= val(omm, gOmm, K) * S.x[at(li - 1, t - 1)];
-          if (t < n - 1) r -= val(omp, gOmp, K) * S.x[at(li - 1, t + 1)];
-        }
-      }
-      if (li < nperp - 1) {
-        r -= val(op, gOp, K) * S.x[at(li + 1, t)];
-        if (NB == 9) {
-          if (t > 0) r -= val(opm, gOpm, K) * S.x[at(li + 1, t - 1)];
-          if (t < n - 1) r -= val(opp, gOpp, K) * S.x[at(li + 1, t + 1)];
-        }
-      }
-    }
-    S.r[K] = r;
-    if constexpr (!STG) {
-      S.lo[K] = t > 0 ? ld32(lo, K) : T(0);
-      S.inv[K] = ld32(inv, K);
-      S.up[K] = ld32(cu, K);
-    }
-  }
-  __syncthreads();
-  const T *s_lo, *s_inv, *s_up;
-  if constexpr (STG) {
-    s_lo = G.a[gLo]; s_inv = G.a[gInv]; s_up = G.a[gUp];
-  } else {
-    s_lo = S.lo; s_inv = S.inv; s_up = S.up;
-  }
-  for (int q = threadIdx.x; q < nl; q += blockDim.x) {
-    const int li = colour + 2 * q;
-    // (unrolled so that the LDS reads of several steps, which do not depend
-    // on the recurrence, are issued together)
-    T d = T(0);
-#pragma unroll 8
-    for (int t = 0; t < n; ++t) {   // forward: d_t = (r_t - lo_t d_{t-1}) / pivot_t
-      const uint32_t K = at(li, t);
-      const T lv = t > 0 ? s_lo[K] : T(0);
-      d = (S.r[K] - lv * d) * s_inv[K];
-      S.r[K] = d;
-    }
-    T xn = T(0);
-#pragma unroll 8
-    for (int t = n - 1; t >= 0; --t) {   // backward: x_t = d_t - u_t x_{t+1}
-      const uint32_t K = at(li, t);
-      xn = S.r[K] - s_up[K] * xn;
-      S.x[K] = xn;
-    }
-  }
-  __syncthreads();
-}
-
-// x of level l: global -> LDS (load) or LDS -> global (store); ends with a
-// barrier.
-template <typename T, int CAP>
-__device__ void fused_x(const InstDev &I, int l, int xid, FuseLds<T, CAP> &S, bool load) {
-  const auto x = gbl(l == 0 ? ptr<T>(vec(I, xid)) : ptr<T>(I.lev[l].x));
-  const int nc = I.lev[l].nx * I.lev[l].ny;
-  for (int K = threadIdx.x; K < nc; K += blockDim.x) {
-    if (load) S.x[K] = x[K];
-    else x[K] = S.x[K];
-  }
-  __syncthreads();
-}
-
-template <typename T, int NB, bool STG, int CAP, int SCAP>
-__device__ void fused_sweeps(const InstDev &I, int l, int bid, bool post_x, bool post_y,
-                             FuseLds<T, CAP> &S, FuseStage<T, SCAP> &G) {
-  if (post_x) {
-    fused_sweep<T, NB, 0, STG>(I, l, bid, 0, false, S, G);
-    fused_sweep<T, NB, 0, STG>(I, l, bid, 1, false, S, G);
-  }
-  if (post_y) {
-    fused_sweep<T, NB, 1, STG>(I, l, bid, 0, false, S, G);
-    fused_sweep<T, NB, 1, STG>(I, l, bid, 1, false, S, G);
-  }
-}
-
-template <typename T, int NB, int CAP, int SCAP>
-__device__ void fused_smooth(const InstDev &I, int l, int xid, int bid, bool post_x, bool post_y,
-                             FuseLds<T, CAP> &S, FuseStage<T, SCAP> &G) {
-  if constexpr (SCAP > 0) {
-    if (I.lev[l].nx * I.lev[l].ny <= SCAP) {   // uniform over the workgroup
-      fused_stage<T, NB>(I, l, bid, G);   // the barrier of fused_x covers it
-      fused_x<T>(I, l, xid, S, true);
-      fused_sweeps<T, NB, true>(I, l, bid, post_x, post_y, S, G);
-      fused_x<T>(I, l, xid, S, false);
-      return;
-    }
-  }
-  fused_x<T>(I, l, xid, S, true);
-  fused_sweeps<T, NB, false>(I, l, bid, post_x, post_y, S, G);
-  fused_x<T>(I, l, xid, S, false);
-}
-
-// smoother: the finest level's schedule in bits 0-3, the coarser levels' in
-// bits 4-7 (post-smoothing bits and the x-line pre-smoothing bit)
-template <typename T, int CAP, int SCAP>
-__global__ void __launch_bounds__(kFuseThreads) k_coarse_cycle(const InstDev *__restrict__ insts,
-                                                               const FuseMap *__restrict__ map,
-                                                               int xid, int bid, int smoother) {
-  __shared__ FuseLds<T, CAP> S;
-  __shared__ FuseStage<T, SCAP> G;
-  const FuseMap fm = map[blockIdx.x];
-  const InstDev &I = insts[fm.inst];
-  if (rsc(I)->status != ST_ACTIVE) return;
-  const int lf = fm.lev, nl = I.nlev;
-  auto sched = [&](int m) { return m == 0 ? (smoother & 15) : (smoother >> 4); };
-  for (int m = lf; m + 1 < nl; ++m) {
-    const int nc = I.lev[m + 1].nx * I.lev[m + 1].ny;
-    if (sched(m) & 1) {
-      // pre-smoothing with x-lines from x_m = 0 (colour 0 from b alone), x_m
-      // kept for the ascent, then b_{m+1} = R r_m with r_m = b_m - A_m x_m,
-      // which is zero on the odd rows (solved last)
-      if (m == 0) {
-        fused_sweep<T, 5, 0, false>(I, m, bid, 0, true, S, G);
-        fused_sweep<T, 5, 0, false>(I, m, bid, 1, false, S, G);
-      } else {
-        fused_sweep<T, 9, 0, false>(I, m, bid, 0, true, S, G);
-        fused_sweep<T, 9, 0, false>(I, m, bid, 1, false, S, G);
-      }
-      fused_x<T>(I, m, xid, S, false);
-      for (int KC = threadIdx.x; KC < nc; KC += blockDim.x) {
-        if (m == 0) restrict_residual_point<T, 5>(I, m, xid, bid, KC);
-        else restrict_residual_point<T, 9>(I, m, xid, bid, KC);
-      }
-    } else {   // b_{m+1} = R b_m (x_m = 0)
-      for (int KC = threadIdx.x; KC < nc; KC += blockDim.x)
-        restrict_point<T, true>(I, m, xid, bid, KC);
-    }
-    __syncthreads();
-  }
-  {   // exact solve of the coarsest level (x = 0): one row or one column
-    const int c = nl - 1;
-    if (I.lev[c].ny == 1) {
-      if (c == 0) fused_sweep<T, 5, 0, false>(I, c, bid, 0, true, S, G);
-      else fused_sweep<T, 9, 0, false>(I, c, bid, 0, true, S, G);
-    } else {
-      if (c == 0) fused_sweep<T, 5, 1, false>(I, c, bid, 0, true, S, G);
-      else fused_sweep<T, 9, 1, false>(I, c, bid, 0, true, S, G);
-    }
-    fused_x<T>(I, c, xid, S, false);
-  }
-  for (int m = nl - 2; m >= lf; --m) {  // x_m (+)= P x_{m+1}, then post-smoothing
-    const Lev &F = I.lev[m];
-    // schedule of level m: the finest level's (low 4 bits) or the coarser ones'
-    const int sml = sched(m);
-    const bool post_x = sml & 4, post_y = sml & 8;
-    const int rows = prolong_rows(sml);
-    const int np = rows == 1 ? prolong_count<1>(F) : rows == 2 ? prolong_count<2>(F)
-                                                                : prolong_count<0>(F);
-    for (int k = threadIdx.x; k < np; k += blockDim.x) {
-      if (sml & 1) {   // pre-smoothed: the correction is added to x_m
-        if (rows == 1) prolong_point<T, false, 1>(I, m, xid, k);
-        else if (rows == 2) prolong_point<T, false, 2>(I, m, xid, k);
-        else prolong_point<T, false, 0>(I, m, xid, k);
-      } else {
-        if (rows == 1) prolong_point<T, true, 1>(I, m, xid, k);
-        else if (rows == 2) prolong_point<T, true, 2>(I, m, xid, k);
-        else prolong_point<T, true, 0>(I, m, xid, k);
-      }
-    }
-    __syncthreads();
-    if (m == 0) fused_smooth<T, 5>(I, m, xid, bid, post_x, post_y, S, G);
-    else fused_smooth<T, 9>(I, m, xid, bid, post_x, post_y, S, G);
-  }
-}
-
-template <typename T>
-void launch_coarse_cycle(hipStream_t s, const InstDev *d, const FuseMap *m, int n, int xid, int bid,
-                         int smoother, int cap) {
-  if (!n) return;
-  if constexpr (sizeof(T) == 8) {
-    k_coarse_cycle<T, 1024, 0><<<n, kFuseThreads, 0, s>>>(d, m, xid, bid, smoother);
-  } else {
-    if (cap <= 1024) k_coarse_cycle<T, 1024, 1024><<<n, kFuseThreads, 0, s>>>(d, m, xid, bid, smoother);
-    else if (cap <= 2048) k_coarse_cycle<T, 2048, 512><<<n, kFuseThreads, 0, s>>>(d, m, xid, bid, smoother);
-    else k_coarse_cycle<T, 4096, 0><<<n, kFuseThreads, 0, s>>>(d, m, xid, bid, smoother);
-  }
-}
-template void launch_coarse_cycle<double>(hipStream_t, const InstDev *, const FuseMap *, int, int,
-                                          int, int, int);
-template void launch_coarse_cycle<float>(hipStream_t, const InstDev *, const FuseMap *, int, int,
-                                         int, int, int);
-
-// ---------------------------------------------------------------------------
 // ---------------------------------------------------------------------------
 // BiCGSTAB (right-preconditioned), precision T for vectors and sums; the
 // operator is the level-0 5-band matrix of the V-cycle precision.

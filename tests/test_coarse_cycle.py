@@ -1,0 +1,51 @@
+"""The fused coarse cycle at the edges of what one workgroup takes: sides at
+and around powers of two (a line occupies a power-of-two segment of a wave's
+lanes) and around the largest side, strips, single rows and columns."""
+import pytest
+
+import oracle as orc
+import sayram_cases as sc
+import sayram_gpu as sg
+from conftest import rel_l2
+
+SHAPES = [(64, 64), (64, 63), (63, 64), (65, 64), (64, 65), (33, 31), (32, 32), (31, 33), (17, 60),
+          (60, 17), (16, 64), (64, 16), (8, 9), (3, 64), (64, 3), (2, 2), (2, 64), (1, 64), (64, 1),
+          (1, 65), (70, 2), (128, 130)]
+
+
+def _run(precision, smoother, coarse, fuse, steps):
+    b = sg.Batch(sg.make_opts(precision=precision, smoother=smoother, coarse_smoother=coarse,
+                              fuse_cells=fuse))
+    probs = [sc.seeded_case(nx, ny, seed=300 + k, scale=10.0 ** (k % 3 - 1))
+             for k, (nx, ny) in enumerate(SHAPES)]
+    slots = [b.add(p) for p in probs]
+    out, its = [], []
+    for _ in range(steps):
+        b.step(1)
+        out.append([b.f(s) for s in slots])
+        its.append([b.stats(s)["last_iters"] for s in slots])
+    b.close()
+    return probs, out, its
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("precision", [sg.SG_FP64, sg.SG_MIXED, sg.SG_PC32])
+@pytest.mark.parametrize("smoother,coarse", [(0, 0), (13, 13), (12, 12), (5, 4), (9, 8)])
+def test_edges_of_the_fused_cycle(gpu_lib, precision, smoother, coarse):
+    """Every step on the oracle (1e-10, the step's specification), equal to the
+    per-level cycle up to the solve tolerance, and as strong: the two cycles
+    are the same operator up to rounding, so they need the same iterations up
+    to one."""
+    caps = [0] if precision == sg.SG_FP64 else [0, 4096]
+    probs, per_level, its0 = _run(precision, smoother, coarse, -1, 3)
+    for cap in caps:
+        _, fused, its = _run(precision, smoother, coarse, cap, 3)
+        for k, p in enumerate(probs):
+            f = p.f0
+            op = orc.OracleProblem(p)
+            for n in range(3):
+                f = orc.step(op, f)
+                assert rel_l2(fused[n][k], f) <= 1e-10, (SHAPES[k], n)
+                assert rel_l2(fused[n][k], per_level[n][k]) <= 1e-11, (SHAPES[k], n)
+                slack = 1 if precision != sg.SG_MIXED else 3   # MIXED counts inner iterations
+                assert abs(its[n][k] - its0[n][k]) <= slack, (SHAPES[k], n, its[n][k], its0[n][k])
