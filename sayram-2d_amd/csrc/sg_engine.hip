@@ -152,16 +152,17 @@ struct Maps {
   std::vector<BlkMap> cmap[kMaxLev], pmap[kMaxLev];
   std::vector<LineGrp> gfac[kMaxLev][2][kNumTileShapes], gcx[kMaxLev][kNumTileShapes],
       gcy[kMaxLev][kNumTileShapes];
+  // (the sweep maps sw, swx, swy go by sweep shape, the factor maps by tile shape)
   // cycle: restriction into level l, prolongation into level l, sweeps and
   // coarsest solves, and every instance with a fused coarse cycle
   std::vector<BlkMap> rmap[kMaxLev], qmap[kMaxLev];
-  std::vector<LineGrp> sw[kMaxLev][2][2][kNumTileShapes], swx[kMaxLev][kNumTileShapes],
-      swy[kMaxLev][kNumTileShapes];
-  // the 256-thread shapes of one colour's sweep of a 9-point level, in one
-  // map (rows: shapes 2, 1, 0; columns: 4, 0, or 1, 0 with FP64 V-cycles),
+  std::vector<LineGrp> sw[kMaxLev][2][2][kNumSweepShapes], swx[kMaxLev][kNumSweepShapes],
+      swy[kMaxLev][kNumSweepShapes];
+  // the 256-thread tile shapes of one colour's sweep of a 9-point level, in
+  // one map (rows: shapes 2, 1, 0; columns: 4, 0, or 1, 0 with FP64 V-cycles),
   // the first two shapes' group counts, and whether the map and the
-  // 1024-thread shape 3 hold every group of the colour (else the shapes are
-  // launched one by one)
+  // 1024-thread shape 3 hold every tiled group of the colour (else the shapes
+  // are launched one by one)
   std::vector<LineGrp> swm[kMaxLev][2][2];
   int swm_na[kMaxLev][2][2], swm_nb[kMaxLev][2][2];
   bool swm_all[kMaxLev][2][2];
@@ -184,6 +185,30 @@ static int tile_shape(const int (&lim)[4], int n, int dir, int l, bool fp64_vcyc
   if (dir == 0) return n <= lim[1] ? 1 : 2;
   if (n <= lim[3]) return fp64_vcycle ? 1 : 4;
   return (fp64_vcycle && l > 0) ? 1 : 3;
+}
+
+// The default line lengths of the tile shapes (sg_opts.line_tiles).
+static const int kDefaultTiles[4] = {16, 160, 16, 768};
+
+// Shape of a line sweep. With the default line lengths the columns of at most
+// kColLongMax steps are solved in registers, one pass over their data. Longer
+// columns, and every column when the caller set other lengths, go by tile
+// shapes. Like the tile shape it depends only on the line, its level and the
+// options.
+static int sweep_shape(const int (&lim)[4], int n, int dir, int l, bool fp64_vcycle) {
+  if (dir == 1 && lim[2] == kDefaultTiles[2] && lim[3] == kDefaultTiles[3]) {
+    if (n <= kColMax) return kColShape;
+    if (n <= kColLongMax) return kColLongShape;
+  }
+  return tile_shape(lim, n, dir, l, fp64_vcycle);
+}
+// Lines per group of a sweep shape.
+static int sweep_lines(int shape, int n, bool fp64_vcycle) {
+  return shape < kNumTileShapes ? tile_lines(shape) : col_lines(n, fp64_vcycle ? 8 : 4);
+}
+// Rank of a sweep shape by the length of the lines it takes.
+static int sweep_rank(int shape) {
+  return shape == kColLongShape ? 8 : shape == kColShape ? 7 : shape == 3 ? 9 : shape_rank(shape);
 }
 
 // Workgroups are dispatched to the 8 XCDs round-robin (workgroup b on XCD
@@ -235,10 +260,10 @@ struct DevMaps {   // offsets into one device buffer
       ngcy[kMaxLev][kNumTileShapes];
   const BlkMap *rmap[kMaxLev], *qmap[kMaxLev];
   int nrmap[kMaxLev], nqmap[kMaxLev];
-  const LineGrp *sw[kMaxLev][2][2][kNumTileShapes], *swx[kMaxLev][kNumTileShapes],
-      *swy[kMaxLev][kNumTileShapes];
-  int nsw[kMaxLev][2][2][kNumTileShapes], nswx[kMaxLev][kNumTileShapes],
-      nswy[kMaxLev][kNumTileShapes];
+  const LineGrp *sw[kMaxLev][2][2][kNumSweepShapes], *swx[kMaxLev][kNumSweepShapes],
+      *swy[kMaxLev][kNumSweepShapes];
+  int nsw[kMaxLev][2][2][kNumSweepShapes], nswx[kMaxLev][kNumSweepShapes],
+      nswy[kMaxLev][kNumSweepShapes];
   const LineGrp *swm[kMaxLev][2][2];
   int nswm[kMaxLev][2][2], swm_na[kMaxLev][2][2], swm_nb[kMaxLev][2][2];
   bool swm_all[kMaxLev][2][2];
@@ -341,7 +366,7 @@ struct Batch {
   template <typename KT, typename VT> void iteration(bool xstate);
   void count_bytes(const std::vector<int> &part);
   template <typename T> void vcycle(int l, int xid, int bid);
-  template <typename F> void fan_out(const int (&cnt)[kNumTileShapes], F &&launch);
+  template <typename F> void fan_out(const int (&cnt)[kNumSweepShapes], F &&launch);
   int read_counter(int which, int *out);
   int scratch(size_t n);
   int get_f(int slot, double *out);
@@ -394,10 +419,9 @@ static void apply_defaults(sg_opts &o) {
   if (o.streams == 0) o.streams = 1;
   if (o.group_cells == 0) o.group_cells = 1 << 21;
   if (o.warm_start == 0) o.warm_start = 1;
-  const int tiles[4] = {16, 160, 16, 768};
   for (int k = 0; k < 4; ++k) {
-    if (o.line_tiles[k] <= 0) o.line_tiles[k] = tiles[k];
-    if (o.coarse_tiles[k] <= 0) o.coarse_tiles[k] = tiles[k];
+    if (o.line_tiles[k] <= 0) o.line_tiles[k] = kDefaultTiles[k];
+    if (o.coarse_tiles[k] <= 0) o.coarse_tiles[k] = kDefaultTiles[k];
   }
 }
 
@@ -707,22 +731,24 @@ int Batch::rebuild() {
         LineGrp g{c, 0, 1, 1};
         auto &set = ly == 1 ? M.gcx[l][tile_shape(lim, lx, 0, l, f64)]
                             : M.gcy[l][tile_shape(lim, ly, 1, l, f64)];
-        auto &cyc = ly == 1 ? M.swx[l][tile_shape(lim, lx, 0, l, f64)]
-                            : M.swy[l][tile_shape(lim, ly, 1, l, f64)];
+        auto &cyc = ly == 1 ? M.swx[l][sweep_shape(lim, lx, 0, l, f64)]
+                            : M.swy[l][sweep_shape(lim, ly, 1, l, f64)];
         set.push_back(g);
         if (l < lf) cyc.push_back(g);
       } else {
-        // groups of tile_lines(shape) lines of one colour
+        // groups of tile_lines / sweep_lines lines of one colour
         for (int d = 0; d < 2; ++d) {
           const int nl = d == 0 ? ly : lx;          // number of lines
-          const int sh = tile_shape(lim, d == 0 ? lx : ly, d, l, f64);
-          const int per = tile_lines(sh);
-          for (int p = 0; p < 2; ++p)
-            for (int f = p; f < nl; f += 2 * per) {
-              const int cntl = std::min(per, (nl - f + 1) / 2);
-              M.gfac[l][d][sh].push_back({c, f, cntl, 2});
-              if (l < lf) M.sw[l][d][p][sh].push_back({c, f, cntl, 2});
-            }
+          const int n = d == 0 ? lx : ly;
+          const int sh = tile_shape(lim, n, d, l, f64), ss = sweep_shape(lim, n, d, l, f64);
+          const int per = tile_lines(sh), sper = sweep_lines(ss, n, f64);
+          for (int p = 0; p < 2; ++p) {
+            for (int f = p; f < nl; f += 2 * per)
+              M.gfac[l][d][sh].push_back({c, f, std::min(per, (nl - f + 1) / 2), 2});
+            if (l < lf)
+              for (int f = p; f < nl; f += 2 * sper)
+                M.sw[l][d][p][ss].push_back({c, f, std::min(sper, (nl - f + 1) / 2), 2});
+          }
         }
       }
     }
@@ -735,12 +761,12 @@ int Batch::rebuild() {
   // on one XCD; in the factor maps both colours of an instance follow one
   // another in the same way.
   for (int l = 0; l < kMaxLev; ++l)
-    for (int sh = 0; sh < kNumTileShapes; ++sh)
+    for (int sh = 0; sh < kNumSweepShapes; ++sh)
       for (int d = 0; d < 2; ++d) {
         auto len = [&](const LineGrp &g) {
           return d == 0 ? table[g.inst].lev[l].nx : table[g.inst].lev[l].ny;
         };
-        for (int p = 0; p < 3; ++p) {
+        for (int p = 0; p < (sh < kNumTileShapes ? 3 : 2); ++p) {
           auto &w = p < 2 ? M.sw[l][d][p][sh] : M.gfac[l][d][sh];
           std::stable_sort(w.begin(), w.end(),
                            [&](const LineGrp &a, const LineGrp &b) { return len(a) > len(b); });
@@ -785,11 +811,12 @@ int Batch::rebuild() {
     sz(M.cmap[l].size(), sizeof(BlkMap)); sz(M.pmap[l].size(), sizeof(BlkMap));
     sz(M.rmap[l].size(), sizeof(BlkMap)); sz(M.qmap[l].size(), sizeof(BlkMap));
     for (int sh = 0; sh < kNumTileShapes; ++sh) {
-      for (int d = 0; d < 2; ++d) {
-        sz(M.gfac[l][d][sh].size(), sizeof(LineGrp));
-        for (int p = 0; p < 2; ++p) sz(M.sw[l][d][p][sh].size(), sizeof(LineGrp));
-      }
+      for (int d = 0; d < 2; ++d) sz(M.gfac[l][d][sh].size(), sizeof(LineGrp));
       sz(M.gcx[l][sh].size(), sizeof(LineGrp)); sz(M.gcy[l][sh].size(), sizeof(LineGrp));
+    }
+    for (int sh = 0; sh < kNumSweepShapes; ++sh) {
+      for (int d = 0; d < 2; ++d)
+        for (int p = 0; p < 2; ++p) sz(M.sw[l][d][p][sh].size(), sizeof(LineGrp));
       sz(M.swx[l][sh].size(), sizeof(LineGrp)); sz(M.swy[l][sh].size(), sizeof(LineGrp));
     }
     for (int d = 0; d < 2; ++d)
@@ -827,16 +854,19 @@ int Batch::rebuild() {
         auto &v = M.gfac[l][d][sh];
         dmn.gfac[l][d][sh] = (const LineGrp *)put(v.data(), v.size(), sizeof(LineGrp));
         dmn.ngfac[l][d][sh] = (int)v.size();
-        for (int p = 0; p < 2; ++p) {
-          auto &w = M.sw[l][d][p][sh];
-          dmn.sw[l][d][p][sh] = (const LineGrp *)put(w.data(), w.size(), sizeof(LineGrp));
-          dmn.nsw[l][d][p][sh] = (int)w.size();
-        }
       }
       dmn.gcx[l][sh] = (const LineGrp *)put(M.gcx[l][sh].data(), M.gcx[l][sh].size(), sizeof(LineGrp));
       dmn.ngcx[l][sh] = (int)M.gcx[l][sh].size();
       dmn.gcy[l][sh] = (const LineGrp *)put(M.gcy[l][sh].data(), M.gcy[l][sh].size(), sizeof(LineGrp));
       dmn.ngcy[l][sh] = (int)M.gcy[l][sh].size();
+    }
+    for (int sh = 0; sh < kNumSweepShapes; ++sh) {
+      for (int d = 0; d < 2; ++d)
+        for (int p = 0; p < 2; ++p) {
+          auto &w = M.sw[l][d][p][sh];
+          dmn.sw[l][d][p][sh] = (const LineGrp *)put(w.data(), w.size(), sizeof(LineGrp));
+          dmn.nsw[l][d][p][sh] = (int)w.size();
+        }
       dmn.swx[l][sh] = (const LineGrp *)put(M.swx[l][sh].data(), M.swx[l][sh].size(), sizeof(LineGrp));
       dmn.nswx[l][sh] = (int)M.swx[l][sh].size();
       dmn.swy[l][sh] = (const LineGrp *)put(M.swy[l][sh].data(), M.swy[l][sh].size(), sizeof(LineGrp));
@@ -910,15 +940,15 @@ int Batch::collect_time() {
 // are the critical path) runs on `side`, forked from and joined back into
 // `stream`; the shapes write disjoint lines, so the results do not change.
 // Under stream capture the fork and join become graph edges.
-template <typename F> void Batch::fan_out(const int (&cnt)[kNumTileShapes], F &&launch) {
+template <typename F> void Batch::fan_out(const int (&cnt)[kNumSweepShapes], F &&launch) {
   int nshape = 0, last = -1;
-  for (int sh = 0; sh < kNumTileShapes; ++sh)
+  for (int sh = 0; sh < kNumSweepShapes; ++sh)
     if (cnt[sh]) {
       ++nshape;
-      if (last < 0 || shape_rank(sh) >= shape_rank(last)) last = sh;
+      if (last < 0 || sweep_rank(sh) >= sweep_rank(last)) last = sh;
     }
   if (nshape < 2 || !side) {
-    for (int sh = 0; sh < kNumTileShapes; ++sh)
+    for (int sh = 0; sh < kNumSweepShapes; ++sh)
       if (cnt[sh]) launch(stream, sh);
     return;
   }
@@ -927,7 +957,7 @@ template <typename F> void Batch::fan_out(const int (&cnt)[kNumTileShapes], F &&
   note(hipStreamWaitEvent(side, ev_fork, 0));
   launch(side, last);
   note(hipEventRecord(ev_join, side));
-  for (int sh = 0; sh < kNumTileShapes; ++sh)
+  for (int sh = 0; sh < kNumSweepShapes; ++sh)
     if (cnt[sh] && sh != last) launch(stream, sh);
   note(hipStreamWaitEvent(stream, ev_join, 0));
 }
@@ -938,12 +968,24 @@ template <typename T> void Batch::vcycle(int l, int xid, int bid) {
   const bool pre_x = sm & 1, pre_y = sm & 2, post_x = sm & 4, post_y = sm & 8;
   const int lid = l == 0 ? 2 : 3;
   bool zero = true;
+  // the groups of sweep shape sh in one launch
+  auto lines = [&](hipStream_t s, const LineGrp *g, int ng, int dir, int sh, bool z) {
+    if (sh < kNumTileShapes) launch_line<T>(s, d_insts, g, ng, l, dir, sh, z, xid, bid);
+    else launch_cols<T>(s, d_insts, g, ng, l, sh == kColLongShape, z, xid, bid);
+  };
   auto sweep = [&](int dir) {
     for (int p = 0; p < 2; ++p) {
       if (l >= 1 && m.swm_all[l][dir][p]) {
-        // a 9-point level, with one stream or two: the 1024-thread long-column
-        // groups, then every other shape of the colour in one launch (so that
-        // both stream modes run the same kernels and agree bit for bit)
+        // a 9-point level, with one stream or two (so that both stream modes
+        // run the same kernels and agree bit for bit): the register shapes,
+        // longest lines first, the 1024-thread long-column groups, then every
+        // other tile shape of the colour in one launch
+        for (int sh = kNumSweepShapes - 1; sh >= kNumTileShapes; --sh)
+          if (m.nsw[l][dir][p][sh]) {
+            tbegin(lid);
+            lines(stream, m.sw[l][dir][p][sh], m.nsw[l][dir][p][sh], dir, sh, zero);
+            tend(lid);
+          }
         if (m.nsw[l][dir][p][3]) {
           tbegin(lid);
           launch_line<T>(stream, d_insts, m.sw[l][dir][p][3], m.nsw[l][dir][p][3], l, dir, 3,
@@ -959,8 +1001,7 @@ template <typename T> void Batch::vcycle(int l, int xid, int bid) {
       } else {
         fan_out(m.nsw[l][dir][p], [&](hipStream_t s, int sh) {
           tbegin(lid, s);   // one timed interval per kernel dispatch
-          launch_line<T>(s, d_insts, m.sw[l][dir][p][sh], m.nsw[l][dir][p][sh], l, dir, sh, zero,
-                         xid, bid);
+          lines(s, m.sw[l][dir][p][sh], m.nsw[l][dir][p][sh], dir, sh, zero);
           tend(lid, s);
         });
       }
@@ -983,15 +1024,15 @@ template <typename T> void Batch::vcycle(int l, int xid, int bid) {
   if (pre_y) sweep(1);
   const bool pre_zero = zero;
   // exact solve on the coarsest level of the instances that end here
-  for (int sh = 0; sh < kNumTileShapes; ++sh) {
+  for (int sh = 0; sh < kNumSweepShapes; ++sh) {
     if (m.nswx[l][sh]) {
       tbegin(3);
-      launch_line<T>(stream, d_insts, m.swx[l][sh], m.nswx[l][sh], l, 0, sh, true, xid, bid);
+      lines(stream, m.swx[l][sh], m.nswx[l][sh], 0, sh, true);
       tend(3);
     }
     if (m.nswy[l][sh]) {
       tbegin(3);
-      launch_line<T>(stream, d_insts, m.swy[l][sh], m.nswy[l][sh], l, 1, sh, true, xid, bid);
+      lines(stream, m.swy[l][sh], m.nswy[l][sh], 1, sh, true);
       tend(3);
     }
   }

@@ -71,6 +71,22 @@ __host__ __device__ constexpr int ring_tiles(int sh, int tbytes, int nb) {
   }
 }
 
+// The sweeps with the lines in registers (sg_sweeps.hip), as further shapes of
+// the sweep maps: 5 columns of at most 512 steps, 6 columns of at most 4096
+// (another kernel: its runs need more registers).
+constexpr int kNumSweepShapes = 7;
+constexpr int kColShape = 5, kColLongShape = 6;
+constexpr int kColThreads = 512, kColMax = 512, kColLongMax = 4096;
+// Columns per workgroup by line length n and value size: as many as leave a
+// thread runs that its registers hold, so that a row's load is as long a
+// piece of memory as can be.
+__host__ __device__ constexpr int col_lines(int n, int tbytes) {
+  if (n <= 64) return 32;
+  if (n <= 512) return 16;
+  if (tbytes == 4) return n <= 768 ? 16 : 8;
+  return n <= 1024 ? 8 : 4;
+}
+
 __host__ __device__ inline int half_x(int nx) { return (nx + 1) >> 1; }
 
 // The prolongation fills only the lines the first post-smoothing sweep reads:

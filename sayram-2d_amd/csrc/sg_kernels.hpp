@@ -22,6 +22,11 @@ void launch_line(hipStream_t s, const InstDev *d, const LineGrp *m, int ngroups,
 template <typename T>
 void launch_line_shapes(hipStream_t s, const InstDev *d, const LineGrp *m, int na, int nb,
                         int ngroups, int l, int dir, bool zero, int xid, int bid);
+// one colour of a column sweep with the columns in registers (col_lines
+// columns per group, of at most kColMax steps, is_long: kColLongMax)
+template <typename T>
+void launch_cols(hipStream_t s, const InstDev *d, const LineGrp *m, int ngroups, int l, bool is_long,
+                 bool zero, int xid, int bid);
 template <typename T>
 void launch_residual(hipStream_t s, const InstDev *d, const BlkMap *m, int nb, int l, int xid,
                      int bid);

@@ -1,0 +1,211 @@
+// sg_sweeps.hip -- zebra line sweeps with the lines held in registers.
+//
+// A sweep solves every line of one colour exactly with the precomputed
+// factors, the off-line couplings moved to the right-hand side. Both Thomas
+// recurrences are first-order affine maps (d_t = a_t d_{t-1} + b_t forward,
+// x_t = d_t - u_t x_{t+1} backward): a thread takes a run of consecutive
+// steps of one line into registers, composes their maps, the threads of the
+// line combine the compositions (wave shuffles, then one LDS exchange
+// between the waves), and each thread reruns its steps from the value that
+// enters them. A line is solved in one pass over its data, with one barrier
+// per recurrence, however long it is.
+#include "sg_device.hpp"
+#include "sg_kernels.hpp"
+#include "sg_scan.hpp"
+
+namespace sg {
+
+// LDS values of a column sweep of L columns in C runs: the composed maps of
+// every wave and column, forward and backward.
+template <int L, int C> constexpr int col_lds() { return 4 * (L * C / 64) * L; }
+
+// Columns. L columns of one colour (neighbouring lanes, so a step's loads are
+// L contiguous values) times C runs of at most K steps; consecutive runs
+// follow one another in a wave, then across the waves. The values of a thread's
+// steps are loaded in one go, so a sweep costs about one memory round trip
+// and the chip's bandwidth, where the tiled sweep (k_line) walked a line in
+// serial tiles of a load, two scans and three barriers each. Measured, tiled
+// against this, per launch of one colour: 765-step columns of a 1021 x 765
+// grid (FP32) 56 -> 13.4 us, its coarser columns 18.8 -> 7.2; 4096 steps
+// 131 -> 94 us; 2048 steps FP64 106 -> 41 us; the 9-point columns of a batch of
+// 48 uneven grids 14.4 -> 6.8 us, its 5-point ones 34.5 -> 16.5.
+// Run lengths: K steps of three values each must fit the registers; 4096 steps
+// as 8 columns x 64 runs of 64 took 94 us, as 4 columns x 128 runs of 32 (16
+// byte pieces of a row) 158.
+template <typename T, int NB, bool ZERO, int L, int C, int K>
+__device__ __forceinline__ void col_sweep(const InstDev &I, const LineGrp gr, int l, int xid,
+                                          int bid, T *lds) {
+  constexpr int NW = L * C / 64;   // waves
+  static_assert(L <= 64 && 64 % L == 0 && (L * C) % 64 == 0, "whole runs per wave");
+  T *const s_a = lds, *const s_b = s_a + NW * L, *const r_a = s_b + NW * L, *const r_b = r_a + NW * L;
+  const Lev &Lv = I.lev[l];
+  const int nx = Lv.nx, n = Lv.ny, hx = half_x(nx);
+  T *x; const T *b;
+  level_xb<T>(I, l, xid, bid, x, b);
+  const T *__restrict__ lo = cptr<T>(Lv.band[BS]);
+  const T *__restrict__ inv = cptr<T>(Lv.linv[1]);
+  const T *__restrict__ cu = cptr<T>(Lv.lup[1]);
+  const T *__restrict__ om = cptr<T>(Lv.band[BW]);
+  const T *__restrict__ op = cptr<T>(Lv.band[BE]);
+  const T *omm = nullptr, *omp = nullptr, *opm = nullptr, *opp = nullptr;
+  if (NB == 9) {
+    omm = cptr<T>(Lv.band[BSW]); omp = cptr<T>(Lv.band[BNW]);
+    opm = cptr<T>(Lv.band[BSE]); opp = cptr<T>(Lv.band[BNE]);
+  }
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int k = tid % L, c = tid / L;
+  const int kc = (n + C - 1) / C;                  // steps per run (uniform, <= K)
+  const int t0 = c * kc, cnt = min(kc, n - t0);    // this run's steps (cnt < 1: none)
+  const bool on = k < gr.count;                    // lanes past the group repeat its last column
+  const int li = gr.first + min(k, gr.count - 1) * gr.step;
+  // Slots of the column and of its neighbours in a row. Couplings to columns
+  // outside the grid are zero; such a neighbour is replaced by the one on the
+  // other side, which holds a value of the other colour (this colour's own x
+  // may never have been written, and 0 times a NaN is not 0).
+  const int lm = li > 0 ? li - 1 : min(1, nx - 1), lp = li < nx - 1 ? li + 1 : max(nx - 2, 0);
+  const uint32_t s0 = xslot(li, hx), sm = xslot(lm, hx), sp = xslot(lp, hx);
+  auto row = [&](int t) -> uint32_t { return (uint32_t)(max(0, min(t, n - 1)) * nx); };
+  // d_t = al d_{t-1} + be of every step; steps past the run are the identity
+  T al[K], be[K], up[K];
+  T xm0 = T(0), xm1 = T(0), xp0 = T(0), xp1 = T(0);   // x beside at steps t - 1 and t
+  if (!ZERO && NB == 9) {
+    xm0 = ld32(x, row(t0 - 1) + sm); xp0 = ld32(x, row(t0 - 1) + sp);
+    xm1 = ld32(x, row(t0) + sm); xp1 = ld32(x, row(t0) + sp);
+  }
+#pragma unroll
+  for (int e = 0; e < K; ++e) {
+    const bool ok = e < cnt;
+    const uint32_t q = row(t0 + e);
+    T r = ld32(b, q + s0);
+    const T v = ld32(inv, q + s0), w = ld32(lo, q + s0);
+    up[e] = ld32(cu, q + s0);
+    if (!ZERO) {
+      if (NB == 9) {
+        const uint32_t qn = row(t0 + e + 1);
+        const T xm2 = ld32(x, qn + sm), xp2 = ld32(x, qn + sp);
+        r = r - ld32(om, q + s0) * xm1 - ld32(op, q + s0) * xp1;
+        r = r - ld32(omm, q + s0) * xm0 - ld32(omp, q + s0) * xm2;
+        r = r - ld32(opm, q + s0) * xp0 - ld32(opp, q + s0) * xp2;
+        xm0 = xm1; xm1 = xm2; xp0 = xp1; xp1 = xp2;
+      } else {
+        r = r - ld32(om, q + s0) * ld32(x, q + sm) - ld32(op, q + s0) * ld32(x, q + sp);
+      }
+    }
+    al[e] = ok ? -w * v : T(1);
+    be[e] = ok ? r * v : T(0);
+  }
+  T A = T(1), B = T(0);
+#pragma unroll
+  for (int e = 0; e < K; ++e) { B = al[e] * B + be[e]; A = al[e] * A; }
+#pragma unroll
+  for (int off = L; off < 64; off <<= 1) {
+    const T Ap = __shfl_up(A, off, 64), Bp = __shfl_up(B, off, 64);
+    if (lane >= off) { B = A * Bp + B; A = A * Ap; }
+  }
+  T Ae = T(1), Be = T(0);
+  if (L < 64) {
+    Ae = __shfl_up(A, L, 64); Be = __shfl_up(B, L, 64);
+    if (lane < L) { Ae = T(1); Be = T(0); }
+  }
+  if (lane >= 64 - L) { s_a[wave * L + k] = A; s_b[wave * L + k] = B; }
+  lds_barrier();
+  T d = T(0);
+#pragma unroll
+  for (int w = 0; w < NW - 1; ++w) {
+    const T a = s_a[w * L + k], bb = s_b[w * L + k];
+    d = w < wave ? a * d + bb : d;
+  }
+  d = Ae * d + Be;
+#pragma unroll
+  for (int e = 0; e < K; ++e) {
+    const bool ok = e < cnt;
+    d = al[e] * d + be[e];
+    be[e] = ok ? d : T(0);
+    al[e] = ok ? -up[e] : T(1);
+  }
+  // backward: x_t = al x_{t+1} + be
+  A = T(1); B = T(0);
+#pragma unroll
+  for (int e = K - 1; e >= 0; --e) { B = al[e] * B + be[e]; A = al[e] * A; }
+#pragma unroll
+  for (int off = L; off < 64; off <<= 1) {
+    const T An = __shfl_down(A, off, 64), Bn = __shfl_down(B, off, 64);
+    if (lane + off < 64) { B = A * Bn + B; A = A * An; }
+  }
+  Ae = T(1); Be = T(0);
+  if (L < 64) {
+    Ae = __shfl_down(A, L, 64); Be = __shfl_down(B, L, 64);
+    if (lane >= 64 - L) { Ae = T(1); Be = T(0); }
+  }
+  if (lane < L) { r_a[wave * L + k] = A; r_b[wave * L + k] = B; }
+  lds_barrier();
+  T xv = T(0);
+#pragma unroll
+  for (int w = NW - 1; w > 0; --w) {
+    const T a = r_a[w * L + k], bb = r_b[w * L + k];
+    xv = w > wave ? a * xv + bb : xv;
+  }
+  xv = Ae * xv + Be;
+#pragma unroll
+  for (int e = K - 1; e >= 0; --e) {
+    xv = al[e] * xv + be[e];
+    if (on && e < cnt) st32(x, row(t0 + e) + s0, xv);
+  }
+}
+
+template <typename T, int NB, bool ZERO>
+__global__ void __launch_bounds__(kColThreads) k_cols(const InstDev *__restrict__ insts,
+                                                      const LineGrp *__restrict__ map, int l,
+                                                      int xid, int bid) {
+  __shared__ T lds[col_lds<32, 16>()];
+  const LineGrp gr = map[blockIdx.x];
+  const InstDev &I = insts[gr.inst];
+  if (rsc(I)->status != ST_ACTIVE) return;
+  const int n = I.lev[l].ny;
+  if (n <= 64) col_sweep<T, NB, ZERO, 32, 16, 4>(I, gr, l, xid, bid, lds);
+  else if (n <= 128) col_sweep<T, NB, ZERO, 16, 32, 4>(I, gr, l, xid, bid, lds);
+  else if (n <= 256) col_sweep<T, NB, ZERO, 16, 32, 8>(I, gr, l, xid, bid, lds);
+  else if (n <= 384) col_sweep<T, NB, ZERO, 16, 32, 12>(I, gr, l, xid, bid, lds);
+  else col_sweep<T, NB, ZERO, 16, 32, 16>(I, gr, l, xid, bid, lds);
+}
+
+template <typename T, int NB, bool ZERO>
+__global__ void __launch_bounds__(kColThreads) k_cols_long(const InstDev *__restrict__ insts,
+                                                           const LineGrp *__restrict__ map, int l,
+                                                           int xid, int bid) {
+  __shared__ T lds[col_lds<16, 32>()];
+  const LineGrp gr = map[blockIdx.x];
+  const InstDev &I = insts[gr.inst];
+  if (rsc(I)->status != ST_ACTIVE) return;
+  const int n = I.lev[l].ny;
+  if constexpr (sizeof(T) == 4) {
+    if (n <= 768) col_sweep<T, NB, ZERO, 16, 32, 24>(I, gr, l, xid, bid, lds);
+    else if (n <= 1024) col_sweep<T, NB, ZERO, 8, 64, 16>(I, gr, l, xid, bid, lds);
+    else if (n <= 2048) col_sweep<T, NB, ZERO, 8, 64, 32>(I, gr, l, xid, bid, lds);
+    else col_sweep<T, NB, ZERO, 8, 64, 64>(I, gr, l, xid, bid, lds);
+  } else {
+    if (n <= 1024) col_sweep<T, NB, ZERO, 8, 64, 16>(I, gr, l, xid, bid, lds);
+    else if (n <= 2048) col_sweep<T, NB, ZERO, 4, 128, 16>(I, gr, l, xid, bid, lds);
+    else col_sweep<T, NB, ZERO, 4, 128, 32>(I, gr, l, xid, bid, lds);
+  }
+}
+
+template <typename T>
+void launch_cols(hipStream_t s, const InstDev *d, const LineGrp *m, int ngroups, int l, bool is_long,
+                 bool zero, int xid, int bid) {
+  if (!ngroups) return;
+#define SG_COLS(NB, Z)                                                                    \
+  do {                                                                                    \
+    if (is_long) k_cols_long<T, NB, Z><<<ngroups, kColThreads, 0, s>>>(d, m, l, xid, bid); \
+    else k_cols<T, NB, Z><<<ngroups, kColThreads, 0, s>>>(d, m, l, xid, bid);              \
+  } while (0)
+  if (l > 0) { if (zero) SG_COLS(9, true); else SG_COLS(9, false); }
+  else { if (zero) SG_COLS(5, true); else SG_COLS(5, false); }
+#undef SG_COLS
+}
+template void launch_cols<double>(hipStream_t, const InstDev *, const LineGrp *, int, int, bool,
+                                  bool, int, int);
+template void launch_cols<float>(hipStream_t, const InstDev *, const LineGrp *, int, int, bool,
+                                 bool, int, int);
+
+}  // namespace sg
