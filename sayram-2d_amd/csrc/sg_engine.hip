@@ -190,25 +190,32 @@ static int tile_shape(const int (&lim)[4], int n, int dir, int l, bool fp64_vcyc
 // The default line lengths of the tile shapes (sg_opts.line_tiles).
 static const int kDefaultTiles[4] = {16, 160, 16, 768};
 
-// Shape of a line sweep. With the default line lengths the columns of at most
-// kColLongMax steps are solved in registers, one pass over their data. Longer
-// columns, and every column when the caller set other lengths, go by tile
-// shapes. Like the tile shape it depends only on the line, its level and the
+// Shape of a line sweep. With the default line lengths the lines of at most
+// kRowLongMax / kColLongMax steps are solved in registers, one pass over their
+// data. Longer lines, and every line of a direction for which the caller set
+// other lengths, go by tile shapes. Like the tile shape it depends only on the line, its level and the
 // options.
 static int sweep_shape(const int (&lim)[4], int n, int dir, int l, bool fp64_vcycle) {
   if (dir == 1 && lim[2] == kDefaultTiles[2] && lim[3] == kDefaultTiles[3]) {
     if (n <= kColMax) return kColShape;
     if (n <= kColLongMax) return kColLongShape;
   }
+  if (dir == 0 && lim[0] == kDefaultTiles[0] && lim[1] == kDefaultTiles[1]) {
+    if (n <= kRowMax) return kRowShape;
+    if (n <= kRowLongMax) return kRowLongShape;
+  }
   return tile_shape(lim, n, dir, l, fp64_vcycle);
 }
 // Lines per group of a sweep shape.
 static int sweep_lines(int shape, int n, bool fp64_vcycle) {
-  return shape < kNumTileShapes ? tile_lines(shape) : col_lines(n, fp64_vcycle ? 8 : 4);
+  const int tbytes = fp64_vcycle ? 8 : 4;
+  return shape < kNumTileShapes ? tile_lines(shape)
+         : shape == kColShape || shape == kColLongShape ? col_lines(n, tbytes)
+                                                        : row_lines(n, tbytes);
 }
 // Rank of a sweep shape by the length of the lines it takes.
 static int sweep_rank(int shape) {
-  return shape == kColLongShape ? 8 : shape == kColShape ? 7 : shape == 3 ? 9 : shape_rank(shape);
+  return shape >= kNumTileShapes ? shape : shape == 2 || shape == 3 ? 10 + shape : shape_rank(shape);
 }
 
 // Workgroups are dispatched to the 8 XCDs round-robin (workgroup b on XCD
@@ -971,7 +978,8 @@ template <typename T> void Batch::vcycle(int l, int xid, int bid) {
   // the groups of sweep shape sh in one launch
   auto lines = [&](hipStream_t s, const LineGrp *g, int ng, int dir, int sh, bool z) {
     if (sh < kNumTileShapes) launch_line<T>(s, d_insts, g, ng, l, dir, sh, z, xid, bid);
-    else launch_cols<T>(s, d_insts, g, ng, l, sh == kColLongShape, z, xid, bid);
+    else if (dir == 1) launch_cols<T>(s, d_insts, g, ng, l, sh == kColLongShape, z, xid, bid);
+    else launch_rows<T>(s, d_insts, g, ng, l, sh == kRowLongShape, z, xid, bid);
   };
   auto sweep = [&](int dir) {
     for (int p = 0; p < 2; ++p) {

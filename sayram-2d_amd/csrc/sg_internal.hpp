@@ -73,10 +73,12 @@ __host__ __device__ constexpr int ring_tiles(int sh, int tbytes, int nb) {
 
 // The sweeps with the lines in registers (sg_sweeps.hip), as further shapes of
 // the sweep maps: 5 columns of at most 512 steps, 6 columns of at most 4096
-// (another kernel: its runs need more registers).
-constexpr int kNumSweepShapes = 7;
-constexpr int kColShape = 5, kColLongShape = 6;
+// (another kernel: its runs need more registers), 7 rows of at most 2048, 8
+// rows of at most 4096.
+constexpr int kNumSweepShapes = 9;
+constexpr int kColShape = 5, kColLongShape = 6, kRowShape = 7, kRowLongShape = 8;
 constexpr int kColThreads = 512, kColMax = 512, kColLongMax = 4096;
+constexpr int kRowThreads = 256, kRowMax = 2048, kRowLongMax = 4096;
 // Columns per workgroup by line length n and value size: as many as leave a
 // thread runs that its registers hold, so that a row's load is as long a
 // piece of memory as can be.
@@ -85,6 +87,18 @@ __host__ __device__ constexpr int col_lines(int n, int tbytes) {
   if (n <= 512) return 16;
   if (tbytes == 4) return n <= 768 ? 16 : 8;
   return n <= 1024 ? 8 : 4;
+}
+
+// Rows per workgroup: as many as its four waves take, each a segment of the
+// lanes that 8 (FP64 rows of at most 256: 4) steps per lane make, a power of
+// two, at most 64; longer rows take 2 or 4 waves.
+__host__ __device__ constexpr int row_lines(int n, int tbytes) {
+  if (n > 1024) return 1;
+  if (n > 512) return 2;
+  const int k = tbytes == 8 && n <= 256 ? 4 : 8;
+  int w = 1;
+  while (w * k < n) w *= 2;
+  return kRowThreads / w;
 }
 
 __host__ __device__ inline int half_x(int nx) { return (nx + 1) >> 1; }

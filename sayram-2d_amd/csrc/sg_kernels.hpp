@@ -27,6 +27,11 @@ void launch_line_shapes(hipStream_t s, const InstDev *d, const LineGrp *m, int n
 template <typename T>
 void launch_cols(hipStream_t s, const InstDev *d, const LineGrp *m, int ngroups, int l, bool is_long,
                  bool zero, int xid, int bid);
+// one colour of a row sweep with the rows in registers (row_lines rows per
+// group, of at most kRowMax steps, is_long: kRowLongMax)
+template <typename T>
+void launch_rows(hipStream_t s, const InstDev *d, const LineGrp *m, int ngroups, int l, bool is_long,
+                 bool zero, int xid, int bid);
 template <typename T>
 void launch_residual(hipStream_t s, const InstDev *d, const BlkMap *m, int nb, int l, int xid,
                      int bid);

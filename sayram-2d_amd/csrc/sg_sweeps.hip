@@ -208,4 +208,218 @@ template void launch_cols<double>(hipStream_t, const InstDev *, const LineGrp *,
 template void launch_cols<float>(hipStream_t, const InstDev *, const LineGrp *, int, int, bool,
                                  bool, int, int);
 
+// H consecutive values from slot on, in one load (global loads take any
+// alignment of the element; a row's halves start at any slot).
+template <typename T, int H>
+__device__ __forceinline__ void ldv(const T *base, uint32_t slot, T (&v)[H]) {
+  typedef T VT __attribute__((ext_vector_type(H), aligned(sizeof(T))));
+  using GC = const __attribute__((address_space(1))) char;
+  using GV = const __attribute__((address_space(1))) VT;
+  const VT t = *(GV *)((GC *)base + slot * (uint32_t)sizeof(T));
+#pragma unroll
+  for (int e = 0; e < H; ++e) v[e] = t[e];
+}
+template <typename T, int H>
+__device__ __forceinline__ void stv(T *base, uint32_t slot, const T (&v)[H]) {
+  typedef T VT __attribute__((ext_vector_type(H), aligned(sizeof(T))));
+  using GC = __attribute__((address_space(1))) char;
+  using GV = __attribute__((address_space(1))) VT;
+  VT t;
+#pragma unroll
+  for (int e = 0; e < H; ++e) t[e] = v[e];
+  *(GV *)((GC *)base + slot * (uint32_t)sizeof(T)) = t;
+}
+
+// Rows. A lane takes K consecutive steps of a row, K/2 from each half of the
+// split layout, as vector loads; WL = 1: a row is a segment of W lanes (64/W
+// rows per wave) and nothing goes through LDS; WL > 1: a row is WL waves,
+// chained through LDS. The last lane's vectors may reach up to K/2 values past
+// the row (past the array for the last row, into the next array of the
+// instance's slab; the slab ends with the last level's scratch, which no sweep
+// reads): those values are never used.
+// Measured per launch of one colour, tiled against this: the 9-point rows of a
+// 1021 x 765 grid (FP32) 7.5 -> 4.1 us and its 5-point ones 12.2 -> 5.2;
+// 2048 x 2048 FP64 12.5 -> 6.6 and 39 -> 27; 4096-step rows 62 -> 45 us (3.0
+// TB/s); a batch of 48 uneven grids 8.9 -> 5.5 and 21 (two launches) -> 11.3.
+template <typename T, int NB, bool ZERO, int K, int WL>
+__device__ __forceinline__ void row_sweep(const InstDev &I, const LineGrp gr, int l, int xid,
+                                          int bid, T *lds) {
+  constexpr int H = K / 2;
+  const Lev &Lv = I.lev[l];
+  const int n = Lv.nx, ny = Lv.ny, hx = half_x(n);
+  T *x; const T *b;
+  level_xb<T>(I, l, xid, bid, x, b);
+  const T *__restrict__ lo = cptr<T>(Lv.band[BW]);
+  const T *__restrict__ inv = cptr<T>(Lv.linv[0]);
+  const T *__restrict__ cu = cptr<T>(Lv.lup[0]);
+  const T *__restrict__ om = cptr<T>(Lv.band[BS]);
+  const T *__restrict__ op = cptr<T>(Lv.band[BN]);
+  const T *omm = nullptr, *omp = nullptr, *opm = nullptr, *opp = nullptr;
+  if (NB == 9) {
+    omm = cptr<T>(Lv.band[BSW]); omp = cptr<T>(Lv.band[BSE]);
+    opm = cptr<T>(Lv.band[BNW]); opp = cptr<T>(Lv.band[BNE]);
+  }
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int W = WL > 1 ? 64 : seg_width((n + K - 1) / K);   // lanes per row in a wave
+  const int u = lane & (W - 1);
+  const int k = WL > 1 ? wave / WL : wave * (64 / W) + lane / W;   // row of the group
+  const int q = WL > 1 ? (wave % WL) * 64 + lane : u;              // run of the row
+  const bool on = k < gr.count;
+  const int li = gr.first + min(k, gr.count - 1) * gr.step;
+  // rows beside; outside the grid the couplings are zero and the row on the
+  // other side stands in (it holds values of the other colour)
+  const int lm = li > 0 ? li - 1 : min(1, ny - 1), lp = li < ny - 1 ? li + 1 : max(ny - 2, 0);
+  const int t0 = q * K;                    // this lane's first step
+  const int h0 = t0 < n ? q * H : 0;       // its place in each half
+  const uint32_t r0 = (uint32_t)li * n, se = r0 + h0, so = r0 + hx + h0;
+  // one array's K values in step order
+  auto get = [&](const T *p, uint32_t a, uint32_t c, T (&v)[K]) {
+    T ev[H], od[H];
+    ldv<T, H>(p, a, ev);
+    ldv<T, H>(p, c, od);
+#pragma unroll
+    for (int e = 0; e < H; ++e) { v[2 * e] = ev[e]; v[2 * e + 1] = od[e]; }
+  };
+  T al[K], be[K], up[K];
+  {
+    T vb[K], vl[K], vi[K];
+    get(b, se, so, vb);
+    get(lo, se, so, vl);
+    get(inv, se, so, vi);
+    get(cu, se, so, up);
+    if (!ZERO) {
+      // x of the row beside with its steps t0 - 1 and t0 + K (9-point), zero
+      // past the end of the row
+      auto beside = [&](int lj, const T *pc, const T *pm, const T *pp) {
+        const uint32_t rj = (uint32_t)lj * n;
+        T xv[K], c[K];
+        get(x, rj + h0, rj + hx + h0, xv);
+        get(pc, se, so, c);
+        T xl = T(0), xr = T(0), cm[K], cp[K];
+        if (NB == 9) {
+          xl = ld32(x, rj + hx + max(h0 - 1, 0));
+          xr = ld32(x, rj + min(h0 + H, hx - 1));
+          get(pm, se, so, cm);
+          get(pp, se, so, cp);
+        }
+#pragma unroll
+        for (int e = 0; e < K; ++e) xv[e] = t0 + e < n ? xv[e] : T(0);
+#pragma unroll
+        for (int e = 0; e < K; ++e) {
+          vb[e] -= c[e] * xv[e];
+          if (NB == 9) {
+            vb[e] -= cm[e] * (e > 0 ? xv[e - 1] : xl);
+            vb[e] -= cp[e] * (e + 1 < K ? xv[e + 1] : xr);
+          }
+        }
+      };
+      beside(lm, om, omm, omp);
+      beside(lp, op, opm, opp);
+    }
+#pragma unroll
+    for (int e = 0; e < K; ++e) {
+      const bool ok = t0 + e < n;
+      al[e] = ok ? -vl[e] * vi[e] : T(1);
+      be[e] = ok ? vb[e] * vi[e] : T(0);
+    }
+  }
+  // the value entering this lane's steps, from the lanes (and waves) before
+  auto carry = [&](auto fwdc, T A, T B, T *s) -> T {
+    constexpr bool FWD = decltype(fwdc)::value;
+    scan_rows<FWD>(A, B, u, W);
+    RowMaps<T> m{};
+    if (W > 16) m = row_maps<FWD>(A, B);
+    T in = T(0);
+    if (WL > 1) {
+      T a, bb;
+      wave_map<FWD>(m, a, bb);
+      if (lane == 0) { s[2 * wave] = a; s[2 * wave + 1] = bb; }
+      lds_barrier();
+      const int w0 = wave - wave % WL;
+#pragma unroll
+      for (int w = 0; w < WL - 1; ++w) {
+        const int ww = FWD ? w0 + w : w0 + WL - 1 - w;
+        const T a2 = s[2 * ww], b2 = s[2 * ww + 1];
+        in = (FWD ? ww < wave : ww > wave) ? a2 * in + b2 : in;
+      }
+    }
+    return enter<FWD>(A, B, m, u, W, in);
+  };
+  T A = T(1), B = T(0);
+#pragma unroll
+  for (int e = 0; e < K; ++e) { B = al[e] * B + be[e]; A = al[e] * A; }
+  T d = carry(std::true_type(), A, B, lds);
+#pragma unroll
+  for (int e = 0; e < K; ++e) {
+    const bool ok = t0 + e < n;
+    d = al[e] * d + be[e];
+    be[e] = ok ? d : T(0);
+    al[e] = ok ? -up[e] : T(1);
+  }
+  A = T(1); B = T(0);
+#pragma unroll
+  for (int e = K - 1; e >= 0; --e) { B = al[e] * B + be[e]; A = al[e] * A; }
+  T xv = carry(std::false_type(), A, B, lds + 8);
+  T ev[H], od[H];
+#pragma unroll
+  for (int e = K - 1; e >= 0; --e) {
+    xv = al[e] * xv + be[e];
+    if (e & 1) od[e / 2] = xv; else ev[e / 2] = xv;
+  }
+  if (!on) return;
+  if (t0 + K <= n) {
+    stv<T, H>(x, se, ev);
+    stv<T, H>(x, so, od);
+  } else {
+#pragma unroll
+    for (int e = 0; e < H; ++e) {
+      if (t0 + 2 * e < n) st32(x, se + e, ev[e]);
+      if (t0 + 2 * e + 1 < n) st32(x, so + e, od[e]);
+    }
+  }
+}
+
+template <typename T, int NB, bool ZERO>
+__global__ void __launch_bounds__(kRowThreads) k_rows(const InstDev *__restrict__ insts,
+                                                      const LineGrp *__restrict__ map, int l,
+                                                      int xid, int bid) {
+  __shared__ T lds[16];
+  const LineGrp gr = map[blockIdx.x];
+  const InstDev &I = insts[gr.inst];
+  if (rsc(I)->status != ST_ACTIVE) return;
+  const int n = I.lev[l].nx;
+  if (sizeof(T) == 8 && n <= 256) row_sweep<T, NB, ZERO, 4, 1>(I, gr, l, xid, bid, lds);
+  else if (n <= 512) row_sweep<T, NB, ZERO, 8, 1>(I, gr, l, xid, bid, lds);
+  else if (n <= 1024) row_sweep<T, NB, ZERO, 8, 2>(I, gr, l, xid, bid, lds);
+  else row_sweep<T, NB, ZERO, 8, 4>(I, gr, l, xid, bid, lds);
+}
+template <typename T, int NB, bool ZERO>
+__global__ void __launch_bounds__(kRowThreads) k_rows_long(const InstDev *__restrict__ insts,
+                                                           const LineGrp *__restrict__ map, int l,
+                                                           int xid, int bid) {
+  __shared__ T lds[16];
+  const LineGrp gr = map[blockIdx.x];
+  const InstDev &I = insts[gr.inst];
+  if (rsc(I)->status != ST_ACTIVE) return;
+  row_sweep<T, NB, ZERO, 16, 4>(I, gr, l, xid, bid, lds);
+}
+
+template <typename T>
+void launch_rows(hipStream_t s, const InstDev *d, const LineGrp *m, int ngroups, int l, bool is_long,
+                 bool zero, int xid, int bid) {
+  if (!ngroups) return;
+#define SG_ROWS(NB, Z)                                                                    \
+  do {                                                                                    \
+    if (is_long) k_rows_long<T, NB, Z><<<ngroups, kRowThreads, 0, s>>>(d, m, l, xid, bid); \
+    else k_rows<T, NB, Z><<<ngroups, kRowThreads, 0, s>>>(d, m, l, xid, bid);              \
+  } while (0)
+  if (l > 0) { if (zero) SG_ROWS(9, true); else SG_ROWS(9, false); }
+  else { if (zero) SG_ROWS(5, true); else SG_ROWS(5, false); }
+#undef SG_ROWS
+}
+template void launch_rows<double>(hipStream_t, const InstDev *, const LineGrp *, int, int, bool,
+                                  bool, int, int);
+template void launch_rows<float>(hipStream_t, const InstDev *, const LineGrp *, int, int, bool,
+                                 bool, int, int);
+
 }  // namespace sg
