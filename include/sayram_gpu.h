@@ -103,9 +103,13 @@ typedef struct {
   int line_tiles[4];    /* line-solve tile shapes by line length: rows of at most
                            [0] cells use 64x16 tiles, of at most [1] cells 16x64,
                            longer rows 4x256; columns of at most [2] cells 64x16,
-                           of at most [3] cells 32x32, longer columns 16x256. 0 selects the defaults 16, 160,
-                           16, 768. They change the rounding of the line solves,
-                           so results are reproducible for the same values. */
+                           of at most [3] cells 32x32, longer columns 16x256.
+                           0 selects the defaults 16, 160, 16, 768. With the
+                           defaults of a direction its sweeps hold lines of at
+                           most 4096 cells in registers instead, and the tile
+                           shapes serve longer lines and the factorisations.
+                           They change the rounding of the line solves, so
+                           results are reproducible for the same values. */
   int coarse_tiles[4];  /* as line_tiles, for the line solves of the coarser
                            levels (9-point operators); 0 selects the defaults
                            16, 160, 16, 768. */
@@ -113,10 +117,11 @@ typedef struct {
                            of at most fuse_cells cells and sides of at most 64
                            down run in one fused launch per instance (post-
                            smoothing schedules, with or without an x-line
-                           pre-sweep); 0 selects 1024, the maximum with FP64
-                           V-cycles (4096 with FP32 ones; levels are kept in
-                           LDS); -1 disables. Like line_tiles it changes the
-                           rounding of those line solves. */
+                           pre-sweep). 0 or 1024 (default): any level with sides
+                           of at most 64; other values at most 1024 with FP64
+                           V-cycles, 4096 with FP32 ones; -1 disables. Like
+                           line_tiles it changes the rounding of those line
+                           solves. */
   int streams;          /* 2: the tile shapes of one finest-level line sweep
                            run on two HIP streams (the longest lines beside the
                            rest; a coarser level's shapes share one launch in

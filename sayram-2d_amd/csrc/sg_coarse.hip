@@ -1,372 +1,477 @@
-// sg_coarse.hip -- the fused coarse cycle.
+// sg_coarse.hip -- the coarse end of the V-cycle: the dense inverse of the last
+// level and the fused coarse cycle.
 //
-// The levels of one instance from `lev` (its first level that fits, see
-// fused_fits) down to its coarsest and back, in one workgroup with LDS
-// barriers between the phases, instead of several launches per level. The
-// cycle is the per-level one: per level on the way down an optional
+// Fused cycle: the levels of one instance from `lev` (its first level with
+// sides of at most kFuseSide and at most fuse_cells cells) down to its last and
+// back, in one workgroup with LDS barriers between the phases, instead of
+// several launches per level. Per level on the way down an optional
 // pre-smoothing sweep of x-lines and the restriction of the residual (of b
-// itself without pre-smoothing), the exact line solve of the coarsest level,
-// then per level the prolongation of the lines the first post-sweep reads and
-// the zebra post-sweeps.
+// itself without pre-smoothing); the last level by the inverse of its
+// operator; then per level the prolongation of the lines the first post-sweep
+// reads and the zebra post-sweeps.
 //
-// Bound: latency. One workgroup walks some 8 phases per level, each a few LDS
-// accesses and a barrier, so the time is the sum of the phases' latencies,
-// not bytes. Hence:
-//  * x of every level (with a border of zeros, so that no neighbour needs a
-//    test) and b of every level but the first stay in LDS for the whole cycle;
-//  * a thread owns one cell per sweep colour (R rounds of 1024), with the lanes
-//    of a wave along the line, and solves the line with wave scans of its
-//    affine maps (sg_scan.hpp): one phase per colour. One thread per line
-//    running the recurrences out of LDS took two phases and a chain of 2 n
-//    dependent steps;
-//  * the operator and factors of a cell are read straight into the owner's
-//    registers, a whole level's in one round trip.
-// Measured against one thread per line: 69.0 -> 30.5 us per cycle on a 90 x 100
-// grid (FP64, first level 23 x 25), 76.0 -> 32.0 us at 1021 x 765 (FP32, 32 x
-// 24), 104 -> 42 us for the 192 cycles of an FP64 batch in one launch.
+// Bound: latency of one workgroup, which walks 8 phases per level, each a few
+// LDS accesses and some hundred instructions; bytes do not matter. A wave issues
+// a dependent instruction every 8 to 10 cycles, taken branches and code run for
+// the first time cost more. Hence:
+//  * x and b of every level stay in LDS for the whole cycle, with a border of
+//    zeros, so that no neighbour needs a test;
+//  * a line is a segment of at most 16 lanes (one step per lane, or four), so
+//    that both Thomas recurrences are scans of affine maps inside one DPP row;
+//    the map at a line's first step has A = 0, which separates the lines of a
+//    row without a mask;
+//  * the phases are one loop over a table built with the instance, and the
+//    operator is packed once per step in the order the lanes read it, zero
+//    where a lane has no cell: a phase's operands are a few vector loads from
+//    one base, issued while the phase before runs;
+//  * the hierarchy ends at kDense cells: the four levels that would follow an
+//    8 x 8 level cost 32 phases, the product with its inverse one.
+// Measured per cycle (first level): 90 x 100 FP64 (45 x 50) 32 us and 80 x 80
+// FP32 (40 x 40) 15 us; a version with one thread per line took 69 and 31 from
+// half the sides on, one with every level, direction and colour inlined (60
+// KB of code) 78 and 34 from these.
 #include "sg_device.hpp"
 #include "sg_kernels.hpp"
 #include "sg_scan.hpp"
 
 namespace sg {
 
-// LDS values of a fused cycle of R rounds: the sums over the levels of the
-// bordered x (odd pitch: the stride of a column sweep then spreads over the
-// banks) and of b below the first level, for the largest first level
-// (fused_side_max x fused_side_max, at most 1024 R^2 cells).
-__host__ __device__ constexpr int fused_pitch(int nx) { return (nx + 2) | 1; }
-constexpr int fused_x_elems(int nx, int ny) {
-  int s = 0;
-  for (;;) {
-    s += fused_pitch(nx) * (ny + 2);
-    if (nx == 1 || ny == 1) return s;
-    nx = (nx + 1) / 2; ny = (ny + 1) / 2;
+// ---------------------------------------------------------------------------
+// Inverse of the last level's operator (FP64, stored in the V-cycle precision),
+// once per step: Gauss-Jordan without pivoting (the level-0 operator is a
+// column diagonally dominant M-matrix, and so are its Galerkin products with
+// non-negative weights of row sum at most 1). Wave w holds rows w + 16 r, one
+// lane per column, in registers; the scaled pivot row goes through LDS, the
+// pivot column comes from a lane of the wave itself: one barrier per pivot.
+// ---------------------------------------------------------------------------
+template <typename T>
+__global__ void __launch_bounds__(1024) k_dense_inverse(const InstDev *__restrict__ insts,
+                                                        const FuseMap *__restrict__ map) {
+  constexpr int R = kDense / 16;
+  __shared__ double s_row[2][kDense];
+  const InstDev &I = insts[map[blockIdx.x].inst];
+  if (rsc(I)->ostatus == ST_IDLE) return;
+  const Lev &L = I.lev[I.nlev - 1];
+  const int nx = L.nx, ny = L.ny, n = nx * ny, hx = half_x(nx);
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const bool nine = I.nlev > 1;
+  double a[R];
+  {
+    const int cj = lane / nx, ci = lane - cj * nx;   // column: cell `lane` in row order
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+      const int K = wave + 16 * r;
+      a[r] = K == lane ? 1.0 : 0.0;   // identity outside the matrix
+      if (K >= n || lane >= n) continue;
+      const int j = K / nx, i = K - j * nx;
+      const int di = ci - i, dj = cj - j;
+      if (di < -1 || di > 1 || dj < -1 || dj > 1) continue;
+      const int b = dj == 0 ? (di == 0 ? BC : di < 0 ? BW : BE)
+                    : dj < 0 ? (di == 0 ? BS : di < 0 ? BSW : BSE)
+                             : (di == 0 ? BN : di < 0 ? BNW : BNE);
+      a[r] = (nine || b <= BN) ? gbl(L.band64[b])[j * nx + xslot(i, hx)] : 0.0;
+    }
+  }
+#pragma unroll
+  for (int rp = 0; rp < R; ++rp) {
+#pragma unroll 1
+    for (int w = 0; w < 16; ++w) {
+      const int p = w + 16 * rp;
+      if (p >= n) break;   // uniform
+      if (wave == w) {
+        const double inv = 1.0 / rdlane(a[rp], p);
+        a[rp] = lane == p ? inv : a[rp] * inv;
+        s_row[p & 1][lane] = a[rp];
+      }
+      lds_barrier();
+      const double rv = s_row[p & 1][lane];
+#pragma unroll
+      for (int r = 0; r < R; ++r) {
+        const double c = rdlane(a[r], p);
+        if (r != rp || wave != w) a[r] = (lane == p ? 0.0 : a[r]) - c * rv;
+      }
+    }
+  }
+  T *const out = ptr<T>(L.dinv);
+#pragma unroll
+  for (int r = 0; r < R; ++r) {
+    const int K = wave + 16 * r;
+    if (K < n && lane < n) st32(out, (uint32_t)(lane * n + K), (T)a[r]);
   }
 }
-constexpr int fused_b_elems(int nx, int ny) {
-  int s = 0;
-  while (nx > 1 && ny > 1) {
-    nx = (nx + 1) / 2; ny = (ny + 1) / 2;
-    s += nx * ny;
+
+// ---------------------------------------------------------------------------
+// Packed operator of the fused levels, once per step: one workgroup per level
+// and kind (PackKind) of an instance; a thread fills its lane's values.
+// ---------------------------------------------------------------------------
+template <typename T>
+__global__ void __launch_bounds__(kFuseThreads) k_coarse_pack(const InstDev *__restrict__ insts,
+                                                              const PackMap *__restrict__ map) {
+  const PackMap pm = map[blockIdx.x];
+  const InstDev &I = insts[pm.inst];
+  if (rsc(I)->ostatus == ST_IDLE) return;
+  const Lev &L = I.lev[pm.lev];
+  const int nx = L.nx, ny = L.ny, hx = half_x(nx), kind = pm.kind;
+  const LineLanes g = pack_lanes(nx, ny, kind);
+  const bool col = kind == PK_COL0 || kind == PK_COL1, nine = pm.lev > 0;
+  const int colour = kind == PK_ROW1 || kind == PK_COL1 || kind == PK_PRO;
+  T *const out = ptr<T>(I.pack) + pm.off;
+  const int n = col ? ny : nx, total = g.lanes * g.K, arrays = pack_arrays(kind);
+  // neighbouring threads fill neighbouring values; all loads of a value's
+  // arrays before their stores
+  for (int idx = threadIdx.x; idx < total; idx += kFuseThreads) {
+    const int ln = idx / g.K, t = g.K * (ln & ((1 << g.lw) - 1)) + idx % g.K, k = ln >> g.lw;
+    const int li = colour + 2 * k;
+    const bool on = k < g.nl && t < n;
+    const int i = on ? (col ? li : t) : 0, j = on ? (col ? t : li) : 0;
+    const uint32_t K = (uint32_t)(j * nx + xslot(i, hx));
+    auto get = [&](const void *p) { return ld32(cptr<T>(p), K); };
+    T v[9];
+    if (kind == PK_RES || kind == PK_PRO) {   // the weights that are 0 or 1 are not stored
+      v[0] = get(L.pw[0]);
+      v[1] = get(L.pw[1]);
+      v[2] = get(L.pw[2]);
+      v[3] = get(L.pw[3]);
+      if (kind == PK_RES) v[0] = (t & 1) ? v[0] : T(0);
+      v[1] = (t & 1) ? v[1] : T(0);
+      v[3] = (t & 1) ? v[3] : T(0);
+    } else {
+      v[0] = get(L.band[col ? BS : BW]);
+      v[1] = get(L.linv[col]);
+      v[2] = get(L.lup[col]);
+      v[3] = get(L.band[col ? BW : BS]);
+      v[4] = get(L.band[col ? BE : BN]);
+      if (nine) {
+        v[5] = get(L.band[BSW]);
+        v[6] = get(L.band[col ? BNW : BSE]);
+        v[7] = get(L.band[col ? BSE : BNW]);
+        v[8] = get(L.band[BNE]);
+      } else {
+        v[5] = v[6] = v[7] = v[8] = T(0);
+      }
+      // nothing couples a line's first step to the one before, or its last to
+      // the one after
+      v[0] = t > 0 ? -v[0] * v[1] : T(0);
+      v[2] = t < n - 1 ? -v[2] : T(0);
+    }
+#pragma unroll
+    for (int q = 0; q < 9; ++q)
+      if (q < arrays) st32(out, (uint32_t)(q * total + idx), on ? v[q] : T(0));
   }
-  return s;
 }
-constexpr int fused_rounds(int nx, int ny) {
-  int most = 1;
-  for (int d = 0; d < 2; ++d) {
-    const int n = d ? ny : nx, lines = ((d ? nx : ny) + 1) / 2;
-    int w = 1;
-    while (w < n) w *= 2;
-    const int r = (lines * w + kFuseThreads - 1) / kFuseThreads;
-    most = r > most ? r : most;
-  }
-  return most;
+
+// ---------------------------------------------------------------------------
+// Fused coarse cycle
+// ---------------------------------------------------------------------------
+// LDS values of x (and as many of b): the sum over the levels of the bordered
+// arrays, for the largest shapes, and what the lanes past a line's end may
+// reach after the last one.
+constexpr int fused_elems(int cells) {
+  int most = 0;
+  for (int fx = 1; fx <= kFuseSide; ++fx)
+    for (int fy = 1; fy <= kFuseSide; ++fy) {
+      if (fx * fy > cells) continue;
+      int s = 0;
+      for (int nx = fx, ny = fy;; nx = (nx + 1) / 2, ny = (ny + 1) / 2) {
+        s += fused_pitch(nx) * (ny + 2);
+        if (nx == 1 || ny == 1 || nx * ny <= kDense) break;
+      }
+      most = s > most ? s : most;
+    }
+  return most + 5 * fused_pitch(kFuseSide);
 }
-struct FusedSize { int x, b, rounds; };
-constexpr FusedSize fused_size(int cells) {
-  FusedSize m{0, 0, 0};
+constexpr bool fused_lanes_fit() {
   for (int nx = 1; nx <= kFuseSide; ++nx)
-    for (int ny = 1; ny <= kFuseSide; ++ny) {
-      if (nx * ny > cells) continue;
-      const int x = fused_x_elems(nx, ny), b = fused_b_elems(nx, ny), r = fused_rounds(nx, ny);
-      m.x = x > m.x ? x : m.x;
-      m.b = b > m.b ? b : m.b;
-      m.rounds = r > m.rounds ? r : m.rounds;
-    }
-  return m;
+    for (int ny = 1; ny <= kFuseSide; ++ny)
+      for (int k = 0; k < kNumPack; ++k)
+        if (pack_lanes(nx, ny, k).lanes > kFuseThreads && nx * ny > kDense) return false;
+  return true;
 }
 
-// One cell's row of its line's equations: the factors and the couplings to
-// the lines beside (minus / plus side, at steps t - 1, t, t + 1); zero where
-// there is no cell.
-template <typename T> struct CellEq { T lo, inv, up, m0, p0, mm, mp, pm, pp; };
-
-template <typename T, int DIR>
-__device__ __forceinline__ CellEq<T> cell_eq(const Lev &L, bool nine, uint32_t K, bool on) {
-  CellEq<T> q{};
-  if (on) {
-    q.lo = ld32(cptr<T>(L.band[DIR == 0 ? BW : BS]), K);
-    q.inv = ld32(cptr<T>(L.linv[DIR]), K);
-    q.up = ld32(cptr<T>(L.lup[DIR]), K);
-    q.m0 = ld32(cptr<T>(L.band[DIR == 0 ? BS : BW]), K);
-    q.p0 = ld32(cptr<T>(L.band[DIR == 0 ? BN : BE]), K);
-    if (nine) {
-      q.mm = ld32(cptr<T>(L.band[BSW]), K);
-      q.mp = ld32(cptr<T>(L.band[DIR == 0 ? BSE : BNW]), K);
-      q.pm = ld32(cptr<T>(L.band[DIR == 0 ? BNW : BSE]), K);
-      q.pp = ld32(cptr<T>(L.band[BNE]), K);
-    }
+// Arrays A0 .. A0 + N - 1 of a task's operands: K consecutive values of N packed
+// arrays, `stride` values apart.
+template <int K, int A0, int N, typename T>
+__device__ __forceinline__ void load_pack(const T *p, uint32_t off, uint32_t stride, T (&v)[9][4]) {
+  typedef T VT __attribute__((ext_vector_type(K)));
+  using GC = const __attribute__((address_space(1))) char;
+  using GV = const __attribute__((address_space(1))) VT;
+#pragma unroll
+  for (int a = 0; a < N; ++a) {
+    const VT w = *(GV *)((GC *)p + (off + a * stride) * (uint32_t)sizeof(T));
+#pragma unroll
+    for (int e = 0; e < K; ++e) v[A0 + a][e] = w[e];
   }
-  return q;
 }
 
-// The couplings of a cell to the lines beside it, applied to x in LDS (ix: its
-// place, sl / sp: strides along and across the line).
-template <typename T>
-__device__ __forceinline__ T beside(const CellEq<T> &q, const T *x, int ix, int sl, int sp) {
-  T s = q.m0 * x[ix - sp] + q.p0 * x[ix + sp];
-  s += q.mm * x[ix - sp - sl] + q.mp * x[ix - sp + sl];
-  s += q.pm * x[ix + sp - sl] + q.pp * x[ix + sp + sl];
-  return s;
+// a task by scalar loads
+__device__ __forceinline__ CoarseTask load_task(const CoarseTask *p, int it) {
+  typedef const __attribute__((address_space(4))) int ConstInt;
+  ConstInt *const q = (ConstInt *)(p + it);
+  CoarseTask t;
+  t.kind = q[0]; t.K = q[1]; t.lw = q[2]; t.n = q[3]; t.nl = q[4]; t.lanes = q[5]; t.x0 = q[6];
+  t.sl = q[7]; t.sp = q[8]; t.pack = q[9]; t.aux = q[10]; t.pc = q[11]; t.lev = q[12]; t.pack2 = q[13];
+  return t;
 }
 
-// Solution at step u of the line of this lane's segment with right-hand side
-// r (zero at steps past the line's end, whose factors are zero too).
-template <typename T>
-__device__ __forceinline__ T solve_line(const CellEq<T> &q, T r, int u, int W) {
-  T a = -q.lo * q.inv, d = r * q.inv;
-  T A = a, B = d;
-  scan_rows<true>(A, B, u, W);
-  if (W > 16) {
-    const RowMaps<T> m = row_maps<true>(A, B);
-    B = a * enter<true>(A, B, m, u, W, T(0)) + d;
-  }
-  d = B;   // the eliminated right-hand side
-  a = -q.up;
-  A = a; B = d;
-  scan_rows<false>(A, B, u, W);
-  if (W > 16) {
-    const RowMaps<T> m = row_maps<false>(A, B);
-    B = a * enter<false>(A, B, m, u, W, T(0)) + d;
-  }
-  return B;
-}
-
-// smoother: the finest level's schedule in bits 0-3, the coarser levels' in
-// bits 4-7 (post-smoothing bits and the x-line pre-smoothing bit)
-template <typename T, int R>
+template <typename T, int CAP>
 __global__ void __launch_bounds__(kFuseThreads) k_coarse_cycle(const InstDev *__restrict__ insts,
                                                                const FuseMap *__restrict__ map,
-                                                               int xid, int bid, int smoother) {
-  constexpr FusedSize SZ = fused_size(R == 1 ? 1024 : kFuseCells32);
-  static_assert(SZ.rounds <= R, "a thread owns R cells of a colour at most");
-  __shared__ T sx[SZ.x];
-  __shared__ T sb[SZ.b + 1];
+                                                               int xid, int bid) {
+  static_assert(fused_lanes_fit(), "every line of a colour has its lanes");
+  constexpr int XN = fused_elems(CAP), NW = kFuseThreads / 64, DC = kDense / NW;
+  __shared__ T sx[XN];              // x of the levels, bordered
+  __shared__ T sb[kDense + XN];     // the dense level's b, then b in the places of x
+  __shared__ T sp[NW * kDense];
   const FuseMap fm = map[blockIdx.x];
   const InstDev &I = insts[fm.inst];
   if (rsc(I)->status != ST_ACTIVE) return;
-  const int tid = threadIdx.x;
+  const CoarseTask *const tasks = I.tasks;
+  const T *const pack = cptr<T>(I.pack);
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int lf = fm.lev, last = I.nlev - 1;
-  auto sched = [&](int m) { return m == 0 ? (smoother & 15) : (smoother >> 4); };
   T *xg; const T *bg;
   level_xb<T>(I, lf, xid, bid, xg, bg);
-  int nx = I.lev[lf].nx, ny = I.lev[lf].ny;
-  {
-    int tot = 0, cx = nx, cy = ny;
-    for (int m = lf;; ++m) {
-      tot += fused_pitch(cx) * (cy + 2);
-      if (m == last) break;
-      cx = (cx + 1) >> 1; cy = (cy + 1) >> 1;
-    }
-    for (int k = tid; k < tot; k += kFuseThreads) sx[k] = T(0);
+  const int fx = I.lev[lf].nx, fy = I.lev[lf].ny, px = fused_pitch(fx), hxf = half_x(fx);
+  // this wave's columns of the last level's inverse, rows on the lanes
+  const int dx = I.lev[last].nx, dn = dx * I.lev[last].ny;
+  T dv[DC];
+#pragma unroll
+  for (int c = 0; c < DC; ++c) {
+    const int col = wave * DC + c;
+    dv[c] = col < dn && lane < dn ? ld32(cptr<T>(I.lev[last].dinv), (uint32_t)(col * dn + lane)) : T(0);
   }
+  for (int k = tid; k < XN; k += kFuseThreads) { sx[k] = T(0); sb[kDense + k] = T(0); }
   lds_barrier();
-  int xo = 0, bo = 0;   // LDS offsets of the level's x and b (b of level lf is in global memory)
+  for (int c = tid; c < fx * fy; c += kFuseThreads) {
+    const int j = c / fx, i = xcol(c - j * fx, hxf);
+    const T v = ld32(bg, (uint32_t)c);
+    sb[lf == last ? j * fx + i : kDense + (j + 1) * px + 1 + i] = v;
+  }
 
-  // cell (i, j) of step u on line li
-  auto place = [&](int dir, int li, int u, int &i, int &j) { i = dir ? li : u; j = dir ? u : li; };
-
-  // One level's down-sweeps and restriction, up-sweeps; RR: rounds it needs.
-  auto sweep = [&](auto dirc, auto rc, const Lev &L, bool nine, const CellEq<T> *q, int colour,
-                   const T *b, bool zero) {
-    constexpr int DIR = decltype(dirc)::value, RR = decltype(rc)::value;
-    const int n = DIR == 0 ? nx : ny, np = DIR == 0 ? ny : nx;
-    const int W = seg_width(n), lw = 31 - __builtin_clz(W), nl = (np - colour + 1) >> 1;
-    const int px = fused_pitch(nx);
-    T *const x = sx + xo + px + 1;
-#pragma unroll
-    for (int r = 0; r < RR; ++r) {
-      const int idx = tid + r * kFuseThreads, u = idx & (W - 1), k = idx >> lw;
-      if (((idx & ~63) >> lw) >= nl) continue;   // uniform over the wave
-      const bool on = k < nl && u < n;
-      int i, j;
-      place(DIR, colour + 2 * k, u, i, j);
-      const int ix = on ? j * px + i : 0;
-      T rhs = b[r];
-      if (!zero) rhs -= beside(q[r], x, ix, DIR == 0 ? 1 : px, DIR == 0 ? px : 1);
-      const T v = solve_line(q[r], on ? rhs : T(0), u, W);
-      if (on) x[ix] = v;
-    }
-    lds_barrier();
-  };
-  // equations and right-hand sides of one colour's cells
-  auto load = [&](auto dirc, auto rc, const Lev &L, bool nine, bool first, CellEq<T> *q, T *b,
-                  int colour) {
-    constexpr int DIR = decltype(dirc)::value, RR = decltype(rc)::value;
-    const int n = DIR == 0 ? nx : ny, np = DIR == 0 ? ny : nx, hx = half_x(nx);
-    const int W = seg_width(n), lw = 31 - __builtin_clz(W), nl = (np - colour + 1) >> 1;
-#pragma unroll
-    for (int r = 0; r < RR; ++r) {
-      const int idx = tid + r * kFuseThreads, u = idx & (W - 1), k = idx >> lw;
-      const bool on = k < nl && u < n;
-      int i, j;
-      place(DIR, colour + 2 * k, u, i, j);
-      const uint32_t K = on ? j * nx + xslot(i, hx) : 0;
-      q[r] = cell_eq<T, DIR>(L, nine, K, on);
-      b[r] = !on ? T(0) : first ? ld32(bg, K) : sb[bo + j * nx + i];
+  // Operands of a task, loaded while the one before runs: K steps of up to 9
+  // arrays (TK_RES: 6 couplings and 2 weights; TK_PRO: 4 weights).
+  T v[9][4];
+  auto fetch = [&](const CoarseTask &t) __attribute__((always_inline)) {
+    if ((tid & ~63) >= t.lanes) return;   // no line in this wave
+    const uint32_t s = t.lanes * t.K, o = t.pack + tid * t.K;
+    if (t.K == 4) {
+      if (t.kind == TK_PRO) load_pack<4, 0, 4>(pack, o, s, v);
+      else {
+        if (t.kind != TK_RES) load_pack<4, 0, 3>(pack, o, s, v);
+        else load_pack<4, 0, 2>(pack, t.pack2 + 4 * tid, s, v);
+        if (t.kind != TK_ZERO) load_pack<4, 3, 6>(pack, o + 3 * s, s, v);
+      }
+    } else {
+      if (t.kind == TK_PRO) load_pack<1, 0, 4>(pack, o, s, v);
+      else {
+        if (t.kind != TK_RES) load_pack<1, 0, 3>(pack, o, s, v);
+        else load_pack<1, 0, 2>(pack, t.pack2 + tid, s, v);
+        if (t.kind != TK_ZERO) load_pack<1, 3, 6>(pack, o + 3 * s, s, v);
+      }
     }
   };
-  std::integral_constant<int, 0> X;
-  std::integral_constant<int, 1> Y;
+  // A task by K steps per lane. The operands' registers are refilled for the
+  // next task as soon as they are used up.
+  auto lines = [&](auto kc, const CoarseTask &t, const CoarseTask &tn) __attribute__((always_inline)) {
+    constexpr int K = decltype(kc)::value;
+    const int u = tid & ((1 << t.lw) - 1), k = tid >> t.lw;
+    const int t0 = min(K * u, t.n);   // lanes past the end of the line stay near it
+    const bool line = k < t.nl;
+    T *const x = sx + t.x0 + 2 * min(k, t.nl - 1) * t.sp + t0 * t.sl;
+    const int sl = t.sl, sp_ = t.sp;
+    if (t.kind == TK_PRO) {   // odd rows, which alone are read before they are solved
+      const T *const c = sx + t.aux + min(k, t.nl - 1) * t.pc + (t0 >> 1);
+      T w[4][K], xo[K], s[3], n[3];
+#pragma unroll
+      for (int a = 0; a < 4; ++a)
+#pragma unroll
+        for (int e = 0; e < K; ++e) w[a][e] = v[a][e];
+#pragma unroll
+      for (int e = 0; e < (K == 1 ? 2 : 3); ++e) { s[e] = c[e]; n[e] = c[t.pc + e]; }
+#pragma unroll
+      for (int e = 0; e < K; ++e) xo[e] = x[e];
+#pragma unroll
+      for (int e = 0; e < K; ++e)
+        xo[e] += w[0][e] * s[e / 2] + w[1][e] * s[e / 2 + 1] + w[2][e] * n[e / 2] + w[3][e] * n[e / 2 + 1];
+      fetch(tn);
+#pragma unroll
+      for (int e = 0; e < K; ++e)
+        if (line && K * u + e < t.n) x[e] = xo[e];
+      return;
+    }
+    T r[K];
+    if (t.kind != TK_ZERO) {
+      T xm[K + 2], xp[K + 2];
+#pragma unroll
+      for (int e = 0; e < K + 2; ++e) {
+        xm[e] = x[(e - 1) * sl - sp_];
+        xp[e] = x[(e - 1) * sl + sp_];
+      }
+#pragma unroll
+      for (int e = 0; e < K; ++e) {
+        T s = v[3][e] * xm[e + 1] + v[4][e] * xp[e + 1];
+        s += v[5][e] * xm[e] + v[6][e] * xm[e + 2];
+        s += v[7][e] * xp[e] + v[8][e] * xp[e + 2];
+        r[e] = -s;
+      }
+    } else {
+#pragma unroll
+      for (int e = 0; e < K; ++e) r[e] = T(0);
+    }
+    if (t.kind == TK_RES) {
+      // The even rows satisfy their equations with the odd rows at zero, so
+      // after colour 1 their residual is what the odd rows contribute, r =
+      // -(couplings to the odd rows) x; that of the odd rows vanishes. b of
+      // the coarse point at an even column: the odd columns beside it send
+      // their weighted residuals (a line's last column sends nothing on: its
+      // weight is zero, so the lines of a row need no mask).
+      T *const c = sb + t.aux + min(k, t.nl - 1) * t.pc + (t0 >> 1);
+      if constexpr (K == 1) {
+        const T o = dpp0<kRowShr | 1>(v[1][0] * r[0]) + r[0] + dpp0<kRowShl | 1>(v[0][0] * r[0]);
+        fetch(tn);
+        if (line && u < t.n && !(u & 1)) c[0] = o;
+      } else {
+        const T west = dpp0<kRowShr | 1>(v[1][3] * r[3]);
+        const T o0 = west + r[0] + v[0][1] * r[1];
+        const T o1 = v[1][1] * r[1] + r[2] + v[0][3] * r[3];
+        fetch(tn);
+        if (line && K * u < t.n) c[0] = o0;
+        if (line && K * u + 2 < t.n) c[1] = o1;
+      }
+      return;
+    }
+    // Gauss-Seidel on the lines: d_t = al d_{t-1} + (b_t + r_t) inv_t, then
+    // x_t = nup x_{t+1} + d_t
+    const T *const b = sb + kDense + (x - sx);
+    T al[K], up[K];
+#pragma unroll
+    for (int e = 0; e < K; ++e) {
+      al[e] = v[0][e];
+      up[e] = v[2][e];
+      r[e] = (b[e * sl] + r[e]) * v[1][e];
+    }
+    fetch(tn);
+    if constexpr (K == 1) {
+      r[0] = scan_row0<true>(al[0], r[0]);
+      r[0] = scan_row0<false>(up[0], r[0]);
+    } else {
+      T A = T(1), B = T(0);
+#pragma unroll
+      for (int e = 0; e < K; ++e) { B = al[e] * B + r[e]; A = e ? al[e] * A : al[e]; }
+      T d = dpp0<kRowShr | 1>(scan_row0<true>(A, B));
+#pragma unroll
+      for (int e = 0; e < K; ++e) { d = al[e] * d + r[e]; r[e] = d; }
+      B = T(0);
+#pragma unroll
+      for (int e = K - 1; e >= 0; --e) { B = up[e] * B + r[e]; A = e < K - 1 ? up[e] * A : up[e]; }
+      T xv = dpp0<kRowShl | 1>(scan_row0<false>(A, B));
+#pragma unroll
+      for (int e = K - 1; e >= 0; --e) { xv = up[e] * xv + r[e]; r[e] = xv; }
+    }
+#pragma unroll
+    for (int e = 0; e < K; ++e)
+      if (line && K * u + e < t.n) x[e * sl] = r[e];
+  };
 
-  auto down = [&](auto rc, int m, bool first) {
-    constexpr int RR = decltype(rc)::value;
-    const Lev &L = I.lev[m];
-    const bool nine = m > 0;
-    const int hx = half_x(nx), px = fused_pitch(nx);
-    const int cx = (nx + 1) >> 1, cy = (ny + 1) >> 1;
-    T *const bc = sb + (first ? 0 : bo + nx * ny);
-    if (sched(m) & 1) {
-      // pre-smoothing with x-lines from x = 0: colour 0 from b alone; the
-      // even rows then satisfy their equations with the odd rows at zero, so
-      // after colour 1 their residual is what the odd rows contribute,
-      // r = -(couplings to the odd rows) x, and that of the odd rows vanishes
-      CellEq<T> q0[RR], q1[RR];
-      T b0[RR], b1[RR], w0[RR], w1[RR];
-      load(X, rc, L, nine, first, q0, b0, 0);
-      load(X, rc, L, nine, first, q1, b1, 1);
-      const int W = seg_width(nx), lw = 31 - __builtin_clz(W), nl = (ny + 1) >> 1;
-#pragma unroll
-      for (int r = 0; r < RR; ++r) {   // weights of the odd columns of the even rows
-        const int idx = tid + r * kFuseThreads, u = idx & (W - 1), k = idx >> lw;
-        const bool odd = k < nl && u < nx && (u & 1);
-        const uint32_t K = 2 * k * nx + xslot(u, hx);
-        w0[r] = odd ? ld32(cptr<T>(L.pw[0]), K) : T(0);
-        w1[r] = odd ? ld32(cptr<T>(L.pw[1]), K) : T(0);
+  CoarseTask t = load_task(tasks, 0);
+  fetch(t);
+#pragma unroll 1
+  for (int it = 1; t.kind != TK_END; ++it) {
+    const CoarseTask tn = load_task(tasks, it);
+    lds_barrier();   // the task before is done
+    if (t.kind <= TK_RES || t.kind == TK_PRO) {
+      if ((tid & ~63) < t.lanes) {   // the wave has a line
+        if (t.K == 4) lines(std::integral_constant<int, 4>(), t, tn);
+        else lines(std::integral_constant<int, 1>(), t, tn);
+      } else {
+        fetch(tn);
       }
-      sweep(X, rc, L, nine, q0, 0, b0, true);
-      sweep(X, rc, L, nine, q1, 1, b1, false);
-      const T *const x = sx + xo + px + 1;
-#pragma unroll
-      for (int r = 0; r < RR; ++r) {
-        const int idx = tid + r * kFuseThreads, u = idx & (W - 1), k = idx >> lw;
-        if (((idx & ~63) >> lw) >= nl) continue;
-        const bool on = k < nl && u < nx;
-        const T res = on ? -beside(q0[r], x, 2 * k * px + u, 1, px) : T(0);
-        // b of the coarse point at column u (even): the odd columns beside it
-        // send their weighted residuals
-        const T east = __shfl_down(w0[r] * res, 1, W), west = __shfl_up(w1[r] * res, 1, W);
-        if (on && !(u & 1)) {
-          T s = u > 0 ? west : T(0);
-          s += res;
-          s += u + 1 < nx ? east : T(0);
-          bc[k * cx + (u >> 1)] = s;
-        }
-      }
-    } else {   // x = 0: b of the next level is the restriction of b
-      for (int c = tid; c < cx * cy; c += kFuseThreads) {
-        const int J = c / cx, Ic = c - J * cx;
+    } else {
+      fetch(tn);
+      const Lev &L = I.lev[t.lev];
+      const int nx = L.nx, ny = L.ny, hx = half_x(nx);
+      if (t.kind == TK_DENSE) {
         T s = T(0);
 #pragma unroll
-        for (int db = -1; db <= 1; ++db)
+        for (int c = 0; c < DC; ++c) s += dv[c] * (wave * DC + c < dn ? sb[wave * DC + c] : T(0));
+        sp[wave * kDense + lane] = s;
+        lds_barrier();
+        if (tid < dn) {
+          T o = T(0);
 #pragma unroll
-          for (int da = -1; da <= 1; ++da) {
-            const int fi = 2 * Ic + da, fj = 2 * J + db;
-            if (fi < 0 || fi >= nx || fj < 0 || fj >= ny) continue;
-            const uint32_t K = fj * nx + xslot(fi, hx);
+          for (int w = 0; w < NW; ++w) o += sp[w * kDense + tid];
+          const int j = tid / dx;
+          sx[t.x0 + j * t.sp + tid - j * dx] = o;
+        }
+      } else if (t.kind == TK_RESTB) {   // x = 0: the restriction of b
+        const int cx = (nx + 1) >> 1, cy = (ny + 1) >> 1;
+        for (int c = tid; c < cx * cy; c += kFuseThreads) {
+          const int J = c / cx, Ic = c - J * cx;
+          // all loads first; points outside the grid weigh zero and have the
+          // border's b
+          T w[9];
+#pragma unroll
+          for (int m = 0; m < 9; ++m) {
+            const int da = m % 3 - 1, db = m / 3 - 1, fi = 2 * Ic + da, fj = 2 * J + db;
+            const bool in = fi >= 0 && fi < nx && fj >= 0 && fj < ny;
             const int slot = (da < 0 ? 1 : 0) + 2 * (db < 0 ? 1 : 0);
-            const T w = da == 0 && db == 0 ? T(1) : ld32(cptr<T>(L.pw[slot]), K);
-            s += w * (first ? ld32(bg, K) : sb[bo + fj * nx + fi]);
+            const uint32_t K = in ? fj * nx + xslot(fi, hx) : 0;
+            w[m] = m == 4 ? T(1) : ld32(cptr<T>(L.pw[slot]), K);
+            w[m] = in ? w[m] : T(0);
           }
-        bc[c] = s;
+          T s = T(0);
+          const T *const bf = sb + t.x0 + 2 * J * t.sp + 2 * Ic;
+#pragma unroll
+          for (int m = 0; m < 9; ++m) s += w[m] * bf[(m / 3 - 1) * t.sp + m % 3 - 1];
+          sb[t.aux + J * t.pc + Ic] = s;
+        }
+      } else {   // TK_PROALL: x += P xc at every cell
+        for (int c = tid; c < nx * ny; c += kFuseThreads) {
+          const int j = c / nx, i = c - j * nx;
+          const uint32_t K = j * nx + xslot(i, hx);
+          const bool io = i & 1, jo = j & 1;
+          const T *const xc = sx + t.aux + (j >> 1) * t.pc + (i >> 1);
+          T e = xc[0];
+          if (io || jo) e *= ld32(cptr<T>(L.pw[0]), K);
+          if (io) e += ld32(cptr<T>(L.pw[1]), K) * xc[1];
+          if (jo) e += ld32(cptr<T>(L.pw[2]), K) * xc[t.pc];
+          if (io && jo) e += ld32(cptr<T>(L.pw[3]), K) * xc[t.pc + 1];
+          sx[t.x0 + j * t.sp + i] += e;
+        }
       }
     }
-    lds_barrier();
-  };
-
-  auto up = [&](auto rc, int m, bool first, int xc_off, int cx) {
-    constexpr int RR = decltype(rc)::value;
-    const Lev &L = I.lev[m];
-    const bool nine = m > 0;
-    const int hx = half_x(nx), px = fused_pitch(nx), pc = fused_pitch(cx);
-    const int sml = sched(m);
-    const bool post_x = sml & 4, post_y = sml & 8;
-    T *const x = sx + xo + px + 1;
-    const T *const xc = sx + xc_off + pc + 1;
-    CellEq<T> q0[RR], q1[RR];
-    T b0[RR], b1[RR];
-    // x += P xc at cell (i, j); the weights that are 0 or 1 are not stored
-    auto correct = [&](int i, int j) {
-      const uint32_t K = j * nx + xslot(i, hx);
-      const bool io = i & 1, jo = j & 1;
-      const T *const c = xc + (j >> 1) * pc + (i >> 1);
-      T w0 = T(1), w1 = T(0), w2 = T(0), w3 = T(0);
-      if (io || jo) w0 = ld32(cptr<T>(L.pw[0]), K);
-      if (io) w1 = ld32(cptr<T>(L.pw[1]), K);
-      if (jo) w2 = ld32(cptr<T>(L.pw[2]), K);
-      if (io && jo) w3 = ld32(cptr<T>(L.pw[3]), K);
-      T e = w0 * c[0];
-      e += w1 * c[1];
-      e += w2 * c[pc];
-      e += w3 * c[pc + 1];
-      x[j * px + i] += e;
-    };
-    if (post_x) {
-      load(X, rc, L, nine, first, q0, b0, 0);
-      load(X, rc, L, nine, first, q1, b1, 1);
-      // only the odd rows are read before they are solved
-      for (int c = tid; c < nx * (ny >> 1); c += kFuseThreads) {
-        const int k = c / nx;
-        correct(c - k * nx, 2 * k + 1);
-      }
-      lds_barrier();
-      sweep(X, rc, L, nine, q0, 0, b0, false);
-      sweep(X, rc, L, nine, q1, 1, b1, false);
-    } else {
-      for (int c = tid; c < nx * ny; c += kFuseThreads) {
-        const int j = c / nx;
-        correct(c - j * nx, j);
-      }
-      lds_barrier();
-    }
-    if (post_y) {
-      load(Y, rc, L, nine, first, q0, b0, 0);
-      load(Y, rc, L, nine, first, q1, b1, 1);
-      sweep(Y, rc, L, nine, q0, 0, b0, false);
-      sweep(Y, rc, L, nine, q1, 1, b1, false);
-    }
-  };
-
-  std::integral_constant<int, R> RF;
-  std::integral_constant<int, 1> R1;
-  for (int m = lf; m < last; ++m) {
-    if (m == lf) down(RF, m, true); else down(R1, m, false);
-    xo += fused_pitch(nx) * (ny + 2);
-    if (m > lf) bo += nx * ny;
-    nx = (nx + 1) >> 1; ny = (ny + 1) >> 1;
+    t = tn;
   }
-  {   // exact solve of the coarsest level: one row or one column
-    const Lev &L = I.lev[last];
-    CellEq<T> q[1];
-    T b[1];
-    if (ny == 1) { load(X, R1, L, last > 0, last == lf, q, b, 0); sweep(X, R1, L, last > 0, q, 0, b, true); }
-    else { load(Y, R1, L, last > 0, last == lf, q, b, 0); sweep(Y, R1, L, last > 0, q, 0, b, true); }
-  }
-  for (int m = last - 1; m >= lf; --m) {
-    const int cx = nx, xc = xo;
-    nx = I.lev[m].nx; ny = I.lev[m].ny;
-    xo -= fused_pitch(nx) * (ny + 2);
-    if (m > lf) bo -= nx * ny;
-    if (m == lf) up(RF, m, true, xc, cx); else up(R1, m, false, xc, cx);
-  }
+  lds_barrier();
   // x of the first level
-  const int hx = half_x(nx), px = fused_pitch(nx);
-  for (int c = tid; c < nx * ny; c += kFuseThreads) {
-    const int j = c / nx, p = c - j * nx;
-    st32(xg, (uint32_t)c, sx[(j + 1) * px + 1 + xcol(p, hx)]);
+  for (int c = tid; c < fx * fy; c += kFuseThreads) {
+    const int j = c / fx, i = xcol(c - j * fx, hxf);
+    st32(xg, (uint32_t)c, sx[(j + 1) * px + 1 + i]);
   }
+}
+
+void launch_dense_inverse(hipStream_t s, const InstDev *d, const FuseMap *m, int n, bool h32) {
+  if (!n) return;
+  if (h32) k_dense_inverse<float><<<n, 1024, 0, s>>>(d, m);
+  else k_dense_inverse<double><<<n, 1024, 0, s>>>(d, m);
+}
+void launch_coarse_pack(hipStream_t s, const InstDev *d, const PackMap *m, int n, bool h32) {
+  if (!n) return;
+  if (h32) k_coarse_pack<float><<<n, kFuseThreads, 0, s>>>(d, m);
+  else k_coarse_pack<double><<<n, kFuseThreads, 0, s>>>(d, m);
 }
 
 template <typename T>
 void launch_coarse_cycle(hipStream_t s, const InstDev *d, const FuseMap *m, int n, int xid, int bid,
-                         int smoother, int cap) {
+                         int cap) {
   if (!n) return;
-  if (cap <= 1024) k_coarse_cycle<T, 1><<<n, kFuseThreads, 0, s>>>(d, m, xid, bid, smoother);
-  else k_coarse_cycle<T, 2><<<n, kFuseThreads, 0, s>>>(d, m, xid, bid, smoother);
+  if (cap <= 1024) k_coarse_cycle<T, 1024><<<n, kFuseThreads, 0, s>>>(d, m, xid, bid);
+  else k_coarse_cycle<T, kFuseCells32><<<n, kFuseThreads, 0, s>>>(d, m, xid, bid);
 }
 template void launch_coarse_cycle<double>(hipStream_t, const InstDev *, const FuseMap *, int, int,
-                                          int, int, int);
+                                          int, int);
 template void launch_coarse_cycle<float>(hipStream_t, const InstDev *, const FuseMap *, int, int,
-                                         int, int, int);
+                                         int, int);
 
 }  // namespace sg

@@ -48,11 +48,12 @@ static size_t a256(size_t x) { return (x + 255) & ~size_t(255); }
 
 struct Dims { int nx, ny; };
 
-// Coarsen both directions (ceil halving) until one of them is 1; the last
-// level is then solved exactly by one line solve.
+// Coarsen both directions (ceil halving) until a level has at most kDense cells,
+// which the inverse of its operator solves, or one row or column, solved
+// exactly by one line solve.
 static std::vector<Dims> level_dims(int nx, int ny) {
   std::vector<Dims> v{{nx, ny}};
-  while (std::min(nx, ny) > 1) {
+  while (std::min(nx, ny) > 1 && nx * ny > kDense) {
     nx = (nx + 1) / 2;
     ny = (ny + 1) / 2;
     v.push_back({nx, ny});
@@ -98,6 +99,14 @@ static size_t carve(uintptr_t base, int nx, int ny, int prec, InstDev &I) {
                                                                                  : take(N * KT);
   for (int v = 0; v < kNumVecAll - kNumVec; ++v)
     I.pv[v] = prec == SG_PC32 ? (float *)take(N * sizeof(float)) : nullptr;
+  // fused coarse cycle: its task table and packed operator, for the largest
+  // first level it may have
+  I.tasks = (const CoarseTask *)take(kMaxTasks * sizeof(CoarseTask));
+  size_t packed = 0;
+  for (size_t l = 0; l + 1 < dims.size(); ++l)
+    if (std::max(dims[l].nx, dims[l].ny) <= kFuseSide)
+      packed += pack_offset(dims[l].nx, dims[l].ny, kNumPack);
+  I.pack = packed ? take(packed * T) : nullptr;
   for (int l = 0; l < kMaxLev; ++l) {
     Lev &L = I.lev[l];
     std::memset(&L, 0, sizeof(L));
@@ -119,10 +128,14 @@ static size_t carve(uintptr_t base, int nx, int ny, int prec, InstDev &I) {
     }
     if (l + 1 < I.nlev)
       for (int q = 0; q < 4; ++q) L.pw[q] = take(Nl * T);
-    for (int d = 0; d < 2; ++d) {
+    const bool dense = l + 1 == I.nlev && Nl <= kDense;
+    for (int d = 0; d < 2 && !dense; ++d) {
       L.linv[d] = take(Nl * T);
       L.lup[d] = take(Nl * T);
     }
+    if (dense) L.dinv = take(Nl * Nl * T);
+    // last: the vector loads of a row sweep may reach a few values past an
+    // array, into the next one
     L.cp = take(Nl * T);
     L.dp = nullptr;
   }
@@ -166,7 +179,8 @@ struct Maps {
   std::vector<LineGrp> swm[kMaxLev][2][2];
   int swm_na[kMaxLev][2][2], swm_nb[kMaxLev][2][2];
   bool swm_all[kMaxLev][2][2];
-  std::vector<FuseMap> fmap;
+  std::vector<FuseMap> fmap, dmap;   // dmap: the instances whose last level is dense
+  std::vector<PackMap> kmap;         // packed arrays of the fused levels
 };
 
 // Tile shape of a line solve by line length and direction: short lines in
@@ -274,8 +288,9 @@ struct DevMaps {   // offsets into one device buffer
   const LineGrp *swm[kMaxLev][2][2];
   int nswm[kMaxLev][2][2], swm_na[kMaxLev][2][2], swm_nb[kMaxLev][2][2];
   bool swm_all[kMaxLev][2][2];
-  const FuseMap *fmap;
-  int nfmap;
+  const FuseMap *fmap, *dmap;
+  const PackMap *kmap;
+  int nfmap, ndmap, nkmap;
   int maxlev;
 };
 
@@ -359,6 +374,8 @@ struct Batch {
   int remove(int slot);
   int rebuild();
   int fuse_level(const InstDev &I) const;
+  // largest fused level: the default takes any with sides of at most kFuseSide
+  int fuse_cap() const { return opts.fuse_cells == kFuseCells ? kFuseCells32 : opts.fuse_cells; }
   int step(int nsteps, const int64_t *targets, int ntargets);
   int step_once();
   bool graphs_on() const { return opts.use_graph >= 0 && time_mask == 0; }
@@ -588,6 +605,99 @@ int Batch::upload_bc(Slot &s, int side, const double *vals) {
   return SG_OK;
 }
 
+static bool dense_last(const InstDev &I) {
+  const Lev &L = I.lev[I.nlev - 1];
+  return L.nx * L.ny <= kDense;
+}
+
+// First level of an instance's fused coarse cycle: its first level that fits,
+// but only its dense last level when fusion is off or the schedule has a
+// y-line pre-sweep (which the fused cycle does not run); nlev (none) when the
+// last level is a line. It depends only on the instance and the options.
+int Batch::fuse_level(const InstDev &I) const {
+  if (!dense_last(I)) return I.nlev;
+  if (opts.fuse_cells >= 0 && !((opts.smoother | opts.coarse_smoother) & 2))
+    for (int l = 0; l < I.nlev; ++l)
+      if (std::max(I.lev[l].nx, I.lev[l].ny) <= kFuseSide &&
+          I.lev[l].nx * I.lev[l].ny <= fuse_cap())
+        return l;
+  return I.nlev - 1;
+}
+
+// The phases of an instance's fused coarse cycle from level lf: per level on
+// the way down an x-line pre-sweep and the restriction of its residual (or the
+// restriction of b), the dense solve, per level on the way up the prolongation
+// and the post-sweeps.
+static std::vector<CoarseTask> coarse_tasks(const InstDev &I, int lf, const sg_opts &o) {
+  const int last = I.nlev - 1;
+  std::vector<CoarseTask> v;
+  std::vector<int> xo(1, 0), pk(1, 0);   // by level: places in LDS, packed arrays
+  for (int l = lf; l <= last; ++l) {
+    const int nx = I.lev[l].nx, ny = I.lev[l].ny;
+    xo.push_back(xo.back() + fused_pitch(nx) * (ny + 2));
+    pk.push_back(pk.back() + (l < last ? pack_offset(nx, ny, kNumPack) : 0));
+  }
+  auto place = [&](int l, int i, int j) {
+    return xo[l - lf] + (j + 1) * fused_pitch(I.lev[l].nx) + 1 + i;
+  };
+  // the lines of packed kind `kind` of level l
+  auto lines = [&](int task, int l, int kind) {
+    const int nx = I.lev[l].nx, ny = I.lev[l].ny, px = fused_pitch(nx);
+    const bool col = kind == PK_COL0 || kind == PK_COL1;
+    const int colour = kind == PK_ROW1 || kind == PK_COL1 || kind == PK_PRO;
+    const LineLanes g = pack_lanes(nx, ny, kind);
+    CoarseTask t{};
+    t.kind = task; t.K = g.K; t.lw = g.lw; t.nl = g.nl; t.lanes = g.lanes; t.lev = l;
+    t.n = col ? ny : nx;
+    t.x0 = col ? place(l, colour, 0) : place(l, 0, colour);
+    t.sl = col ? px : 1;
+    t.sp = col ? 1 : px;
+    t.pack = pk[l - lf] + pack_offset(nx, ny, kind);
+    t.pack2 = pk[l - lf] + pack_offset(nx, ny, PK_RES);
+    return t;
+  };
+  auto cells = [&](int task, int l) {
+    CoarseTask t{};
+    t.kind = task; t.lev = l;
+    t.x0 = place(l, 0, 0) + (task == TK_RESTB ? kDense : 0);
+    t.sp = fused_pitch(I.lev[l].nx);
+    return t;
+  };
+  for (int l = lf; l < last; ++l) {
+    const int s = l == 0 ? o.smoother : o.coarse_smoother;
+    // b of the next level: the dense one's in row order, else bordered
+    const int aux = l + 1 == last ? 0 : kDense + place(l + 1, 0, 0);
+    const int pc = l + 1 == last ? I.lev[last].nx : fused_pitch(I.lev[l + 1].nx);
+    if (s & 1) {
+      v.push_back(lines(TK_ZERO, l, PK_ROW0));
+      v.push_back(lines(TK_SWEEP, l, PK_ROW1));
+      v.push_back(lines(TK_RES, l, PK_ROW0));
+    } else {
+      v.push_back(cells(TK_RESTB, l));
+    }
+    v.back().aux = aux;
+    v.back().pc = pc;
+  }
+  v.push_back(cells(TK_DENSE, last));
+  for (int l = last - 1; l >= lf; --l) {
+    const int s = l == 0 ? o.smoother : o.coarse_smoother;
+    v.push_back(s & 4 ? lines(TK_PRO, l, PK_PRO) : cells(TK_PROALL, l));
+    v.back().aux = place(l + 1, 0, 0);
+    v.back().pc = fused_pitch(I.lev[l + 1].nx);
+    if (s & 4) {
+      v.push_back(lines(TK_SWEEP, l, PK_ROW0));
+      v.push_back(lines(TK_SWEEP, l, PK_ROW1));
+    }
+    if (s & 8) {
+      v.push_back(lines(TK_SWEEP, l, PK_COL0));
+      v.push_back(lines(TK_SWEEP, l, PK_COL1));
+    }
+  }
+  v.push_back(CoarseTask{});
+  v.back().kind = TK_END;
+  return v;
+}
+
 int Batch::add(const sg_grid *g, const sg_coeffs *c, const sg_bc *bc, const double *f0, double dt,
                int *slot_out) {
   int rc;
@@ -648,6 +758,13 @@ int Batch::add(const sg_grid *g, const sg_coeffs *c, const sg_bc *bc, const doub
   vertex_weights(g->y_edges, ny, w0, w1);
   (void)hipMemcpy((void *)s.dev.wy0, w0.data(), (ny + 1) * 8, hipMemcpyHostToDevice);
   (void)hipMemcpy((void *)s.dev.wy1, w1.data(), (ny + 1) * 8, hipMemcpyHostToDevice);
+  if (dense_last(s.dev)) {
+    const std::vector<CoarseTask> t = coarse_tasks(s.dev, fuse_level(s.dev), opts);
+    if (t.size() > (size_t)kMaxTasks ||
+        hipMemcpy((void *)s.dev.tasks, t.data(), t.size() * sizeof(CoarseTask),
+                  hipMemcpyHostToDevice) != hipSuccess)
+      return undo(fail(SG_ERR_HIP, "upload of the coarse cycle's tasks failed"));
+  }
   if (!c->inv_tau && hipMemsetAsync((void *)s.dev.itau, 0, N * 8, stream) != hipSuccess)
     return undo(fail(SG_ERR_HIP, "clearing 1/tau failed"));
   if ((rc = set_coeffs(s, c))) return undo(rc);
@@ -683,19 +800,6 @@ int Batch::remove(int slot) {
   return SG_OK;
 }
 
-// First level of an instance's fused coarse cycle: its first level with at
-// most fuse_cells cells; nlev (none) when fusion is off, when the schedule
-// pre-smooths (the fused cycle implements post-smoothing) or when no level is
-// that small. It depends only on the instance and the options.
-int Batch::fuse_level(const InstDev &I) const {
-  // the fused cycle runs post-smoothing, optionally after an x-line pre-sweep
-  if (opts.fuse_cells < 0 || ((opts.smoother | opts.coarse_smoother) & 2)) return I.nlev;
-  for (int l = 0; l < I.nlev; ++l)
-    if (std::max(I.lev[l].nx, I.lev[l].ny) <= kFuseSide && I.lev[l].nx * I.lev[l].ny <= opts.fuse_cells)
-      return l;
-  return I.nlev;
-}
-
 void Batch::drop_graphs() {
   for (auto &g : graphs) (void)hipGraphExecDestroy(g.exec);
   graphs.clear();
@@ -720,6 +824,13 @@ int Batch::rebuild() {
     const int lf = fuse_level(I);
     slots[k].fuse_lev = lf;
     if (lf < I.nlev) M.fmap.push_back({c, lf});
+    const bool dense = dense_last(I);
+    if (dense) M.dmap.push_back({c, I.nlev - 1});
+    for (int l = lf, off = 0; l + 1 < I.nlev; ++l) {
+      for (int kind = 0; kind < kNumPack; ++kind)
+        M.kmap.push_back({c, l, kind, off + pack_offset(I.lev[l].nx, I.lev[l].ny, kind)});
+      off += pack_offset(I.lev[l].nx, I.lev[l].ny, kNumPack);
+    }
     for (int l = 0; l < I.nlev; ++l) {
       const int lx = I.lev[l].nx, ly = I.lev[l].ny, Nl = lx * ly;
       const bool coarsest = (l == I.nlev - 1);
@@ -734,6 +845,7 @@ int Batch::rebuild() {
       const int nq = prow == 1 ? lx * (ly >> 1) : prow == 2 ? (lx - half_x(lx)) * ly : Nl;
       if (!coarsest && l < lf)
         for (int k0 = 0; k0 < nq; k0 += kBlock) M.qmap[l].push_back({c, k0});
+      if (coarsest && dense) continue;
       if (coarsest) {
         LineGrp g{c, 0, 1, 1};
         auto &set = ly == 1 ? M.gcx[l][tile_shape(lim, lx, 0, l, f64)]
@@ -814,6 +926,8 @@ int Batch::rebuild() {
   size_t bytes = 0;
   auto sz = [&](size_t n, size_t e) { bytes += a256(n * e); };
   sz(M.fmap.size(), sizeof(FuseMap));
+  sz(M.dmap.size(), sizeof(FuseMap));
+  sz(M.kmap.size(), sizeof(PackMap));
   for (int l = 0; l < kMaxLev; ++l) {
     sz(M.cmap[l].size(), sizeof(BlkMap)); sz(M.pmap[l].size(), sizeof(BlkMap));
     sz(M.rmap[l].size(), sizeof(BlkMap)); sz(M.qmap[l].size(), sizeof(BlkMap));
@@ -847,6 +961,10 @@ int Batch::rebuild() {
   DevMaps dmn{};
   dmn.fmap = (const FuseMap *)put(M.fmap.data(), M.fmap.size(), sizeof(FuseMap));
   dmn.nfmap = (int)M.fmap.size();
+  dmn.dmap = (const FuseMap *)put(M.dmap.data(), M.dmap.size(), sizeof(FuseMap));
+  dmn.ndmap = (int)M.dmap.size();
+  dmn.kmap = (const PackMap *)put(M.kmap.data(), M.kmap.size(), sizeof(PackMap));
+  dmn.nkmap = (int)M.kmap.size();
   for (int l = 0; l < kMaxLev; ++l) {
     dmn.cmap[l] = (const BlkMap *)put(M.cmap[l].data(), M.cmap[l].size(), sizeof(BlkMap));
     dmn.ncmap[l] = (int)M.cmap[l].size();
@@ -1025,7 +1143,7 @@ template <typename T> void Batch::vcycle(int l, int xid, int bid) {
   if (!deeper && m.nfmap) {
     tbegin(11);
     launch_coarse_cycle<T>(stream, d_insts, m.fmap, m.nfmap, xid, bid,
-                           opts.smoother | opts.coarse_smoother << 4, opts.fuse_cells);
+                           fuse_cap());
     tend(11);
   }
   if (pre_x) sweep(0);
@@ -1121,8 +1239,8 @@ void Batch::setup_kernels(bool start64) {
                mixed ? opts.max_inner : opts.max_iters, opts.max_iters);
   tbegin(0); launch_assemble(stream, d_insts, dm.cmap[0], nb0); tend(0);
   // LU factors of the line matrices of level l: smoothing lines of both
-  // colours (one launch per direction and tile shape) and the exact solve on
-  // the coarsest level
+  // colours (one launch per direction and tile shape) and the exact solve of
+  // a last level that is a line
   auto factors = [&](int l, hipStream_t s) {
     for (int d = 0; d < 2; ++d)
       for (int sh = 0; sh < kNumTileShapes; ++sh)
@@ -1149,8 +1267,10 @@ void Batch::setup_kernels(bool start64) {
       note(hipStreamWaitEvent(side, ev_lev[l], 0));
       factors(l, side);
     }
+    launch_dense_inverse(stream, d_insts, dm.dmap, dm.ndmap, h32);
     note(hipEventRecord(ev_join, side));
     note(hipStreamWaitEvent(stream, ev_join, 0));
+    launch_coarse_pack(stream, d_insts, dm.kmap, dm.nkmap, h32);
   } else {
     for (int l = 0; l < dm.maxlev; ++l) {
       tbegin(1);
@@ -1161,6 +1281,10 @@ void Batch::setup_kernels(bool start64) {
       }
       tend(1);
     }
+    tbegin(1);
+    launch_dense_inverse(stream, d_insts, dm.dmap, dm.ndmap, h32);
+    launch_coarse_pack(stream, d_insts, dm.kmap, dm.nkmap, h32);
+    tend(1);
   }
   if (start64) {
     tbegin(12); launch_finish<double>(stream, FIN_INIT64, d_insts, n, d_cnt); tend(12);

@@ -125,6 +125,51 @@ __host__ __device__ inline size_t cell_slot(int i, int j, int nx) {
 
 // band slots; level 0 uses the first five (the operator is 5-point), coarse
 // Galerkin levels use all nine.
+// The fused coarse cycle. The lanes of a sweep colour: a line of n cells is a
+// segment of W lanes (a power of two, at most 16), K steps each; lanes counts
+// whole waves.
+struct LineLanes { int K, lw, nl, lanes; };
+__host__ __device__ constexpr LineLanes line_lanes(int n, int np, int colour) {
+  LineLanes a{n > 16 ? 4 : 1, 0, (np - colour + 1) >> 1, 0};
+  while ((a.K << a.lw) < n) ++a.lw;
+  a.lanes = ((a.nl << a.lw) + 63) & ~63;
+  return a;
+}
+// (odd pitch: a column's stride then spreads over the LDS banks)
+__host__ __device__ constexpr int fused_pitch(int nx) { return (nx + 2) | 1; }
+// Its operator, packed per step in the order its lanes read it, one group of
+// arrays per level and kind: rows and columns of either colour (9 arrays: -lo
+// inv, inv, -up, and the couplings to the lines beside), the weights of the
+// residual's restriction (2, rows of colour 0) and of the prolongation (4,
+// rows of colour 1). Offsets in values from the level's start.
+enum PackKind { PK_ROW0, PK_ROW1, PK_COL0, PK_COL1, PK_RES, PK_PRO, kNumPack };
+__host__ __device__ constexpr int pack_arrays(int kind) {
+  return kind < PK_RES ? 9 : kind == PK_RES ? 2 : 4;
+}
+__host__ __device__ constexpr LineLanes pack_lanes(int nx, int ny, int kind) {
+  return kind == PK_COL0 || kind == PK_COL1
+             ? line_lanes(ny, nx, kind == PK_COL1)
+             : line_lanes(nx, ny, kind == PK_ROW1 || kind == PK_PRO);
+}
+__host__ __device__ constexpr int pack_offset(int nx, int ny, int kind) {
+  int o = 0;
+  for (int k = 0; k < kind; ++k) {
+    const LineLanes a = pack_lanes(nx, ny, k);
+    o += pack_arrays(k) * a.lanes * a.K;
+  }
+  return o;
+}
+// One phase of the cycle (built once per instance on the host): what it does,
+// the lanes and lines it takes, and its places in LDS: x0 of the first line's
+// step 0, sl and sp the strides along and across the lines; pack: its arrays;
+// aux, pc: place and pitch in the next level (its b or x).
+enum TaskKind { TK_ZERO, TK_SWEEP, TK_RES, TK_RESTB, TK_DENSE, TK_PRO, TK_PROALL, TK_END };
+struct CoarseTask {
+  int kind, K, lw, n, nl, lanes, x0, sl, sp, pack, aux, pc, lev, pack2, pad[2];
+};
+static_assert(sizeof(CoarseTask) == 64, "one scalar load");
+constexpr int kMaxTasks = 64;
+
 enum Band { BC = 0, BW = 1, BE = 2, BS = 3, BN = 4, BSW = 5, BSE = 6, BNW = 7, BNE = 8 };
 
 // Krylov vector slots (precision of the Krylov iteration).
@@ -173,6 +218,9 @@ struct Lev {            // one multigrid level of one instance
   void *linv[2], *lup[2];   // LU factors of the row (0) and column (1) line
                             // matrices: 1/pivot and the eliminated upper entry
   void *x, *b, *cp, *dp;
+  void *dinv;           // last level of at most kDense cells: inverse operator,
+                        // entry (row r, column c) at c * cells + r, cells in
+                        // row order (j nx + i)
 };
 
 struct InstDev {
@@ -201,21 +249,31 @@ struct InstDev {
   double *partial;            // kNumPartials * nblk0
   unsigned int *ticket;       // 2 tickets
   KScal *sc;
+  // fused coarse cycle: its phases, and the packed operator (V-cycle precision)
+  const CoarseTask *tasks;
+  void *pack;
   Lev lev[kMaxLev];
 };
 
 struct BlkMap { int inst; int k0; };      // cell-parallel: 256 cells of one instance
 struct LineGrp { int inst; int first; int count; int step; };   // lines first + k*step, k < count
+struct PackMap { int inst, lev, kind, off; };   // off: of the kind's arrays in InstDev::pack
 struct FuseMap { int inst; int lev; };    // an instance whose levels from lev down run fused
 
 // The coarse end of a V-cycle runs in one workgroup per instance from the
 // first level with at most fuse_cells cells and no side above kFuseSide (a
 // line is then solved by the lanes of one wave): the fused coarse cycle.
-constexpr int kFuseCells = 1024;     // default, and the largest with FP64 V-cycles
+// The default cap takes every level with such sides: a 64 x 48 one costs the
+// cycle 12 us more and saves some nine launches of 4 us.
+constexpr int kFuseCells = 1024;     // default (any level that fits), and the
+                                     // largest other with FP64 V-cycles
 constexpr int kFuseCells32 = 4096;   // the largest with FP32 V-cycles
 constexpr int kFuseSide = 64;
+// Coarsening ends at the first level of at most kDense cells, which is solved by
+// the inverse of its operator (one wave's lanes are the rows).
+constexpr int kDense = 64;
 // Threads of the per-instance finish kernels (sums of the partials).
 constexpr int kFinThreads = 1024;
-constexpr int kFuseThreads = 1024;
+constexpr int kFuseThreads = 512;
 
 }  // namespace sg

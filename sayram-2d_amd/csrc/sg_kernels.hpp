@@ -50,14 +50,17 @@ void launch_restrict(hipStream_t s, const InstDev *d, const BlkMap *m, int nb, i
 template <typename T>
 void launch_prolong(hipStream_t s, const InstDev *d, const BlkMap *m, int nb, int l, bool zero,
                     int xid, int rows);
-// the fused coarse cycle of the instances in m (one workgroup each): post-
-// smoothing in x and/or y (smoother bits 4 and 8), optionally after an x-line
-// pre-sweep (bit 1); a y-line pre-sweep (bit 2) is not fused
-// cap: the largest level a fused instance may have (fuse_cells); it selects
-// the LDS layout of the kernel
+// inverse of the last level's operator of the instances in m (at most kDense
+// cells), in the V-cycle precision
+void launch_dense_inverse(hipStream_t s, const InstDev *d, const FuseMap *m, int n, bool h32);
+// the fused levels' operator in the order of the fused cycle's lanes
+void launch_coarse_pack(hipStream_t s, const InstDev *d, const PackMap *m, int n, bool h32);
+// the fused coarse cycle of the instances in m (one workgroup each) by their
+// task tables; cap: the largest level a fused instance may have (it selects the
+// LDS layout of the kernel)
 template <typename T>
 void launch_coarse_cycle(hipStream_t s, const InstDev *d, const FuseMap *m, int n, int xid, int bid,
-                         int smoother, int cap);
+                         int cap);
 // which: 0 p-update, 1 v = M ph, 2 s-update, 3 t = M sh, 4 x/r update.
 // pc: FP64 Krylov vectors with FP32 preconditioned vectors (T must be double).
 template <typename T>

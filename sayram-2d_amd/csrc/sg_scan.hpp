@@ -113,6 +113,30 @@ __device__ __forceinline__ T enter(T A, T B, const RowMaps<T> &m, int u, int W, 
   return Ae * v + Be;
 }
 
+// v moved by the DPP control CTRL inside the rows of 16 lanes; lanes without a
+// source get 0
+template <int CTRL> __device__ __forceinline__ float dpp0(float v) {
+  return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), CTRL,
+                                                               0xf, 0xf, true));
+}
+template <int CTRL> __device__ __forceinline__ double dpp0(double v) {
+  const long long s = __builtin_bit_cast(long long, v);
+  const unsigned lo = __builtin_amdgcn_update_dpp(0, (int)s, CTRL, 0xf, 0xf, true);
+  const unsigned hi = __builtin_amdgcn_update_dpp(0, (int)(s >> 32), CTRL, 0xf, 0xf, true);
+  return __builtin_bit_cast(double, (unsigned long long)hi << 32 | lo);
+}
+
+// B of the inclusive scan over a row of 16 lanes that starts from 0, for
+// segments whose first map has A = 0 (the recurrence starts anew there), so
+// that no lane needs to know where its segment begins.
+template <bool FWD, typename T> __device__ __forceinline__ T scan_row0(T A, T B) {
+  constexpr int C = FWD ? kRowShr : kRowShl;
+  B = A * dpp0<C | 1>(B) + B; A = A * dpp0<C | 1>(A);
+  B = A * dpp0<C | 2>(B) + B; A = A * dpp0<C | 2>(A);
+  B = A * dpp0<C | 4>(B) + B; A = A * dpp0<C | 4>(A);
+  return A * dpp0<C | 8>(B) + B;
+}
+
 // smallest power of two >= n, at most 64
 __device__ __forceinline__ int seg_width(int n) {
   return n <= 1 ? 1 : n >= 64 ? 64 : 1 << (32 - __builtin_clz(n - 1));

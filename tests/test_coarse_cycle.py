@@ -1,6 +1,7 @@
 """The fused coarse cycle at the edges of what one workgroup takes: sides at
 and around powers of two (a line occupies a power-of-two segment of a wave's
-lanes) and around the largest side, strips, single rows and columns."""
+lanes) and around the largest side, around the size of the dense last level,
+strips, single rows and columns."""
 import pytest
 
 import oracle as orc
@@ -9,7 +10,7 @@ import sayram_gpu as sg
 from conftest import rel_l2
 
 SHAPES = [(64, 64), (64, 63), (63, 64), (65, 64), (64, 65), (33, 31), (32, 32), (31, 33), (17, 60),
-          (60, 17), (16, 64), (64, 16), (8, 9), (3, 64), (64, 3), (2, 2), (2, 64), (1, 64), (64, 1),
+          (60, 17), (5, 13), (13, 5), (4, 16), (7, 9), (16, 64), (64, 16), (8, 9), (3, 64), (64, 3), (2, 2), (2, 64), (1, 64), (64, 1),
           (1, 65), (70, 2), (128, 130)]
 
 
