@@ -45,12 +45,12 @@ namespace sg {
 // pivot column comes from a lane of the wave itself: one barrier per pivot.
 // ---------------------------------------------------------------------------
 template <typename T>
-__global__ void __launch_bounds__(1024) k_dense_inverse(const InstDev *__restrict__ insts,
+__global__ void __launch_bounds__(1024) k_dense_inverse(const Insts insts,
                                                         const FuseMap *__restrict__ map) {
   constexpr int R = kDense / 16;
   __shared__ double s_row[2][kDense];
   const InstDev &I = insts[map[blockIdx.x].inst];
-  if (rsc(I)->ostatus == ST_IDLE) return;
+  if (ostatus_of(insts, map[blockIdx.x].inst) == ST_IDLE) return;
   const Lev &L = I.lev[I.nlev - 1];
   const int nx = L.nx, ny = L.ny, n = nx * ny, hx = half_x(nx);
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -105,11 +105,11 @@ __global__ void __launch_bounds__(1024) k_dense_inverse(const InstDev *__restric
 // and kind (PackKind) of an instance; a thread fills its lane's values.
 // ---------------------------------------------------------------------------
 template <typename T>
-__global__ void __launch_bounds__(kFuseThreads) k_coarse_pack(const InstDev *__restrict__ insts,
+__global__ void __launch_bounds__(kFuseThreads) k_coarse_pack(const Insts insts,
                                                               const PackMap *__restrict__ map) {
   const PackMap pm = map[blockIdx.x];
   const InstDev &I = insts[pm.inst];
-  if (rsc(I)->ostatus == ST_IDLE) return;
+  if (ostatus_of(insts, pm.inst) == ST_IDLE) return;
   const Lev &L = I.lev[pm.lev];
   const int nx = L.nx, ny = L.ny, hx = half_x(nx), kind = pm.kind;
   const LineLanes g = pack_lanes(nx, ny, kind);
@@ -214,7 +214,7 @@ __device__ __forceinline__ CoarseTask load_task(const CoarseTask *p, int it) {
 }
 
 template <typename T, int CAP>
-__global__ void __launch_bounds__(kFuseThreads) k_coarse_cycle(const InstDev *__restrict__ insts,
+__global__ void __launch_bounds__(kFuseThreads) k_coarse_cycle(const Insts insts,
                                                                const FuseMap *__restrict__ map,
                                                                int xid, int bid) {
   static_assert(fused_lanes_fit(), "every line of a colour has its lanes");
@@ -224,22 +224,25 @@ __global__ void __launch_bounds__(kFuseThreads) k_coarse_cycle(const InstDev *__
   __shared__ T sp[NW * kDense];
   const FuseMap fm = map[blockIdx.x];
   const InstDev &I = insts[fm.inst];
-  if (rsc(I)->status != ST_ACTIVE) return;
-  const CoarseTask *const tasks = I.tasks;
-  const T *const pack = cptr<T>(I.pack);
+  const CoarseTask *tasks = I.tasks;
+  const T *pack = cptr<T>(I.pack);
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int lf = fm.lev, last = I.nlev - 1;
+  const int lf = fm.lev, last = fm.last;
   T *xg; const T *bg;
   level_xb<T>(I, lf, xid, bid, xg, bg);
-  const int fx = I.lev[lf].nx, fy = I.lev[lf].ny, px = fused_pitch(fx), hxf = half_x(fx);
+  int fx = I.lev[lf].nx, fy = I.lev[lf].ny, dx = I.lev[last].nx, dy = I.lev[last].ny;
+  const T *dinv = cptr<T>(I.lev[last].dinv);
+  int st = status_of(insts, fm.inst);
+  pin(tasks, pack, xg, bg, fx, fy, dx, dy, dinv, st);
+  if (st != ST_ACTIVE) return;
+  const int px = fused_pitch(fx), hxf = half_x(fx), dn = dx * dy;
   // this wave's columns of the last level's inverse, rows on the lanes
-  const int dx = I.lev[last].nx, dn = dx * I.lev[last].ny;
   T dv[DC];
 #pragma unroll
   for (int c = 0; c < DC; ++c) {
     const int col = wave * DC + c;
-    dv[c] = col < dn && lane < dn ? ld32(cptr<T>(I.lev[last].dinv), (uint32_t)(col * dn + lane)) : T(0);
+    dv[c] = col < dn && lane < dn ? ld32(dinv, (uint32_t)(col * dn + lane)) : T(0);
   }
   for (int k = tid; k < XN; k += kFuseThreads) { sx[k] = T(0); sb[kDense + k] = T(0); }
   lds_barrier();
@@ -451,27 +454,27 @@ __global__ void __launch_bounds__(kFuseThreads) k_coarse_cycle(const InstDev *__
   }
 }
 
-void launch_dense_inverse(hipStream_t s, const InstDev *d, const FuseMap *m, int n, bool h32) {
+void launch_dense_inverse(hipStream_t s, const Insts &d, const FuseMap *m, int n, bool h32) {
   if (!n) return;
   if (h32) k_dense_inverse<float><<<n, 1024, 0, s>>>(d, m);
   else k_dense_inverse<double><<<n, 1024, 0, s>>>(d, m);
 }
-void launch_coarse_pack(hipStream_t s, const InstDev *d, const PackMap *m, int n, bool h32) {
+void launch_coarse_pack(hipStream_t s, const Insts &d, const PackMap *m, int n, bool h32) {
   if (!n) return;
   if (h32) k_coarse_pack<float><<<n, kFuseThreads, 0, s>>>(d, m);
   else k_coarse_pack<double><<<n, kFuseThreads, 0, s>>>(d, m);
 }
 
 template <typename T>
-void launch_coarse_cycle(hipStream_t s, const InstDev *d, const FuseMap *m, int n, int xid, int bid,
+void launch_coarse_cycle(hipStream_t s, const Insts &d, const FuseMap *m, int n, int xid, int bid,
                          int cap) {
   if (!n) return;
   if (cap <= 1024) k_coarse_cycle<T, 1024><<<n, kFuseThreads, 0, s>>>(d, m, xid, bid);
   else k_coarse_cycle<T, kFuseCells32><<<n, kFuseThreads, 0, s>>>(d, m, xid, bid);
 }
-template void launch_coarse_cycle<double>(hipStream_t, const InstDev *, const FuseMap *, int, int,
+template void launch_coarse_cycle<double>(hipStream_t, const Insts &, const FuseMap *, int, int,
                                           int, int);
-template void launch_coarse_cycle<float>(hipStream_t, const InstDev *, const FuseMap *, int, int,
+template void launch_coarse_cycle<float>(hipStream_t, const Insts &, const FuseMap *, int, int,
                                          int, int);
 
 }  // namespace sg

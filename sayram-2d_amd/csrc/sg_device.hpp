@@ -58,6 +58,25 @@ template <typename T> __device__ __forceinline__ const T *cptr(const void *p) {
 typedef const __attribute__((address_space(4))) KScal ConstKScal;
 __device__ __forceinline__ ConstKScal *rsc(const InstDev &I) { return (ConstKScal *)I.sc; }
 
+__device__ __forceinline__ int status_of(const Insts &insts, int k) {
+  return ((const __attribute__((address_space(4))) InstStat *)insts.st)[k].status;
+}
+__device__ __forceinline__ int ostatus_of(const Insts &insts, int k) {
+  return ((const __attribute__((address_space(4))) InstStat *)insts.st)[k].ostatus;
+}
+
+__device__ __forceinline__ int phase_of(const Insts &insts, int k) {
+  return ((const __attribute__((address_space(4))) InstStat *)insts.st)[k].phase;
+}
+
+// Forces uniform values (pointers and sizes read from the instance table) to be
+// in registers here. A dependent load costs about 0.8 us (the caches are cold
+// when a kernel starts), and the compiler sinks the table's reads below a
+// status test, one more round trip; pinned before the test, they are issued
+// with the status read.
+template <typename P> __device__ __forceinline__ void pin1(P &p) { asm volatile("" : "+s"(p)); }
+template <typename... P> __device__ __forceinline__ void pin(P &...p) { (pin1(p), ...); }
+
 // level-0 vector by id: a Krylov slot (Vec) or an FP32 V-cycle vector (PcVec)
 __device__ __forceinline__ void *vec(const InstDev &I, int id) {
   return id < kNumVec ? I.kv[id] : (void *)I.pv[id - kNumVec];

@@ -326,6 +326,7 @@ struct Batch {
   std::vector<Slot> slots;
   int capacity = 0;
   InstDev *d_insts = nullptr;   // compact table
+  InstStat *d_stat = nullptr;   // by compact index
   KScal *d_scal = nullptr;      // by slot
   unsigned *d_ticket = nullptr; // 2 per slot
   int *d_part = nullptr;        // by compact index
@@ -374,6 +375,7 @@ struct Batch {
   int remove(int slot);
   int rebuild();
   int fuse_level(const InstDev &I) const;
+  Insts insts() const { return {d_insts, d_stat}; }
   // largest fused level: the default takes any with sides of at most kFuseSide
   int fuse_cap() const { return opts.fuse_cells == kFuseCells ? kFuseCells32 : opts.fuse_cells; }
   int step(int nsteps, const int64_t *targets, int ntargets);
@@ -407,7 +409,7 @@ Batch::~Batch() {
   if (stream) (void)hipStreamSynchronize(stream);
   for (auto &s : slots)
     if (s.slab) (void)hipFree(s.slab);
-  (void)hipFree(d_insts); (void)hipFree(d_scal); (void)hipFree(d_ticket); (void)hipFree(d_part); (void)hipFree(d_cnt);
+  (void)hipFree(d_insts); (void)hipFree(d_stat); (void)hipFree(d_scal); (void)hipFree(d_ticket); (void)hipFree(d_part); (void)hipFree(d_cnt);
   (void)hipFree(d_maps); (void)hipFree(d_scratch);
   if (h_cnt) (void)hipHostFree(h_cnt);
   if (h_pipe) (void)hipHostFree(h_pipe);
@@ -491,6 +493,8 @@ int Batch::ensure_capacity(int cap) {
   unsigned *nt = nullptr;
   InstDev *ni = nullptr;
   int *np = nullptr;
+  InstStat *nst = nullptr;
+  HIPCHK(hipMalloc(&nst, sizeof(InstStat) * nc));
   HIPCHK(hipMalloc(&ns, sizeof(KScal) * nc));
   HIPCHK(hipMalloc(&nt, sizeof(unsigned) * 2 * nc));
   HIPCHK(hipMalloc(&ni, sizeof(InstDev) * nc));
@@ -507,8 +511,9 @@ int Batch::ensure_capacity(int cap) {
   std::memset(nh, 0, sizeof(KScal) * nc);
   HIPCHK(hipStreamSynchronize(stream));
   (void)hipFree(d_scal); (void)hipFree(d_ticket); (void)hipFree(d_insts); (void)hipFree(d_part);
+  (void)hipFree(d_stat);
   if (h_scal) (void)hipHostFree(h_scal);
-  d_scal = ns; d_ticket = nt; d_insts = ni; d_part = np; h_scal = nh;
+  d_scal = ns; d_ticket = nt; d_insts = ni; d_part = np; h_scal = nh; d_stat = nst;
   capacity = nc;
   for (size_t k = 0; k < slots.size(); ++k) {
     slots[k].dev.sc = d_scal + k;
@@ -823,9 +828,9 @@ int Batch::rebuild() {
     maxlev = std::max(maxlev, I.nlev);
     const int lf = fuse_level(I);
     slots[k].fuse_lev = lf;
-    if (lf < I.nlev) M.fmap.push_back({c, lf});
+    if (lf < I.nlev) M.fmap.push_back({c, lf, I.nlev - 1, 0});
     const bool dense = dense_last(I);
-    if (dense) M.dmap.push_back({c, I.nlev - 1});
+    if (dense) M.dmap.push_back({c, I.nlev - 1, I.nlev - 1, 0});
     for (int l = lf, off = 0; l + 1 < I.nlev; ++l) {
       for (int kind = 0; kind < kNumPack; ++kind)
         M.kmap.push_back({c, l, kind, off + pack_offset(I.lev[l].nx, I.lev[l].ny, kind)});
@@ -1095,9 +1100,9 @@ template <typename T> void Batch::vcycle(int l, int xid, int bid) {
   bool zero = true;
   // the groups of sweep shape sh in one launch
   auto lines = [&](hipStream_t s, const LineGrp *g, int ng, int dir, int sh, bool z) {
-    if (sh < kNumTileShapes) launch_line<T>(s, d_insts, g, ng, l, dir, sh, z, xid, bid);
-    else if (dir == 1) launch_cols<T>(s, d_insts, g, ng, l, sh == kColLongShape, z, xid, bid);
-    else launch_rows<T>(s, d_insts, g, ng, l, sh == kRowLongShape, z, xid, bid);
+    if (sh < kNumTileShapes) launch_line<T>(s, insts(), g, ng, l, dir, sh, z, xid, bid);
+    else if (dir == 1) launch_cols<T>(s, insts(), g, ng, l, sh == kColLongShape, z, xid, bid);
+    else launch_rows<T>(s, insts(), g, ng, l, sh == kRowLongShape, z, xid, bid);
   };
   auto sweep = [&](int dir) {
     for (int p = 0; p < 2; ++p) {
@@ -1114,13 +1119,13 @@ template <typename T> void Batch::vcycle(int l, int xid, int bid) {
           }
         if (m.nsw[l][dir][p][3]) {
           tbegin(lid);
-          launch_line<T>(stream, d_insts, m.sw[l][dir][p][3], m.nsw[l][dir][p][3], l, dir, 3,
+          launch_line<T>(stream, insts(), m.sw[l][dir][p][3], m.nsw[l][dir][p][3], l, dir, 3,
                          zero, xid, bid);
           tend(lid);
         }
         if (m.nswm[l][dir][p]) {
           tbegin(lid);
-          launch_line_shapes<T>(stream, d_insts, m.swm[l][dir][p], m.swm_na[l][dir][p],
+          launch_line_shapes<T>(stream, insts(), m.swm[l][dir][p], m.swm_na[l][dir][p],
                                 m.swm_nb[l][dir][p], m.nswm[l][dir][p], l, dir, zero, xid, bid);
           tend(lid);
         }
@@ -1142,7 +1147,7 @@ template <typename T> void Batch::vcycle(int l, int xid, int bid) {
   const bool deeper = l + 1 < m.maxlev && m.nrmap[l + 1] > 0;
   if (!deeper && m.nfmap) {
     tbegin(11);
-    launch_coarse_cycle<T>(stream, d_insts, m.fmap, m.nfmap, xid, bid,
+    launch_coarse_cycle<T>(stream, insts(), m.fmap, m.nfmap, xid, bid,
                            fuse_cap());
     tend(11);
   }
@@ -1167,16 +1172,16 @@ template <typename T> void Batch::vcycle(int l, int xid, int bid) {
     // after a pre-sweep of x-lines alone the residual vanishes on the odd
     // rows: the even rows' residual is formed inside the restriction
     if (!pre_zero && half_residual(sm)) {
-      launch_restrict_residual<T>(stream, d_insts, m.rmap[l + 1], m.nrmap[l + 1], l, xid, bid);
+      launch_restrict_residual<T>(stream, insts(), m.rmap[l + 1], m.nrmap[l + 1], l, xid, bid);
     } else {
-      if (!pre_zero) launch_residual<T>(stream, d_insts, m.pmap[l], m.npmap[l], l, xid, bid);
-      launch_restrict<T>(stream, d_insts, m.rmap[l + 1], m.nrmap[l + 1], l, pre_zero, xid, bid);
+      if (!pre_zero) launch_residual<T>(stream, insts(), m.pmap[l], m.npmap[l], l, xid, bid);
+      launch_restrict<T>(stream, insts(), m.rmap[l + 1], m.nrmap[l + 1], l, pre_zero, xid, bid);
     }
     tend(4);
     vcycle<T>(l + 1, xid, bid);
     tbegin(5);
     // only the lines the first post-smoothing sweep reads are needed
-    launch_prolong<T>(stream, d_insts, m.qmap[l], m.nqmap[l], l, pre_zero, xid, prolong_rows(sm));
+    launch_prolong<T>(stream, insts(), m.qmap[l], m.nqmap[l], l, pre_zero, xid, prolong_rows(sm));
     tend(5);
     zero = false;
     if (post_x) sweep(0);
@@ -1188,17 +1193,17 @@ template <typename KT, typename VT> void Batch::iteration(bool xstate) {
   const int nb = dm.ncmap[0], n = (int)order.size();
   const BlkMap *m0 = dm.cmap[0];
   constexpr bool pc = sizeof(KT) != sizeof(VT);
-  tbegin(8); launch_bicg<KT>(stream, 0, d_insts, m0, nb, xstate, pc); tend(8);
+  tbegin(8); launch_bicg<KT>(stream, 0, insts(), m0, nb, xstate, pc); tend(8);
   vcycle<VT>(0, pc ? PV_PH : VPH, pc ? PV_P : VP);
-  tbegin(6); launch_bicg<KT>(stream, 1, d_insts, m0, nb, xstate, pc); tend(6);
-  tbegin(12); launch_finish<KT>(stream, FIN_V, d_insts, n, d_cnt); tend(12);
-  tbegin(8); launch_bicg<KT>(stream, 2, d_insts, m0, nb, xstate, pc); tend(8);
-  tbegin(12); launch_finish<KT>(stream, FIN_S, d_insts, n, d_cnt); tend(12);
+  tbegin(6); launch_bicg<KT>(stream, 1, insts(), m0, nb, xstate, pc); tend(6);
+  tbegin(12); launch_finish<KT>(stream, FIN_V, insts(), n, d_cnt); tend(12);
+  tbegin(8); launch_bicg<KT>(stream, 2, insts(), m0, nb, xstate, pc); tend(8);
+  tbegin(12); launch_finish<KT>(stream, FIN_S, insts(), n, d_cnt); tend(12);
   vcycle<VT>(0, pc ? PV_SH : VSH, pc ? PV_B : VS);
-  tbegin(7); launch_bicg<KT>(stream, 3, d_insts, m0, nb, xstate, pc); tend(7);
-  tbegin(12); launch_finish<KT>(stream, FIN_T, d_insts, n, d_cnt); tend(12);
-  tbegin(8); launch_bicg<KT>(stream, 4, d_insts, m0, nb, xstate, pc); tend(8);
-  tbegin(12); launch_finish<KT>(stream, FIN_X, d_insts, n, d_cnt); tend(12);
+  tbegin(7); launch_bicg<KT>(stream, 3, insts(), m0, nb, xstate, pc); tend(7);
+  tbegin(12); launch_finish<KT>(stream, FIN_T, insts(), n, d_cnt); tend(12);
+  tbegin(8); launch_bicg<KT>(stream, 4, insts(), m0, nb, xstate, pc); tend(8);
+  tbegin(12); launch_finish<KT>(stream, FIN_X, insts(), n, d_cnt); tend(12);
 }
 
 template <typename F> int Batch::run_graph(int key, F &&enqueue) {
@@ -1235,19 +1240,19 @@ void Batch::setup_kernels(bool start64) {
   const bool mixed = opts.precision == SG_MIXED;
   const bool h32 = opts.precision != SG_FP64;   // FP32 hierarchy and V-cycle
   const double tol2 = mixed ? opts.inner_rtol * opts.inner_rtol : opts.rtol * opts.rtol;
-  launch_begin(stream, d_insts, n, d_part, d_cnt, d_cnt + 1, tol2, opts.rtol * opts.rtol,
+  launch_begin(stream, insts(), n, d_part, d_cnt, d_cnt + 1, tol2, opts.rtol * opts.rtol,
                mixed ? opts.max_inner : opts.max_iters, opts.max_iters);
-  tbegin(0); launch_assemble(stream, d_insts, dm.cmap[0], nb0); tend(0);
+  tbegin(0); launch_assemble(stream, insts(), dm.cmap[0], nb0); tend(0);
   // LU factors of the line matrices of level l: smoothing lines of both
   // colours (one launch per direction and tile shape) and the exact solve of
   // a last level that is a line
   auto factors = [&](int l, hipStream_t s) {
     for (int d = 0; d < 2; ++d)
       for (int sh = 0; sh < kNumTileShapes; ++sh)
-        launch_line_factor(s, d_insts, dm.gfac[l][d][sh], dm.ngfac[l][d][sh], l, d, sh, h32);
+        launch_line_factor(s, insts(), dm.gfac[l][d][sh], dm.ngfac[l][d][sh], l, d, sh, h32);
     for (int sh = 0; sh < kNumTileShapes; ++sh) {
-      launch_line_factor(s, d_insts, dm.gcx[l][sh], dm.ngcx[l][sh], l, 0, sh, h32);
-      launch_line_factor(s, d_insts, dm.gcy[l][sh], dm.ngcy[l][sh], l, 1, sh, h32);
+      launch_line_factor(s, insts(), dm.gcx[l][sh], dm.ngcx[l][sh], l, 0, sh, h32);
+      launch_line_factor(s, insts(), dm.gcy[l][sh], dm.ngcy[l][sh], l, 1, sh, h32);
     }
   };
   auto note = [&](hipError_t e) { if (e != hipSuccess && fan_err == hipSuccess) fan_err = e; };
@@ -1259,35 +1264,35 @@ void Batch::setup_kernels(bool start64) {
     // main stream waits for them before the solve. Same kernels, same inputs.
     note(hipEventRecord(ev_lev[0], stream));
     for (int l = 0; l + 1 < dm.maxlev; ++l) {
-      launch_pweights(stream, d_insts, dm.pmap[l], dm.npmap[l], l, h32);
-      launch_rap(stream, d_insts, dm.cmap[l + 1], dm.ncmap[l + 1], l, h32);
+      launch_pweights(stream, insts(), dm.pmap[l], dm.npmap[l], l, h32);
+      launch_rap(stream, insts(), dm.cmap[l + 1], dm.ncmap[l + 1], l, h32);
       note(hipEventRecord(ev_lev[l + 1], stream));
     }
     for (int l = 0; l < dm.maxlev; ++l) {
       note(hipStreamWaitEvent(side, ev_lev[l], 0));
       factors(l, side);
     }
-    launch_dense_inverse(stream, d_insts, dm.dmap, dm.ndmap, h32);
+    launch_dense_inverse(stream, insts(), dm.dmap, dm.ndmap, h32);
     note(hipEventRecord(ev_join, side));
     note(hipStreamWaitEvent(stream, ev_join, 0));
-    launch_coarse_pack(stream, d_insts, dm.kmap, dm.nkmap, h32);
+    launch_coarse_pack(stream, insts(), dm.kmap, dm.nkmap, h32);
   } else {
     for (int l = 0; l < dm.maxlev; ++l) {
       tbegin(1);
       factors(l, stream);
       if (l + 1 < dm.maxlev) {
-        launch_pweights(stream, d_insts, dm.pmap[l], dm.npmap[l], l, h32);
-        launch_rap(stream, d_insts, dm.cmap[l + 1], dm.ncmap[l + 1], l, h32);
+        launch_pweights(stream, insts(), dm.pmap[l], dm.npmap[l], l, h32);
+        launch_rap(stream, insts(), dm.cmap[l + 1], dm.ncmap[l + 1], l, h32);
       }
       tend(1);
     }
     tbegin(1);
-    launch_dense_inverse(stream, d_insts, dm.dmap, dm.ndmap, h32);
-    launch_coarse_pack(stream, d_insts, dm.kmap, dm.nkmap, h32);
+    launch_dense_inverse(stream, insts(), dm.dmap, dm.ndmap, h32);
+    launch_coarse_pack(stream, insts(), dm.kmap, dm.nkmap, h32);
     tend(1);
   }
   if (start64) {
-    tbegin(12); launch_finish<double>(stream, FIN_INIT64, d_insts, n, d_cnt); tend(12);
+    tbegin(12); launch_finish<double>(stream, FIN_INIT64, insts(), n, d_cnt); tend(12);
   }
 }
 
@@ -1297,11 +1302,11 @@ void Batch::setup_kernels(bool start64) {
 // passes may follow every chunk of iterations.
 void Batch::end_pass() {
   const int n = (int)order.size(), nb0 = dm.ncmap[0];
-  tbegin(10); launch_finalize(stream, d_insts, dm.cmap[0], nb0); tend(10);
-  tbegin(12); launch_finish<double>(stream, FIN_FINALIZE, d_insts, n, d_cnt); tend(12);
-  tbegin(10); launch_commit(stream, d_insts, dm.cmap[0], nb0); tend(10);
+  tbegin(10); launch_finalize(stream, insts(), dm.cmap[0], nb0); tend(10);
+  tbegin(12); launch_finish<double>(stream, FIN_FINALIZE, insts(), n, d_cnt); tend(12);
+  tbegin(10); launch_commit(stream, insts(), dm.cmap[0], nb0); tend(10);
   if (opts.warm_start > 0) {
-    tbegin(12); launch_finish<double>(stream, FIN_EXTRAP, d_insts, n, d_cnt); tend(12);
+    tbegin(12); launch_finish<double>(stream, FIN_EXTRAP, insts(), n, d_cnt); tend(12);
   }
 }
 
@@ -1486,16 +1491,16 @@ int Batch::step_once() {
     if ((rc = run_graph(graph_key(1, 0), [&] { setup_kernels(false); }))) return rc;
     const int nb0 = dm.ncmap[0];
     for (int ref = 0; ref <= opts.max_iters; ++ref) {
-      tbegin(9); launch_ir_residual(stream, d_insts, dm.cmap[0], nb0); tend(9);
-      tbegin(12); launch_finish<double>(stream, FIN_IR_RES, d_insts, n, d_cnt + 1); tend(12);
+      tbegin(9); launch_ir_residual(stream, insts(), dm.cmap[0], nb0); tend(9);
+      tbegin(12); launch_finish<double>(stream, FIN_IR_RES, insts(), n, d_cnt + 1); tend(12);
       int oactive = 0;
       if ((rc = read_counter(1, &oactive))) return rc;
       if (!oactive) break;
-      launch_ir_inner_init(stream, d_insts, dm.cmap[0], nb0);
-      tbegin(12); launch_finish<float>(stream, FIN_INNER_INIT, d_insts, n, d_cnt); tend(12);
+      launch_ir_inner_init(stream, insts(), dm.cmap[0], nb0);
+      tbegin(12); launch_finish<float>(stream, FIN_INNER_INIT, insts(), n, d_cnt); tend(12);
       launch_copy_counter(stream, d_cnt + 1, d_cnt);
       if ((rc = krylov<float, float>(opts.max_inner, false, 0, false))) return rc;
-      launch_ir_update(stream, d_insts, dm.cmap[0], nb0);
+      launch_ir_update(stream, insts(), dm.cmap[0], nb0);
     }
     end_pass();
   }
@@ -1610,8 +1615,8 @@ int Batch::debug_assemble(int slot, double *bands, double *R) {
   for (int c = 0; c < n; ++c) part[c] = order[c] == slot;
   HIPCHK(hipMemcpyAsync(d_part, part.data(), n * sizeof(int), hipMemcpyHostToDevice, stream));
   part_host = part;
-  launch_begin(stream, d_insts, n, d_part, d_cnt, d_cnt + 1, 0, 0, 1, 1);
-  launch_assemble(stream, d_insts, dm.cmap[0], dm.ncmap[0]);
+  launch_begin(stream, insts(), n, d_part, d_cnt, d_cnt + 1, 0, 0, 1, 1);
+  launch_assemble(stream, insts(), dm.cmap[0], dm.ncmap[0]);
   HIPCHK(hipGetLastError());
   const Slot &s = slots[slot];
   const size_t N = (size_t)s.nx * s.ny;

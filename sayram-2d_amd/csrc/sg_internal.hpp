@@ -257,8 +257,18 @@ struct InstDev {
 
 struct BlkMap { int inst; int k0; };      // cell-parallel: 256 cells of one instance
 struct LineGrp { int inst; int first; int count; int step; };   // lines first + k*step, k < count
+// The instance table a kernel gets, with the statuses of the instances beside
+// it (KScal::status and ostatus by compact index, mirrored by the kernels that
+// change them): a workgroup reads its status and its instance's pointers in
+// the same round trip instead of following the table to the scalars first.
+struct InstStat { int status, ostatus, phase, pad; };
+struct Insts {
+  const InstDev *t;
+  InstStat *st;
+  __device__ __forceinline__ const InstDev &operator[](int k) const { return t[k]; }
+};
 struct PackMap { int inst, lev, kind, off; };   // off: of the kind's arrays in InstDev::pack
-struct FuseMap { int inst; int lev; };    // an instance whose levels from lev down run fused
+struct FuseMap { int inst, lev, last, pad; };   // an instance whose levels lev .. last run fused
 
 // The coarse end of a V-cycle runs in one workgroup per instance from the
 // first level with at most fuse_cells cells and no side above kFuseSide (a

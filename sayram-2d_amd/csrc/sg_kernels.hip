@@ -76,7 +76,7 @@ __device__ __forceinline__ void store_partials(const InstDev &I, int lblk, A (&v
 // step start: statuses, tolerances and the active counters (a kernel rather
 // than a memset, so the sequence can be captured into a graph)
 // ---------------------------------------------------------------------------
-__global__ void k_begin(const InstDev *__restrict__ insts, int n, const int *__restrict__ part,
+__global__ void k_begin(const Insts insts, int n, const int *__restrict__ part,
                         int *__restrict__ active, int *__restrict__ oactive, double tol2,
                         double otol2, int maxit, int omaxit) {
   __shared__ int cnt;
@@ -92,6 +92,7 @@ __global__ void k_begin(const InstDev *__restrict__ insts, int n, const int *__r
     s.tol2 = tol2; s.otol2 = otol2; s.maxit = maxit; s.omaxit = omaxit;
     s.iters = 0; s.titers = 0; s.orefs = 0; s.clamps = 0; s.vcyc = 0;
     s.phase = 0; s.nonfin = 0;
+    insts.st[k] = {s.status, s.ostatus, 0, 0};
     mine += p;
   }
   atomicAdd(&cnt, mine);
@@ -242,12 +243,12 @@ __device__ __forceinline__ double start_residual(double R, double ac, double x0,
 // used), so that a work-item waits for memory once rather than behind each
 // boundary test; only the Dirichlet vertex arrays, read by boundary cells, are
 // loaded where they are used.
-__global__ void __launch_bounds__(kBlock) k_assemble(const InstDev *__restrict__ insts,
+__global__ void __launch_bounds__(kBlock) k_assemble(const Insts insts,
                                                     const BlkMap *__restrict__ map) {
 #pragma clang fp contract(off)
   const BlkMap m = map[blockIdx.x];
   const InstDev &I = insts[m.inst];
-  if (rsc(I)->ostatus == ST_IDLE) return;
+  if (ostatus_of(insts, m.inst) == ST_IDLE) return;
   const int nx = I.nx, ny = I.ny;
   const int K = m.k0 + threadIdx.x;
   const bool krylov64 = I.prec != SG_MIXED;   // uniform over the workgroup
@@ -426,11 +427,11 @@ __device__ __forceinline__ void w_yedge(const Lev &L, size_t K, int j, double &w
 }
 
 template <typename T, int NB>
-__global__ void __launch_bounds__(kBlock) k_pweights(const InstDev *__restrict__ insts,
+__global__ void __launch_bounds__(kBlock) k_pweights(const Insts insts,
                                                     const BlkMap *__restrict__ map, int l) {
   const BlkMap m = map[blockIdx.x];
   const InstDev &I = insts[m.inst];
-  if (rsc(I)->ostatus == ST_IDLE) return;
+  if (ostatus_of(insts, m.inst) == ST_IDLE) return;
   const Lev &L = I.lev[l];
   const int nx = L.nx, ny = L.ny;
   const int K = m.k0 + threadIdx.x;
@@ -468,8 +469,8 @@ __global__ void __launch_bounds__(kBlock) k_pweights(const InstDev *__restrict__
   // Only the weights that are neither structurally zero nor exactly one are
   // stored: an even-even point's single weight is 1 and its others are 0, and
   // the parent at I0 + 1 of an even i (at J0 + 1 of an even j) has weight 0.
-  // Every reader takes those values as constants (rap_row, restrict_point,
-  // prolong_point, k_prolong), so the unstored entries are never read.
+  // Every reader takes those values as constants (rap_row, k_restrict,
+  // k_prolong, the fused cycle), so the unstored entries are never used.
   if (io || jo) ptr<T>(L.pw[0])[K] = (T)w0;
   if (io) ptr<T>(L.pw[1])[K] = (T)w1;
   if (jo) ptr<T>(L.pw[2])[K] = (T)w2;
@@ -528,11 +529,11 @@ __device__ __forceinline__ void rap_row(const Lev &F, const T *const (&pw)[4], i
 }
 
 template <typename T, int NB, bool COPY>
-__global__ void __launch_bounds__(kBlock) k_rap(const InstDev *__restrict__ insts,
+__global__ void __launch_bounds__(kBlock) k_rap(const Insts insts,
                                                const BlkMap *__restrict__ map, int l) {
   const BlkMap m = map[blockIdx.x];
   const InstDev &I = insts[m.inst];
-  if (rsc(I)->ostatus == ST_IDLE) return;
+  if (ostatus_of(insts, m.inst) == ST_IDLE) return;
   const Lev &F = I.lev[l];
   const Lev &Cl = I.lev[l + 1];
   const int cx = Cl.nx, cy = Cl.ny, fx = F.nx;
@@ -573,7 +574,7 @@ __global__ void __launch_bounds__(kBlock) k_rap(const InstDev *__restrict__ inst
 // them across the line and carry (P, Q) between tiles; each thread then runs
 // the exact recurrence over its 4 steps from the value the scan gives it.
 template <typename T, int DIR, int SH>
-__global__ void __launch_bounds__(tile_threads(SH)) k_line_factor(const InstDev *__restrict__ insts,
+__global__ void __launch_bounds__(tile_threads(SH)) k_line_factor(const Insts insts,
                                                                   const LineGrp *__restrict__ map,
                                                                   int l) {
   constexpr int S = tile_steps(SH), L = tile_lines(SH), NT = tile_threads(SH);
@@ -586,7 +587,7 @@ __global__ void __launch_bounds__(tile_threads(SH)) k_line_factor(const InstDev 
   __shared__ double s_c[L];
   const LineGrp gr = map[blockIdx.x];
   const InstDev &I = insts[gr.inst];
-  if (rsc(I)->ostatus == ST_IDLE) return;
+  if (ostatus_of(insts, gr.inst) == ST_IDLE) return;
   const Lev &Lv = I.lev[l];
   const int nx = Lv.nx, ny = Lv.ny;
   const double *__restrict__ bc = Lv.band64[BC];
@@ -735,7 +736,7 @@ template <typename T, int NB, int SH> constexpr int line_lds_elems() {
 // threads, in the LDS lds (line_lds_elems<T, NB, SH>() values); k_line and
 // k_line_shapes below are its kernels.
 template <typename T, int NB, int DIR, bool ZERO, int SH>
-__device__ __forceinline__ void line_sweep(const InstDev *__restrict__ insts, const LineGrp gr,
+__device__ __forceinline__ void line_sweep(const Insts insts, const LineGrp gr,
                                            int l, int xid, int bid, T *lds) {
   constexpr int S = tile_steps(SH), L = tile_lines(SH), NT = tile_threads(SH);
   constexpr int W = NT / L;          // threads per line in the solve, 4 steps each
@@ -748,7 +749,7 @@ __device__ __forceinline__ void line_sweep(const InstDev *__restrict__ insts, co
   T *const s_i = s_a + TB;
   T *const s_c = s_i + TB;         // L values
   const InstDev &I = insts[gr.inst];
-  if (rsc(I)->status != ST_ACTIVE) return;
+  if (status_of(insts, gr.inst) != ST_ACTIVE) return;
   const Lev &Lv = I.lev[l];
   const int nx = Lv.nx, ny = Lv.ny;
   T *x; const T *b;
@@ -956,7 +957,7 @@ __device__ __forceinline__ void line_sweep(const InstDev *__restrict__ insts, co
 }
 
 template <typename T, int NB, int DIR, bool ZERO, int SH>
-__global__ void __launch_bounds__(tile_threads(SH)) k_line(const InstDev *__restrict__ insts,
+__global__ void __launch_bounds__(tile_threads(SH)) k_line(const Insts insts,
                                                            const LineGrp *__restrict__ map, int l,
                                                            int xid, int bid) {
   __shared__ T lds[line_lds_elems<T, NB, SH>()];
@@ -973,7 +974,7 @@ __global__ void __launch_bounds__(tile_threads(SH)) k_line(const InstDev *__rest
 // bodies take 140 and it runs 3, as the shapes alone do not).
 template <typename T, int NB, int DIR, bool ZERO, int SA, int SB, int SC>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(DIR == 0 && sizeof(T) == 4 ? 4 : 1)))
-k_line_shapes(const InstDev *__restrict__ insts,
+k_line_shapes(const Insts insts,
                                                      const LineGrp *__restrict__ map, int na,
                                                      int nb, int l, int xid, int bid) {
   static_assert(tile_threads(SA) == 256 && tile_threads(SB) == 256 &&
@@ -991,6 +992,22 @@ k_line_shapes(const InstDev *__restrict__ insts,
   else line_sweep<T, NB, DIR, ZERO, SC_>(insts, gr, l, xid, bid, lds);
 }
 
+// The operator of a level: its bands and size (hold: pinned, sg_device.hpp).
+template <typename T, int NB> struct Sten {
+  const T *b[NB];
+  int nx, ny;
+  __device__ __forceinline__ Sten(const Lev &L) {
+#pragma unroll
+    for (int k = 0; k < NB; ++k) b[k] = cptr<T>(L.band[k]);
+    nx = L.nx; ny = L.ny;
+  }
+  __device__ __forceinline__ void hold() {
+#pragma unroll
+    for (int k = 0; k < NB; ++k) pin(b[k]);
+    pin(nx, ny);
+  }
+};
+
 // (A x)(i, j) at slot K. Every operand is loaded before the sum, so that a
 // work-item waits for memory once (with the loads behind the boundary tests
 // the compiler issues one round trip per neighbour): neighbour slots are
@@ -999,18 +1016,18 @@ k_line_shapes(const InstDev *__restrict__ insts,
 // centre, west, east, south (south-west, south-east), north (north-west,
 // north-east).
 template <typename T, int NB>
-__device__ __forceinline__ T stencil_apply(const Lev &L, size_t K, int i, int j, const T *xp) {
+__device__ __forceinline__ T stencil_apply(const Sten<T, NB> &L, size_t K, int i, int j, const T *xp) {
   const int nx = L.nx, ny = L.ny, hx = half_x(nx);
   const bool hw = i > 0, he = i < nx - 1, hs = j > 0, hn = j < ny - 1;
   const size_t row = (size_t)j * nx;
   const size_t kw = row + xslot(hw ? i - 1 : i, hx), ke = row + xslot(he ? i + 1 : i, hx);
   const size_t ds = hs ? nx : 0, dn = hn ? nx : 0;
   const auto x = gbl(xp);
-  auto band = [&](int b) { return gbl(cptr<T>(L.band[b]))[K]; };
+  auto band = [&](int b) { return gbl(L.b[b])[K]; };
   const T ac = band(BC), aw = band(BW), ae = band(BE), as = band(BS), an = band(BN);
   const T x0 = x[K], xw = x[kw], xe = x[ke], xs = x[K - ds], xn = x[K + dn];
   T asw = T(0), ase = T(0), anw = T(0), ane = T(0), xsw = T(0), xse = T(0), xnw = T(0), xne = T(0);
-  if (NB == 9) {
+  if constexpr (NB == 9) {
     asw = band(BSW); ase = band(BSE); anw = band(BNW); ane = band(BNE);
     xsw = x[kw - ds]; xse = x[ke - ds]; xnw = x[kw + dn]; xne = x[ke + dn];
   }
@@ -1031,17 +1048,31 @@ __device__ __forceinline__ T stencil_apply(const Lev &L, size_t K, int i, int j,
   return s;
 }
 
+// The FP64 level-0 operator.
+struct Sten64 {
+  const double *b[5];
+  int nx, ny;
+  __device__ __forceinline__ Sten64(const InstDev &I) {
+#pragma unroll
+    for (int k = 0; k < 5; ++k) b[k] = I.band64[k];
+    nx = I.nx; ny = I.ny;
+  }
+  __device__ __forceinline__ void hold() {
+    pin(b[0], b[1], b[2], b[3], b[4], nx, ny);
+  }
+};
+
 // M x at slot K with the FP64 level-0 bands (x in FP64, or an FP32 vector
 // promoted on load); loads first, as in stencil_apply
 template <typename X>
-__device__ __forceinline__ double spmv64(const InstDev &I, size_t K, int i, int j, const X *xp) {
-  const int nx = I.nx, hx = half_x(nx);
-  const bool hw = i > 0, he = i < nx - 1, hs = j > 0, hn = j < I.ny - 1;
+__device__ __forceinline__ double spmv64(const Sten64 &M, size_t K, int i, int j, const X *xp) {
+  const int nx = M.nx, hx = half_x(nx);
+  const bool hw = i > 0, he = i < nx - 1, hs = j > 0, hn = j < M.ny - 1;
   const size_t row = (size_t)j * nx;
   const size_t kw = row + xslot(hw ? i - 1 : i, hx), ke = row + xslot(he ? i + 1 : i, hx);
   const auto x = gbl(xp);
-  const double ac = gbl(I.band64[BC])[K], aw = gbl(I.band64[BW])[K], ae = gbl(I.band64[BE])[K];
-  const double as = gbl(I.band64[BS])[K], an = gbl(I.band64[BN])[K];
+  const double ac = gbl(M.b[BC])[K], aw = gbl(M.b[BW])[K], ae = gbl(M.b[BE])[K];
+  const double as = gbl(M.b[BS])[K], an = gbl(M.b[BN])[K];
   const double x0 = (double)x[K], xw = (double)x[kw], xe = (double)x[ke];
   const double xs = (double)x[hs ? K - nx : K], xn = (double)x[hn ? K + nx : K];
   double s = ac * x0;
@@ -1055,22 +1086,26 @@ __device__ __forceinline__ double spmv64(const InstDev &I, size_t K, int i, int 
 // r_l = b_l - A_l x_l into the level's scratch (the line-solve buffer cp is
 // free between the pre- and post-smoothing sweeps), after a pre-smoothing
 // sweep: with x_l = 0 the restriction reads b_l itself, and after an x-line
-// pre-sweep alone restrict_residual_point forms the residual it needs.
+// pre-sweep alone k_restrict_residual forms the residual it needs.
 template <typename T, int NB>
-__global__ void __launch_bounds__(kBlock) k_residual(const InstDev *__restrict__ insts,
+__global__ void __launch_bounds__(kBlock) k_residual(const Insts insts,
                                                     const BlkMap *__restrict__ map, int l,
                                                     int xid, int bid) {
   const BlkMap m = map[blockIdx.x];
   const InstDev &I = insts[m.inst];
-  if (rsc(I)->status != ST_ACTIVE) return;
-  const Lev &F = I.lev[l];
+  Sten<T, NB> F(I.lev[l]);
+  T *x; const T *b;
+  level_xb<T>(I, l, xid, bid, x, b);
+  T *r = ptr<T>(I.lev[l].cp);
+  int st = status_of(insts, m.inst);
+  F.hold();
+  pin(x, b, r, st);
+  if (st != ST_ACTIVE) return;
   const int K = m.k0 + threadIdx.x;
   if (K >= F.nx * F.ny) return;
   int i, j;
   cell_ij(K, F.nx, half_x(F.nx), i, j);
-  T *x; const T *b;
-  level_xb<T>(I, l, xid, bid, x, b);
-  ptr<T>(F.cp)[K] = b[K] - stencil_apply<T, NB>(F, K, i, j, x);
+  gbl(r)[K] = gbl(b)[K] - stencil_apply<T, NB>(F, K, i, j, x);
 }
 
 // b_{l+1}(C) = sum_f P(f, C) r_l(f) over the 3x3 fine block around (2I, 2J).
@@ -1081,16 +1116,27 @@ __global__ void __launch_bounds__(kBlock) k_residual(const InstDev *__restrict__
 // contiguous across the wave; the coarse store alternates between the two
 // contiguous halves of the coarse row.
 template <typename T, bool FROM_B>
-__device__ __forceinline__ void restrict_point(const InstDev &I, int l, int xid, int bid, int KC) {
-  const Lev &F = I.lev[l];
-  const Lev &Cl = I.lev[l + 1];
-  const int J = KC / Cl.nx, Ic = KC - J * Cl.nx;    // column order
-  const int hxf = half_x(F.nx);
+__global__ void __launch_bounds__(kBlock) k_restrict(const Insts insts,
+                                                    const BlkMap *__restrict__ map, int l,
+                                                    int xid, int bid) {
+  const BlkMap m = map[blockIdx.x];
+  const InstDev &I = insts[m.inst];
   T *x; const T *b;
   level_xb<T>(I, l, xid, bid, x, b);
-  const auto r = gbl(FROM_B ? b : cptr<T>(F.cp));
-  const auto pw0 = gbl(cptr<T>(F.pw[0])), pw1 = gbl(cptr<T>(F.pw[1]));
-  const auto pw2 = gbl(cptr<T>(F.pw[2])), pw3 = gbl(cptr<T>(F.pw[3]));
+  const T *rp = FROM_B ? b : cptr<T>(I.lev[l].cp);
+  const T *w0 = cptr<T>(I.lev[l].pw[0]), *w1 = cptr<T>(I.lev[l].pw[1]);
+  const T *w2 = cptr<T>(I.lev[l].pw[2]), *w3 = cptr<T>(I.lev[l].pw[3]);
+  T *out = ptr<T>(I.lev[l + 1].b);
+  int fx = I.lev[l].nx, fy = I.lev[l].ny, cx = I.lev[l + 1].nx, cy = I.lev[l + 1].ny;
+  int st = status_of(insts, m.inst);
+  pin(rp, w0, w1, w2, w3, out, fx, fy, cx, cy, st);
+  if (st != ST_ACTIVE) return;
+  const int KC = m.k0 + threadIdx.x;
+  if (KC >= cx * cy) return;
+  const int J = KC / cx, Ic = KC - J * cx;    // column order
+  const int hxf = half_x(fx);
+  const auto r = gbl(rp);
+  const auto pw0 = gbl(w0), pw1 = gbl(w1), pw2 = gbl(w2), pw3 = gbl(w3);
   // All 18 loads are issued before the sum (fine points outside the grid are
   // clamped in and weighted by zero), then added in row-major order.
   T wv[3][3], rv[3][3];
@@ -1098,12 +1144,12 @@ __device__ __forceinline__ void restrict_point(const InstDev &I, int l, int xid,
 #pragma unroll
   for (int db = -1; db <= 1; ++db) {
     const int fj = 2 * J + db;
-    const bool okj = fj >= 0 && fj < F.ny;
-    const size_t rowf = (size_t)(okj ? fj : 2 * J) * F.nx;
+    const bool okj = fj >= 0 && fj < fy;
+    const size_t rowf = (size_t)(okj ? fj : 2 * J) * fx;
 #pragma unroll
     for (int da = -1; da <= 1; ++da) {
       const int fi = 2 * Ic + da;
-      const bool oki = fi >= 0 && fi < F.nx;
+      const bool oki = fi >= 0 && fi < fx;
       const size_t kf = rowf + xslot(oki ? fi : 2 * Ic, hxf);
       // slot of C among the parents of f: (I - (fi >> 1)) + 2 (J - (fj >> 1))
       const int slot = (da < 0 ? 1 : 0) + 2 * (db < 0 ? 1 : 0);
@@ -1120,69 +1166,89 @@ __device__ __forceinline__ void restrict_point(const InstDev &I, int l, int xid,
   for (int b = 0; b < 3; ++b)
 #pragma unroll
     for (int a = 0; a < 3; ++a) s = fma(ok[b][a] ? wv[b][a] : T(0), rv[b][a], s);
-  gbl(ptr<T>(Cl.b))[(size_t)J * Cl.nx + xslot(Ic, half_x(Cl.nx))] = s;
+  gbl(out)[(size_t)J * cx + xslot(Ic, half_x(cx))] = s;
 }
 
-// b_{l+1}(C) = sum_f P(f, C) r_l(f) after an x-line pre-sweep: r_l vanishes
-// on the odd rows, and the three fine points of row 2 J form theirs here,
-// r = b - A x as residual_point does (same operations), instead of reading a
-// stored residual: one launch per level and no residual array written or
-// read. The odd fine points are shared by two coarse points, so they are
-// formed twice.
+// b_{l+1}(C) = sum_f P(f, C) r_l(f) after an x-line pre-sweep from x = 0: r_l
+// vanishes on the odd rows (solved last), and the even rows satisfied their
+// equations with the odd rows at zero, so their residual is what the odd rows
+// contribute, r = -(couplings to the odd rows) x. Only the six (5-point: two)
+// off-row couplings and the odd rows' x are read: half the bands of b - A x, and
+// the three fine points of row 2 J share most of the x they read. The odd fine
+// points are shared by two coarse points, so they are formed twice.
 template <typename T, int NB>
-__device__ __forceinline__ void restrict_residual_point(const InstDev &I, int l, int xid, int bid,
-                                                        int KC) {
-  const Lev &F = I.lev[l];
-  const Lev &Cl = I.lev[l + 1];
-  const int J = KC / Cl.nx, Ic = KC - J * Cl.nx;    // column order
-  const int hxf = half_x(F.nx);
-  T *x; const T *b;
-  level_xb<T>(I, l, xid, bid, x, b);
-  const auto pw0 = gbl(cptr<T>(F.pw[0])), pw1 = gbl(cptr<T>(F.pw[1]));
-  const int fj = 2 * J;
-  const size_t rowf = (size_t)fj * F.nx;
-  T wv[3], rv[3];
-  bool ok[3];
-#pragma unroll
-  for (int da = -1; da <= 1; ++da) {
-    const int fi = 2 * Ic + da;
-    const bool oki = fi >= 0 && fi < F.nx;
-    const int ci = oki ? fi : 2 * Ic;
-    const size_t kf = rowf + xslot(ci, hxf);
-    // parent slot of C: 1 for the point to the west (da < 0), 0 otherwise;
-    // the point at C itself is injected with weight exactly 1
-    wv[da + 1] = da == 0 ? T(1) : T(da < 0 ? pw1[kf] : pw0[kf]);
-    rv[da + 1] = gbl(b)[kf] - stencil_apply<T, NB>(F, kf, ci, fj, x);
-    ok[da + 1] = oki;
-  }
-  T s = T(0);
-#pragma unroll
-  for (int a = 0; a < 3; ++a) s = fma(ok[a] ? wv[a] : T(0), rv[a], s);
-  gbl(ptr<T>(Cl.b))[(size_t)J * Cl.nx + xslot(Ic, half_x(Cl.nx))] = s;
-}
-
-template <typename T, int NB>
-__global__ void __launch_bounds__(kBlock) k_restrict_residual(const InstDev *__restrict__ insts,
+__global__ void __launch_bounds__(kBlock) k_restrict_residual(const Insts insts,
                                                              const BlkMap *__restrict__ map, int l,
                                                              int xid, int bid) {
   const BlkMap m = map[blockIdx.x];
   const InstDev &I = insts[m.inst];
-  if (rsc(I)->status != ST_ACTIVE) return;
+  const Lev &F = I.lev[l];
+  T *xp; const T *bp;
+  level_xb<T>(I, l, xid, bid, xp, bp);
+  const T *s0 = cptr<T>(F.band[BS]), *n0 = cptr<T>(F.band[BN]);
+  const T *sw = nullptr, *se = nullptr, *nw = nullptr, *ne = nullptr;
+  if constexpr (NB == 9) {
+    sw = cptr<T>(F.band[BSW]); se = cptr<T>(F.band[BSE]);
+    nw = cptr<T>(F.band[BNW]); ne = cptr<T>(F.band[BNE]);
+  }
+  const T *w0 = cptr<T>(F.pw[0]), *w1 = cptr<T>(F.pw[1]);
+  T *out = ptr<T>(I.lev[l + 1].b);
+  int fx = F.nx, fy = F.ny, cx = I.lev[l + 1].nx, cy = I.lev[l + 1].ny;
+  int st = status_of(insts, m.inst);
+  if constexpr (NB == 9) pin(sw, se, nw, ne);
+  pin(xp, s0, n0, w0, w1, out, fx, fy, cx, cy, st);
+  if (st != ST_ACTIVE) return;
   const int KC = m.k0 + threadIdx.x;
-  if (KC >= I.lev[l + 1].nx * I.lev[l + 1].ny) return;
-  restrict_residual_point<T, NB>(I, l, xid, bid, KC);
-}
-
-template <typename T, bool FROM_B>
-__global__ void __launch_bounds__(kBlock) k_restrict(const InstDev *__restrict__ insts,
-                                                    const BlkMap *__restrict__ map, int l,
-                                                    int xid, int bid) {
-  const BlkMap m = map[blockIdx.x];
-  const InstDev &I = insts[m.inst];
-  if (rsc(I)->status != ST_ACTIVE) return;
-  const int KC = m.k0 + threadIdx.x;
-  if (KC >= I.lev[l + 1].nx * I.lev[l + 1].ny) return;
-  restrict_point<T, FROM_B>(I, l, xid, bid, KC);
+  if (KC >= cx * cy) return;
+  const int J = KC / cx, Ic = KC - J * cx;    // column order
+  const int hxf = half_x(fx), fj = 2 * J;
+  const size_t rowf = (size_t)fj * fx;
+  // the rows beside: one outside the grid is replaced by the other (its
+  // couplings are taken as zero)
+  const bool hs = fj > 0, hn = fj < fy - 1;
+  const size_t rs = hs ? rowf - fx : rowf + fx, rn = hn ? rowf + fx : rowf - fx;
+  const auto x = gbl(xp);
+  // columns 2 Ic - 2 .. 2 Ic + 2, clamped into the grid, of both rows (the
+  // outer two only meet the diagonal couplings)
+  T xs[5], xn[5];
+  int col[5];
+#pragma unroll
+  for (int a = 0; a < 5; ++a) {
+    const int fi = 2 * Ic + a - 2;
+    col[a] = xslot(fi < 0 ? 0 : fi < fx ? fi : fx - 1, hxf);
+    if (NB == 5 && (a == 0 || a == 4)) continue;
+    xs[a] = x[rs + col[a]];
+    xn[a] = x[rn + col[a]];
+  }
+  T wv[3], cs[3], cn[3], csw[3], cse[3], cnw[3], cne[3];
+#pragma unroll
+  for (int a = 0; a < 3; ++a) {
+    const size_t kf = rowf + col[a + 1];
+    // parent slot of C: 1 for the point to the west, 0 for the one to the
+    // east; the point at C itself is injected with weight exactly 1
+    wv[a] = a == 1 ? T(1) : T(gbl(a == 0 ? w1 : w0)[kf]);
+    cs[a] = gbl(s0)[kf];
+    cn[a] = gbl(n0)[kf];
+    if constexpr (NB == 9) {
+      csw[a] = gbl(sw)[kf]; cse[a] = gbl(se)[kf];
+      cnw[a] = gbl(nw)[kf]; cne[a] = gbl(ne)[kf];
+    }
+  }
+  T sum = T(0);
+#pragma unroll
+  for (int a = 0; a < 3; ++a) {
+    const int fi = 2 * Ic + a - 1;
+    T r = (hs ? cs[a] : T(0)) * xs[a + 1] + (hn ? cn[a] : T(0)) * xn[a + 1];
+    if constexpr (NB == 9) {
+      const bool hw = fi > 0, he = fi < fx - 1;
+      r = fma(hs && hw ? csw[a] : T(0), xs[a], r);
+      r = fma(hs && he ? cse[a] : T(0), xs[a + 2], r);
+      r = fma(hn && hw ? cnw[a] : T(0), xn[a], r);
+      r = fma(hn && he ? cne[a] : T(0), xn[a + 2], r);
+    }
+    sum = fma(fi >= 0 && fi < fx ? wv[a] : T(0), -r, sum);
+  }
+  gbl(out)[(size_t)J * cx + xslot(Ic, half_x(cx))] = sum;
 }
 
 // x_l += P x_{l+1}. ZERO: x_l = P x_{l+1}.
@@ -1192,40 +1258,44 @@ __global__ void __launch_bounds__(kBlock) k_restrict(const InstDev *__restrict__
 // after the prolongation only the colour-1 lines of the first post-smoothing
 // sweep are read (rows 1, 3, .. for x-lines; columns 1, 3, .. for y-lines).
 // The block map covers that compact range.
-template <int ROWS> __device__ __forceinline__ int prolong_count(const Lev &F) {
-  return ROWS == 1 ? F.nx * (F.ny >> 1) : ROWS == 2 ? (F.nx - half_x(F.nx)) * F.ny : F.nx * F.ny;
-}
-
-// A workgroup takes kEnt map entries. Each entry's chain of dependent reads
-// (map entry, instance, its status, its level's pointers) and then its loads
-// are issued before any entry is computed or stored, so a workgroup has
-// kEnt x 256 cells' loads in flight instead of waiting out one chain per 256
-// cells. The terms are those of prolong_point in its order (a zero weight of
-// a parent that point skips adds fma(0, 0, e) = e).
+// A workgroup takes kEnt map entries. The entries' chains of dependent reads
+// (map entry, then the instance's status and level, then the data) run side by
+// side: all map entries, all pointers and statuses (pinned), all data loads, and
+// only then the arithmetic and the stores. A parent outside the coarse grid, at
+// I0 + 1 of an even i or at J0 + 1 of an even j has weight zero, which
+// k_pweights does not store; those terms are skipped.
 template <typename T, bool ZERO, int ROWS>
-__global__ void __launch_bounds__(kBlock) k_prolong(const InstDev *__restrict__ insts,
+__global__ void __launch_bounds__(kBlock) k_prolong(const Insts insts,
                                                    const BlkMap *__restrict__ map, int l,
                                                    int xid, int nmap) {
+  struct Ent { const T *w0, *w1, *w2, *w3, *xc; T *x; int nx, ny, cx, cy, st, k0; } E[kEnt];
+  BlkMap m[kEnt];
+#pragma unroll
+  for (int e = 0; e < kEnt; ++e) m[e] = map[min((int)(kEnt * blockIdx.x) + e, nmap - 1)];
+#pragma unroll
+  for (int e = 0; e < kEnt; ++e) {
+    const InstDev &I = insts[m[e].inst];
+    const Lev &F = I.lev[l], &Cl = I.lev[l + 1];
+    E[e] = {cptr<T>(F.pw[0]), cptr<T>(F.pw[1]), cptr<T>(F.pw[2]), cptr<T>(F.pw[3]), cptr<T>(Cl.x),
+            l == 0 ? ptr<T>(vec(I, xid)) : ptr<T>(F.x), F.nx, F.ny, Cl.nx, Cl.ny,
+            status_of(insts, m[e].inst), m[e].k0};
+  }
+#pragma unroll
+  for (int e = 0; e < kEnt; ++e)
+    pin(E[e].w0, E[e].w1, E[e].w2, E[e].w3, E[e].xc, E[e].x, E[e].nx, E[e].ny, E[e].cx, E[e].cy,
+        E[e].st);
   T a0[kEnt], a1[kEnt], a2[kEnt], a3[kEnt], c0[kEnt], c1[kEnt], c2[kEnt], c3[kEnt], xo[kEnt];
-  T *xs[kEnt];
   int Ks[kEnt];
   bool on[kEnt];
 #pragma unroll
   for (int e = 0; e < kEnt; ++e) {
-    const int bi = kEnt * blockIdx.x + e;
-    on[e] = false;
+    const Ent &F = E[e];
+    const int hx = half_x(F.nx), idx = F.k0 + threadIdx.x;
+    const int count = ROWS == 1 ? F.nx * (F.ny >> 1) : ROWS == 2 ? (F.nx - hx) * F.ny : F.nx * F.ny;
+    on[e] = F.st == ST_ACTIVE && (int)(kEnt * blockIdx.x) + e < nmap && idx < count;
     a0[e] = a1[e] = a2[e] = a3[e] = c0[e] = c1[e] = c2[e] = c3[e] = xo[e] = T(0);
-    xs[e] = nullptr;
     Ks[e] = 0;
-    if (bi >= nmap) continue;
-    const BlkMap m = map[bi];
-    const InstDev &I = insts[m.inst];
-    if (rsc(I)->status != ST_ACTIVE) continue;
-    const Lev &F = I.lev[l];
-    const Lev &Cl = I.lev[l + 1];
-    const int idx = m.k0 + threadIdx.x;
-    if (idx >= prolong_count<ROWS>(F)) continue;
-    const int hx = half_x(F.nx);
+    if (!on[e]) continue;
     int K, i, j;
     if (ROWS == 1) {            // rows 1, 3, ..: nx cells each
       const int r = idx / F.nx, p = idx - r * F.nx;
@@ -1240,22 +1310,19 @@ __global__ void __launch_bounds__(kBlock) k_prolong(const InstDev *__restrict__ 
       cell_ij(K, F.nx, hx, i, j);
     }
     const int I0 = i >> 1, J0 = j >> 1;
-    const int I1 = I0 + 1 < Cl.nx ? I0 + 1 : I0, J1 = J0 + 1 < Cl.ny ? J0 + 1 : J0;
-    const auto xc = gbl(cptr<T>(Cl.x));
-    const int hxc = half_x(Cl.nx);
-    const size_t r0 = (size_t)J0 * Cl.nx, r1 = (size_t)J1 * Cl.nx;
+    const int I1 = I0 + 1 < F.cx ? I0 + 1 : I0, J1 = J0 + 1 < F.cy ? J0 + 1 : J0;
+    const auto xc = gbl(F.xc);
+    const int hxc = half_x(F.cx);
+    const size_t r0 = (size_t)J0 * F.cx, r1 = (size_t)J1 * F.cx;
     const int s0 = xslot(I0, hxc), s1 = xslot(I1, hxc);
     const bool io = i & 1, jo = j & 1;
-    a0[e] = (io || jo) ? gbl(cptr<T>(F.pw[0]))[K] : T(1);   // even-even: injected
+    a0[e] = (io || jo) ? gbl(F.w0)[K] : T(1);   // even-even: injected
     c0[e] = xc[r0 + s0];
-    if (io) { a1[e] = gbl(cptr<T>(F.pw[1]))[K]; c1[e] = xc[r0 + s1]; }
-    if (jo) { a2[e] = gbl(cptr<T>(F.pw[2]))[K]; c2[e] = xc[r1 + s0]; }
-    if (io && jo) { a3[e] = gbl(cptr<T>(F.pw[3]))[K]; c3[e] = xc[r1 + s1]; }
-    T *x = l == 0 ? ptr<T>(vec(I, xid)) : ptr<T>(F.x);
-    if (!ZERO) xo[e] = gbl(x)[K];
-    xs[e] = x;
+    if (io) { a1[e] = gbl(F.w1)[K]; c1[e] = xc[r0 + s1]; }
+    if (jo) { a2[e] = gbl(F.w2)[K]; c2[e] = xc[r1 + s0]; }
+    if (io && jo) { a3[e] = gbl(F.w3)[K]; c3[e] = xc[r1 + s1]; }
+    if (!ZERO) xo[e] = gbl(F.x)[K];
     Ks[e] = K;
-    on[e] = true;
   }
 #pragma unroll
   for (int e = 0; e < kEnt; ++e) {
@@ -1264,7 +1331,7 @@ __global__ void __launch_bounds__(kBlock) k_prolong(const InstDev *__restrict__ 
     v += a1[e] * c1[e];
     v += a2[e] * c2[e];
     v += a3[e] * c3[e];
-    gbl(xs[e])[Ks[e]] = ZERO ? v : xo[e] + v;
+    gbl(E[e].x)[Ks[e]] = ZERO ? v : xo[e] + v;
   }
 }
 
@@ -1278,20 +1345,16 @@ __global__ void __launch_bounds__(kBlock) k_prolong(const InstDev *__restrict__ 
 // no device-wide fence or atomic is needed, and the result of an instance does
 // not depend on the rest of the batch.
 // ---------------------------------------------------------------------------
-template <typename T>
-__device__ __forceinline__ T spmv5(const InstDev &I, size_t K, int i, int j, const T *x) {
-  return stencil_apply<T, 5>(I.lev[0], K, i, j, x);
-}
 
 // PC (FP64 Krylov, FP32 V-cycle): the preconditioned vectors ph = M^-1 p and
 // sh = M^-1 s are FP32 V-cycle outputs scaled by pcs, the residual norm of
 // the iteration (the V-cycle input is the vector divided by pcs, so it stays
 // in FP32 range however far the residual has fallen).
-template <typename T, bool PC>
-__device__ __forceinline__ T precond_vec(const InstDev &I, int id, int pcid, size_t K) {
-  if (PC) return (T)(rsc(I)->pcs * (double)gbl(I.pv[pcid - kNumVec])[K]);
-  return gbl(cptr<T>(I.kv[id]))[K];
-}
+//
+// The SpMVs and the x update read their instance's sizes and vector pointers
+// together with the status (pinned before the status test).
+template <bool PC, typename T> struct Pick { using type = T; };
+template <typename T> struct Pick<true, T> { using type = float; };
 
 // p = r + beta (p - omega v).
 // PC: p is stored only in FP32, divided by the residual norm pcs (it is the
@@ -1309,9 +1372,10 @@ __device__ __forceinline__ T precond_vec(const InstDev &I, int id, int pcid, siz
 // scalars) is latency this light kernel cannot hide within one 256-cell
 // block, and the next entries' chains are issued while the first one's
 // vectors move (the map, the instance table and the scalars are read-only
-// here).
+// here). All entries' loads before any arithmetic measured slower: 82 against
+// 70 us at 4096 x 4096.
 template <typename T, bool PC>
-__global__ void __launch_bounds__(kBlock) k_bicg_p(const InstDev *__restrict__ insts,
+__global__ void __launch_bounds__(kBlock) k_bicg_p(const Insts insts,
                                                   const BlkMap *__restrict__ map, int nmap) {
 #pragma unroll
   for (int e = 0; e < kLightBlocks; ++e) {
@@ -1319,7 +1383,7 @@ __global__ void __launch_bounds__(kBlock) k_bicg_p(const InstDev *__restrict__ i
     if (bi >= nmap) break;
     const BlkMap m = map[bi];
     const InstDev &I = insts[m.inst];
-    if (rsc(I)->status != ST_ACTIVE) continue;
+    if (status_of(insts, m.inst) != ST_ACTIVE) continue;
     const int K = m.k0 + threadIdx.x;
     if (K >= I.nx * I.ny) continue;
     const T beta = (T)rsc(I)->beta, omega = (T)rsc(I)->omega;
@@ -1340,38 +1404,65 @@ __global__ void __launch_bounds__(kBlock) k_bicg_p(const InstDev *__restrict__ i
   }
 }
 
-// the shadow residual rh at slot K (PC: FP32, see k_bicg_p)
+// The level-0 operator of the Krylov iteration: FP64 bands (FP64 and PC32), or
+// the V-cycle's FP32 copies (MIXED).
+template <typename T, bool PC, typename X, typename M>
+__device__ __forceinline__ T krylov_spmv(const M &A, double pcs, int K, const X *x) {
+  int i, j;
+  cell_ij(K, A.nx, half_x(A.nx), i, j);
+  if constexpr (PC) return (T)(pcs * spmv64(A, K, i, j, x));
+  else return stencil_apply<T, 5>(A, K, i, j, x);
+}
+template <typename T, bool PC> struct KrylovOp { using type = Sten<T, 5>; };
+template <typename T> struct KrylovOp<T, true> { using type = Sten64; };
 template <typename T, bool PC>
-__device__ __forceinline__ T shadow(const InstDev &I, size_t K) {
-  if (PC) return (T)gbl(I.pv[PV_RH - kNumVec])[K];
-  return gbl(cptr<T>(I.kv[VRH]))[K];
+__device__ __forceinline__ typename KrylovOp<T, PC>::type krylov_op(const InstDev &I) {
+  if constexpr (PC) return Sten64(I);
+  else return Sten<T, 5>(I.lev[0]);
+}
+
+// partial sums of a workgroup's block by the instance's pinned pointers
+template <typename A, int NV>
+__device__ __forceinline__ void store_partials_at(double *partial, int nblk0, int lblk, A (&v)[NV]) {
+  block_sum<A, NV>(v);
+  if (threadIdx.x == 0) {
+#pragma unroll
+    for (int k = 0; k < NV; ++k) gbl(partial)[(size_t)k * nblk0 + lblk] = (double)v[k];
+  }
 }
 
 // v = M ph; partial (rh, v)
 template <typename T, bool PC>
-__global__ void __launch_bounds__(kBlock) k_bicg_v(const InstDev *__restrict__ insts,
+__global__ void __launch_bounds__(kBlock) k_bicg_v(const Insts insts,
                                                   const BlkMap *__restrict__ map) {
+  using V32 = typename Pick<PC, T>::type;
   const BlkMap m = map[blockIdx.x];
   const InstDev &I = insts[m.inst];
-  if (rsc(I)->status != ST_ACTIVE) return;
+  auto A = krylov_op<T, PC>(I);
+  const V32 *ph = PC ? (const V32 *)I.pv[PV_PH - kNumVec] : (const V32 *)I.kv[VPH];
+  const V32 *rhp = PC ? (const V32 *)I.pv[PV_RH - kNumVec] : (const V32 *)I.kv[VRH];
+  T *vp = ptr<T>(I.kv[VV]);
+  double *partial = I.partial;
+  const KScal *sc = I.sc;
+  int nblk0 = I.nblk0;
+  int st = status_of(insts, m.inst);
+  A.hold();
+  pin(ph, rhp, vp, partial, sc, nblk0, st);
+  if (st != ST_ACTIVE) return;
   const int K = m.k0 + threadIdx.x;
-  const int N = I.nx * I.ny;
   T acc[1] = {T(0)};
-  if (K < N) {
-    int i, j;
-    cell_ij(K, I.nx, half_x(I.nx), i, j);
-    const T rh = shadow<T, PC>(I, K);   // loaded before the store below
-    const T v = PC ? (T)(rsc(I)->pcs * spmv64(I, K, i, j, cptr<float>(I.pv[PV_PH - kNumVec])))
-                   : spmv5<T>(I, K, i, j, cptr<T>(I.kv[VPH]));
-    gbl(ptr<T>(I.kv[VV]))[K] = v;
+  if (K < A.nx * A.ny) {
+    const T rh = (T)gbl(rhp)[K];   // loaded before the store below
+    const T v = krylov_spmv<T, PC>(A, PC ? ((ConstKScal *)sc)->pcs : 1.0, K, ph);
+    gbl(vp)[K] = v;
     acc[0] = rh * v;
   }
-  store_partials<T, 1>(I, m.k0 / kBlock, acc);
+  store_partials_at<T, 1>(partial, nblk0, m.k0 / kBlock, acc);
 }
 
 // s = r - alpha v; partial (s, s); PC: also the scaled FP32 V-cycle input
 template <typename T, bool PC>
-__global__ void __launch_bounds__(kBlock) k_bicg_s(const InstDev *__restrict__ insts,
+__global__ void __launch_bounds__(kBlock) k_bicg_s(const Insts insts,
                                                   const BlkMap *__restrict__ map, int nmap) {
 #pragma unroll
   for (int e = 0; e < kLightBlocks; ++e) {   // kLightBlocks map entries, as k_bicg_p
@@ -1379,7 +1470,7 @@ __global__ void __launch_bounds__(kBlock) k_bicg_s(const InstDev *__restrict__ i
     if (bi >= nmap) break;
     const BlkMap m = map[bi];
     const InstDev &I = insts[m.inst];
-    if (rsc(I)->status != ST_ACTIVE) continue;   // uniform over the workgroup
+    if (status_of(insts, m.inst) != ST_ACTIVE) continue;   // uniform over the workgroup
     const int K = m.k0 + threadIdx.x;
     const int N = I.nx * I.ny;
     T acc[1] = {T(0)};
@@ -1396,40 +1487,57 @@ __global__ void __launch_bounds__(kBlock) k_bicg_s(const InstDev *__restrict__ i
 
 // t = M sh; partials (t, s), (t, t)
 template <typename T, bool PC>
-__global__ void __launch_bounds__(kBlock) k_bicg_t(const InstDev *__restrict__ insts,
+__global__ void __launch_bounds__(kBlock) k_bicg_t(const Insts insts,
                                                   const BlkMap *__restrict__ map) {
+  using V32 = typename Pick<PC, T>::type;
   const BlkMap m = map[blockIdx.x];
   const InstDev &I = insts[m.inst];
-  if (rsc(I)->status != ST_ACTIVE) return;
+  auto A = krylov_op<T, PC>(I);
+  const V32 *sh = PC ? (const V32 *)I.pv[PV_SH - kNumVec] : (const V32 *)I.kv[VSH];
+  const T *sp = cptr<T>(I.kv[VS]);
+  T *tp = ptr<T>(I.kv[VT]);
+  double *partial = I.partial;
+  const KScal *sc = I.sc;
+  int nblk0 = I.nblk0;
+  int st = status_of(insts, m.inst);
+  A.hold();
+  pin(sh, sp, tp, partial, sc, nblk0, st);
+  if (st != ST_ACTIVE) return;
   const int K = m.k0 + threadIdx.x;
-  const int N = I.nx * I.ny;
   T acc[2] = {T(0), T(0)};
-  if (K < N) {
-    int i, j;
-    cell_ij(K, I.nx, half_x(I.nx), i, j);
-    const T sv = gbl(cptr<T>(I.kv[VS]))[K];   // loaded before the store below
-    const T t = PC ? (T)(rsc(I)->pcs * spmv64(I, K, i, j, cptr<float>(I.pv[PV_SH - kNumVec])))
-                   : spmv5<T>(I, K, i, j, cptr<T>(I.kv[VSH]));
-    gbl(ptr<T>(I.kv[VT]))[K] = t;
+  if (K < A.nx * A.ny) {
+    const T sv = gbl(sp)[K];   // loaded before the store below
+    const T t = krylov_spmv<T, PC>(A, PC ? ((ConstKScal *)sc)->pcs : 1.0, K, sh);
+    gbl(tp)[K] = t;
     acc[0] = t * sv;
     acc[1] = t * t;
   }
-  store_partials<T, 2>(I, m.k0 / kBlock, acc);
+  store_partials_at<T, 2>(partial, nblk0, m.k0 / kBlock, acc);
 }
 
 // x += alpha ph + omega sh; r = s - omega t; partials (rh, r), (r, r).
 // HALF (converged at s): x += alpha ph only. XSTATE: x is the FP64 state,
 // otherwise the inner FP32 correction of mixed precision.
 template <typename T, bool XSTATE, bool PC>
-__global__ void __launch_bounds__(kBlock) k_bicg_x(const InstDev *__restrict__ insts,
+__global__ void __launch_bounds__(kBlock) k_bicg_x(const Insts insts,
                                                   const BlkMap *__restrict__ map) {
+  using V32 = typename Pick<PC, T>::type;
   const BlkMap m = map[blockIdx.x];
   const InstDev &I = insts[m.inst];
-  const int st = rsc(I)->status;
+  T *xp = XSTATE ? (T *)I.x : ptr<T>(I.kv[VXK]);
+  const V32 *php = PC ? (const V32 *)I.pv[PV_PH - kNumVec] : (const V32 *)I.kv[VPH];
+  const V32 *shp = PC ? (const V32 *)I.pv[PV_SH - kNumVec] : (const V32 *)I.kv[VSH];
+  const V32 *rhp = PC ? (const V32 *)I.pv[PV_RH - kNumVec] : (const V32 *)I.kv[VRH];
+  const T *sp = cptr<T>(I.kv[VS]), *tp = cptr<T>(I.kv[VT]);
+  T *rp = ptr<T>(I.kv[VR]);
+  double *partial = I.partial;
+  const KScal *scp = I.sc;
+  int nblk0 = I.nblk0, N = I.nx * I.ny;
+  int st = status_of(insts, m.inst);
+  pin(xp, php, shp, rhp, sp, tp, rp, partial, scp, nblk0, N, st);
   if (st != ST_ACTIVE && st != ST_HALF) return;
   const int K = m.k0 + threadIdx.x;
-  const int N = I.nx * I.ny;
-  const T alpha = (T)rsc(I)->alpha, omega = (T)rsc(I)->omega;
+  ConstKScal *const sc = (ConstKScal *)scp;
   T acc[2] = {T(0), T(0)};
   if (K < N) {
     // every load before the first store (the stores could alias the later
@@ -1437,36 +1545,41 @@ __global__ void __launch_bounds__(kBlock) k_bicg_x(const InstDev *__restrict__ i
     // (an instance that converged at s reads sh, s, t and rh needlessly, once;
     // they enter both cases through selects so that their loads are issued
     // with the others)
-    T *x = XSTATE ? (T *)I.x : ptr<T>(I.kv[VXK]);
-    const T xv = gbl(x)[K];
-    const T ph = precond_vec<T, PC>(I, VPH, PV_PH, K);
-    const T sh = precond_vec<T, PC>(I, VSH, PV_SH, K);
-    const T sv = gbl(cptr<T>(I.kv[VS]))[K], tv = gbl(cptr<T>(I.kv[VT]))[K];
-    const T rh = shadow<T, PC>(I, K);
+    const T xv = gbl(xp)[K];
+    const V32 ph0 = gbl(php)[K], sh0 = gbl(shp)[K], rh0 = gbl(rhp)[K];
+    const T sv = gbl(sp)[K], tv = gbl(tp)[K];
+    const T alpha = (T)sc->alpha, omega = (T)sc->omega;
+    const T ph = PC ? (T)(sc->pcs * (double)ph0) : (T)ph0;
+    const T sh = PC ? (T)(sc->pcs * (double)sh0) : (T)sh0;
+    const T rh = (T)rh0;
     const bool act = st != ST_HALF;
     const T xh = xv + alpha * ph;
     const T r = sv - omega * tv;
-    gbl(x)[K] = act ? xh + omega * sh : xh;
+    gbl(xp)[K] = act ? xh + omega * sh : xh;
     acc[0] = act ? rh * r : T(0);
     acc[1] = act ? r * r : T(0);
-    if (act) gbl(ptr<T>(I.kv[VR]))[K] = r;
+    if (act) gbl(rp)[K] = r;
   }
-  if (st == ST_ACTIVE) store_partials<T, 2>(I, m.k0 / kBlock, acc);
+  if (st == ST_ACTIVE) store_partials_at<T, 2>(partial, nblk0, m.k0 / kBlock, acc);
 }
 
 // mixed precision: r64 = R - M x with the FP64 bands; partials (r, r), (R, R)
-__global__ void __launch_bounds__(kBlock) k_ir_residual(const InstDev *__restrict__ insts,
+__global__ void __launch_bounds__(kBlock) k_ir_residual(const Insts insts,
                                                        const BlkMap *__restrict__ map) {
   const BlkMap m = map[blockIdx.x];
   const InstDev &I = insts[m.inst];
-  if (rsc(I)->ostatus != ST_ACTIVE) return;
+  Sten64 M(I);
+  int ost = ostatus_of(insts, m.inst);
+  M.hold();
+  pin(ost);
+  if (ost != ST_ACTIVE) return;
   const int K = m.k0 + threadIdx.x;
   const int N = I.nx * I.ny;
   double v[2] = {0.0, 0.0};
   if (K < N) {
     int i, j;
     cell_ij(K, I.nx, half_x(I.nx), i, j);
-    const double r = gbl(I.R)[K] - spmv64(I, K, i, j, I.x);
+    const double r = gbl(I.R)[K] - spmv64(M, K, i, j, I.x);
     gbl(I.r64)[K] = r;
     v[0] = r * r;
     v[1] = gbl(I.R)[K] * gbl(I.R)[K];
@@ -1475,11 +1588,11 @@ __global__ void __launch_bounds__(kBlock) k_ir_residual(const InstDev *__restric
 }
 
 // inner start: r = r64 / ||r64|| (FP32), rh = r, p = v = xk = 0; partial (r, r)
-__global__ void __launch_bounds__(kBlock) k_ir_inner_init(const InstDev *__restrict__ insts,
+__global__ void __launch_bounds__(kBlock) k_ir_inner_init(const Insts insts,
                                                          const BlkMap *__restrict__ map) {
   const BlkMap m = map[blockIdx.x];
   const InstDev &I = insts[m.inst];
-  if (rsc(I)->ostatus != ST_ACTIVE) return;
+  if (ostatus_of(insts, m.inst) != ST_ACTIVE) return;
   const int K = m.k0 + threadIdx.x;
   const int N = I.nx * I.ny;
   float v[1] = {0.0f};
@@ -1496,11 +1609,11 @@ __global__ void __launch_bounds__(kBlock) k_ir_inner_init(const InstDev *__restr
 }
 
 // x += ||r64|| * xk (FP64)
-__global__ void __launch_bounds__(kBlock) k_ir_update(const InstDev *__restrict__ insts,
+__global__ void __launch_bounds__(kBlock) k_ir_update(const Insts insts,
                                                      const BlkMap *__restrict__ map) {
   const BlkMap m = map[blockIdx.x];
   const InstDev &I = insts[m.inst];
-  if (rsc(I)->ostatus != ST_ACTIVE) return;
+  if (ostatus_of(insts, m.inst) != ST_ACTIVE) return;
   const int K = m.k0 + threadIdx.x;
   if (K >= I.nx * I.ny) return;
   gbl(I.x)[K] += rsc(I)->scale * (double)gbl(ptr<float>(I.kv[VXK]))[K];
@@ -1519,11 +1632,16 @@ __device__ __forceinline__ bool solve_ended(int prec, int status, int ostatus) {
 // clamps), the count of non-finite x and min x (slot 4). The finish
 // kernel decides from them whether the step is accepted; k_commit then writes
 // f. Nothing here writes f.
-__global__ void __launch_bounds__(kBlock) k_finalize(const InstDev *__restrict__ insts,
+__global__ void __launch_bounds__(kBlock) k_finalize(const Insts insts,
                                                     const BlkMap *__restrict__ map) {
   const BlkMap m = map[blockIdx.x];
   const InstDev &I = insts[m.inst];
-  if (rsc(I)->phase != 0 || !solve_ended(I.prec, rsc(I)->status, rsc(I)->ostatus)) return;
+  Sten64 M(I);
+  int phase = phase_of(insts, m.inst), st = status_of(insts, m.inst), ost = ostatus_of(insts, m.inst);
+  int prec = I.prec;
+  M.hold();
+  pin(phase, st, ost, prec);
+  if (phase != 0 || !solve_ended(prec, st, ost)) return;
   const int K = m.k0 + threadIdx.x;
   const int N = I.nx * I.ny;
   double v[4] = {0.0, 0.0, 0.0, 0.0};
@@ -1532,7 +1650,7 @@ __global__ void __launch_bounds__(kBlock) k_finalize(const InstDev *__restrict__
     int i, j;
     cell_ij(K, I.nx, half_x(I.nx), i, j);
     const double xv = gbl(I.x)[K];
-    const double r = gbl(I.R)[K] - spmv64(I, K, i, j, I.x);
+    const double r = gbl(I.R)[K] - spmv64(M, K, i, j, I.x);
     v[0] = r * r;
     v[1] = gbl(I.R)[K] * gbl(I.R)[K];
     v[2] = xv < 0.0 ? 1.0 : 0.0;
@@ -1564,11 +1682,11 @@ __global__ void __launch_bounds__(kBlock) k_finalize(const InstDev *__restrict__
 // With the warm start it also keeps the step's increment df = f_new - f_old
 // and the partial sums (df_new, df_old), (df_old, df_old) from which F_EXTRAP
 // forms the next start's extrapolation factor.
-__global__ void __launch_bounds__(kBlock) k_commit(const InstDev *__restrict__ insts,
+__global__ void __launch_bounds__(kBlock) k_commit(const Insts insts,
                                                   const BlkMap *__restrict__ map) {
   const BlkMap m = map[blockIdx.x];
   const InstDev &I = insts[m.inst];
-  if (rsc(I)->phase != 1 || rsc(I)->ostatus != ST_DONE) return;   // uniform
+  if (phase_of(insts, m.inst) != 1 || ostatus_of(insts, m.inst) != ST_DONE) return;   // uniform
   const int K = m.k0 + threadIdx.x;
   const bool hist = rsc(I)->hist;   // df holds an earlier increment (uniform)
   double v[2] = {0.0, 0.0};
@@ -1625,7 +1743,7 @@ __device__ __forceinline__ void sum_partials(const InstDev &I, A (&tot)[NV]) {
 }
 
 template <typename T, int MODE>
-__global__ void __launch_bounds__(kFinThreads) k_finish(const InstDev *__restrict__ insts, int n,
+__global__ void __launch_bounds__(kFinThreads) k_finish(const Insts insts, int n,
                                                   int *__restrict__ cnt) {
   const int k = blockIdx.x;
   if (k >= n) return;
@@ -1638,7 +1756,7 @@ __global__ void __launch_bounds__(kFinThreads) k_finish(const InstDev *__restric
     if (s.phase != 1 || ost != ST_DONE) return;   // committed in this pass
   } else if (MODE == F_FINALIZE) {
     if (s.phase == 1) {   // committed by the previous pass
-      if (threadIdx.x == 0) s.phase = 2;
+      if (threadIdx.x == 0) s.phase = insts.st[k].phase = 2;
       return;
     }
     if (s.phase != 0 || !solve_ended(I.prec, st, ost)) return;
@@ -1832,6 +1950,7 @@ __global__ void __launch_bounds__(kFinThreads) k_finish(const InstDev *__restric
       s.phase = 1;
     }
   }
+  if (threadIdx.x == 0) insts.st[k] = {s.status, s.ostatus, s.phase, 0};
 }
 
 // (nx,ny) i-major (the reference's Xtensor2d) <-> device cell order, for the
@@ -1872,17 +1991,17 @@ __global__ void __launch_bounds__(kBlock) k_to_imajor(const double *__restrict__
 // ---------------------------------------------------------------------------
 static inline unsigned nblocks(long long n, int b) { return (unsigned)((n + b - 1) / b); }
 
-void launch_begin(hipStream_t s, const InstDev *d, int n, const int *part, int *active,
+void launch_begin(hipStream_t s, const Insts &d, int n, const int *part, int *active,
                   int *oactive, double tol2, double otol2, int maxit, int omaxit) {
   k_begin<<<1, 1024, 0, s>>>(d, n, part, active, oactive, tol2, otol2, maxit, omaxit);
 }
 void launch_copy_counter(hipStream_t s, const int *src, int *dst) {
   k_copy_counter<<<1, 64, 0, s>>>(src, dst);
 }
-void launch_assemble(hipStream_t s, const InstDev *d, const BlkMap *m, int nb) {
+void launch_assemble(hipStream_t s, const Insts &d, const BlkMap *m, int nb) {
   if (nb) k_assemble<<<nb, kBlock, 0, s>>>(d, m);
 }
-void launch_pweights(hipStream_t s, const InstDev *d, const BlkMap *m, int nb, int l, bool mixed) {
+void launch_pweights(hipStream_t s, const Insts &d, const BlkMap *m, int nb, int l, bool mixed) {
   if (!nb) return;
   if (l == 0) {
     if (mixed) k_pweights<float, 5><<<nb, kBlock, 0, s>>>(d, m, l);
@@ -1892,7 +2011,7 @@ void launch_pweights(hipStream_t s, const InstDev *d, const BlkMap *m, int nb, i
     else k_pweights<double, 9><<<nb, kBlock, 0, s>>>(d, m, l);
   }
 }
-void launch_rap(hipStream_t s, const InstDev *d, const BlkMap *m, int nb, int l, bool mixed) {
+void launch_rap(hipStream_t s, const Insts &d, const BlkMap *m, int nb, int l, bool mixed) {
   if (!nb) return;
   if (l == 0) {
     if (mixed) k_rap<float, 5, true><<<nb, kBlock, 0, s>>>(d, m, l);
@@ -1903,7 +2022,7 @@ void launch_rap(hipStream_t s, const InstDev *d, const BlkMap *m, int nb, int l,
   }
 }
 
-void launch_line_factor(hipStream_t s, const InstDev *d, const LineGrp *m, int ngroups, int l,
+void launch_line_factor(hipStream_t s, const Insts &d, const LineGrp *m, int ngroups, int l,
                         int dir, int shape, bool mixed) {
   if (!ngroups) return;
 #define SG_FAC(T, DIR, SH) k_line_factor<T, DIR, SH><<<ngroups, tile_threads(SH), 0, s>>>(d, m, l)
@@ -1922,7 +2041,7 @@ void launch_line_factor(hipStream_t s, const InstDev *d, const LineGrp *m, int n
 }
 
 template <typename T, int SH>
-static void launch_line_s(hipStream_t s, const InstDev *d, const LineGrp *m, int ngroups, int l,
+static void launch_line_s(hipStream_t s, const Insts &d, const LineGrp *m, int ngroups, int l,
                           int dir, bool zero, int xid, int bid) {
   const bool nine = l > 0;
 #define SG_LINE(NB, DIR, Z) \
@@ -1938,7 +2057,7 @@ static void launch_line_s(hipStream_t s, const InstDev *d, const LineGrp *m, int
 }
 
 template <typename T>
-void launch_line(hipStream_t s, const InstDev *d, const LineGrp *m, int ngroups, int l, int dir,
+void launch_line(hipStream_t s, const Insts &d, const LineGrp *m, int ngroups, int l, int dir,
                  int shape, bool zero, int xid, int bid) {
   if (!ngroups) return;
   if (shape == 0) launch_line_s<T, 0>(s, d, m, ngroups, l, dir, zero, xid, bid);
@@ -1947,13 +2066,13 @@ void launch_line(hipStream_t s, const InstDev *d, const LineGrp *m, int ngroups,
   else if (shape == 3) launch_line_s<T, 3>(s, d, m, ngroups, l, dir, zero, xid, bid);
   else launch_line_s<T, 4>(s, d, m, ngroups, l, dir, zero, xid, bid);
 }
-template void launch_line<double>(hipStream_t, const InstDev *, const LineGrp *, int, int, int,
+template void launch_line<double>(hipStream_t, const Insts &, const LineGrp *, int, int, int,
                                   int, bool, int, int);
-template void launch_line<float>(hipStream_t, const InstDev *, const LineGrp *, int, int, int,
+template void launch_line<float>(hipStream_t, const Insts &, const LineGrp *, int, int, int,
                                  int, bool, int, int);
 
 template <typename T>
-void launch_line_shapes(hipStream_t s, const InstDev *d, const LineGrp *m, int na, int nb,
+void launch_line_shapes(hipStream_t s, const Insts &d, const LineGrp *m, int na, int nb,
                         int ngroups, int l, int dir, bool zero, int xid, int bid) {
   if (!ngroups) return;
   if (dir == 0) {
@@ -1967,49 +2086,49 @@ void launch_line_shapes(hipStream_t s, const InstDev *d, const LineGrp *m, int n
     else k_line_shapes<T, 9, 1, false, SA, 0, -1><<<ngroups, 256, 0, s>>>(d, m, na, nb, l, xid, bid);
   }
 }
-template void launch_line_shapes<double>(hipStream_t, const InstDev *, const LineGrp *, int, int,
+template void launch_line_shapes<double>(hipStream_t, const Insts &, const LineGrp *, int, int,
                                          int, int, int, bool, int, int);
-template void launch_line_shapes<float>(hipStream_t, const InstDev *, const LineGrp *, int, int,
+template void launch_line_shapes<float>(hipStream_t, const Insts &, const LineGrp *, int, int,
                                         int, int, int, bool, int, int);
 
 template <typename T>
-void launch_residual(hipStream_t s, const InstDev *d, const BlkMap *m, int nb, int l, int xid,
+void launch_residual(hipStream_t s, const Insts &d, const BlkMap *m, int nb, int l, int xid,
                      int bid) {
   if (!nb) return;
   if (l == 0) k_residual<T, 5><<<nb, kBlock, 0, s>>>(d, m, l, xid, bid);
   else k_residual<T, 9><<<nb, kBlock, 0, s>>>(d, m, l, xid, bid);
 }
-template void launch_residual<double>(hipStream_t, const InstDev *, const BlkMap *, int, int, int,
+template void launch_residual<double>(hipStream_t, const Insts &, const BlkMap *, int, int, int,
                                       int);
-template void launch_residual<float>(hipStream_t, const InstDev *, const BlkMap *, int, int, int,
+template void launch_residual<float>(hipStream_t, const Insts &, const BlkMap *, int, int, int,
                                      int);
 
 template <typename T>
-void launch_restrict_residual(hipStream_t s, const InstDev *d, const BlkMap *m, int nb, int l,
+void launch_restrict_residual(hipStream_t s, const Insts &d, const BlkMap *m, int nb, int l,
                               int xid, int bid) {
   if (!nb) return;
   if (l == 0) k_restrict_residual<T, 5><<<nb, kBlock, 0, s>>>(d, m, l, xid, bid);
   else k_restrict_residual<T, 9><<<nb, kBlock, 0, s>>>(d, m, l, xid, bid);
 }
-template void launch_restrict_residual<double>(hipStream_t, const InstDev *, const BlkMap *, int,
+template void launch_restrict_residual<double>(hipStream_t, const Insts &, const BlkMap *, int,
                                                int, int, int);
-template void launch_restrict_residual<float>(hipStream_t, const InstDev *, const BlkMap *, int,
+template void launch_restrict_residual<float>(hipStream_t, const Insts &, const BlkMap *, int,
                                               int, int, int);
 
 template <typename T>
-void launch_restrict(hipStream_t s, const InstDev *d, const BlkMap *m, int nb, int l, bool from_b,
+void launch_restrict(hipStream_t s, const Insts &d, const BlkMap *m, int nb, int l, bool from_b,
                      int xid, int bid) {
   if (!nb) return;
   if (from_b) k_restrict<T, true><<<nb, kBlock, 0, s>>>(d, m, l, xid, bid);
   else k_restrict<T, false><<<nb, kBlock, 0, s>>>(d, m, l, xid, bid);
 }
-template void launch_restrict<double>(hipStream_t, const InstDev *, const BlkMap *, int, int, bool,
+template void launch_restrict<double>(hipStream_t, const Insts &, const BlkMap *, int, int, bool,
                                       int, int);
-template void launch_restrict<float>(hipStream_t, const InstDev *, const BlkMap *, int, int, bool,
+template void launch_restrict<float>(hipStream_t, const Insts &, const BlkMap *, int, int, bool,
                                      int, int);
 
 template <typename T>
-void launch_prolong(hipStream_t s, const InstDev *d, const BlkMap *m, int nb, int l, bool zero,
+void launch_prolong(hipStream_t s, const Insts &d, const BlkMap *m, int nb, int l, bool zero,
                     int xid, int rows) {
   if (!nb) return;
 #define SG_PRO(Z, R) k_prolong<T, Z, R><<<(nb + kEnt - 1) / kEnt, kBlock, 0, s>>>(d, m, l, xid, nb)
@@ -2017,13 +2136,13 @@ void launch_prolong(hipStream_t s, const InstDev *d, const BlkMap *m, int nb, in
   else { if (rows == 1) SG_PRO(false, 1); else if (rows == 2) SG_PRO(false, 2); else SG_PRO(false, 0); }
 #undef SG_PRO
 }
-template void launch_prolong<double>(hipStream_t, const InstDev *, const BlkMap *, int, int, bool,
+template void launch_prolong<double>(hipStream_t, const Insts &, const BlkMap *, int, int, bool,
                                      int, int);
-template void launch_prolong<float>(hipStream_t, const InstDev *, const BlkMap *, int, int, bool,
+template void launch_prolong<float>(hipStream_t, const Insts &, const BlkMap *, int, int, bool,
                                     int, int);
 
 template <typename T, bool PC>
-static void launch_bicg_t(hipStream_t s, int which, const InstDev *d, const BlkMap *m, int nb,
+static void launch_bicg_t(hipStream_t s, int which, const Insts &d, const BlkMap *m, int nb,
                           bool xstate) {
   switch (which) {
     case 0: k_bicg_p<T, PC><<<(nb + kLightBlocks - 1) / kLightBlocks, kBlock, 0, s>>>(d, m, nb); break;
@@ -2037,19 +2156,19 @@ static void launch_bicg_t(hipStream_t s, int which, const InstDev *d, const BlkM
 }
 
 template <typename T>
-void launch_bicg(hipStream_t s, int which, const InstDev *d, const BlkMap *m, int nb, bool xstate,
+void launch_bicg(hipStream_t s, int which, const Insts &d, const BlkMap *m, int nb, bool xstate,
                  bool pc) {
   if (!nb) return;
   if (pc) launch_bicg_t<double, true>(s, which, d, m, nb, xstate);
   else launch_bicg_t<T, false>(s, which, d, m, nb, xstate);
 }
-template void launch_bicg<double>(hipStream_t, int, const InstDev *, const BlkMap *, int, bool,
+template void launch_bicg<double>(hipStream_t, int, const Insts &, const BlkMap *, int, bool,
                                   bool);
-template void launch_bicg<float>(hipStream_t, int, const InstDev *, const BlkMap *, int, bool,
+template void launch_bicg<float>(hipStream_t, int, const Insts &, const BlkMap *, int, bool,
                                  bool);
 
 template <typename T>
-void launch_finish(hipStream_t s, int mode, const InstDev *d, int n, int *cnt) {
+void launch_finish(hipStream_t s, int mode, const Insts &d, int n, int *cnt) {
   if (!n) return;
   switch (mode) {
     case F_INIT64: k_finish<T, F_INIT64><<<n, kFinThreads, 0, s>>>(d, n, cnt); break;
@@ -2063,22 +2182,22 @@ void launch_finish(hipStream_t s, int mode, const InstDev *d, int n, int *cnt) {
     default: k_finish<T, F_EXTRAP><<<n, kFinThreads, 0, s>>>(d, n, cnt); break;
   }
 }
-template void launch_finish<double>(hipStream_t, int, const InstDev *, int, int *);
-template void launch_finish<float>(hipStream_t, int, const InstDev *, int, int *);
+template void launch_finish<double>(hipStream_t, int, const Insts &, int, int *);
+template void launch_finish<float>(hipStream_t, int, const Insts &, int, int *);
 
-void launch_ir_residual(hipStream_t s, const InstDev *d, const BlkMap *m, int nb) {
+void launch_ir_residual(hipStream_t s, const Insts &d, const BlkMap *m, int nb) {
   if (nb) k_ir_residual<<<nb, kBlock, 0, s>>>(d, m);
 }
-void launch_ir_inner_init(hipStream_t s, const InstDev *d, const BlkMap *m, int nb) {
+void launch_ir_inner_init(hipStream_t s, const Insts &d, const BlkMap *m, int nb) {
   if (nb) k_ir_inner_init<<<nb, kBlock, 0, s>>>(d, m);
 }
-void launch_ir_update(hipStream_t s, const InstDev *d, const BlkMap *m, int nb) {
+void launch_ir_update(hipStream_t s, const Insts &d, const BlkMap *m, int nb) {
   if (nb) k_ir_update<<<nb, kBlock, 0, s>>>(d, m);
 }
-void launch_finalize(hipStream_t s, const InstDev *d, const BlkMap *m, int nb) {
+void launch_finalize(hipStream_t s, const Insts &d, const BlkMap *m, int nb) {
   if (nb) k_finalize<<<nb, kBlock, 0, s>>>(d, m);
 }
-void launch_commit(hipStream_t s, const InstDev *d, const BlkMap *m, int nb) {
+void launch_commit(hipStream_t s, const Insts &d, const BlkMap *m, int nb) {
   if (nb) k_commit<<<nb, kBlock, 0, s>>>(d, m);
 }
 void launch_empty(hipStream_t s, int *p) { k_zero_int<<<1, 64, 0, s>>>(p, 1); }

@@ -15,6 +15,37 @@
 
 namespace sg {
 
+// What a sweep of level l reads: its size, x, b, the line factors and the
+// couplings along and across the lines (DIR 0: rows, 1: columns), read from the
+// instance table together with the status (pinned: sg_device.hpp).
+template <typename T, int NB, bool ZERO, int DIR> struct Lines {
+  T *x;
+  const T *b, *lo, *inv, *cu, *om, *op, *omm, *omp, *opm, *opp;
+  int nx, ny, st;
+  __device__ __forceinline__ Lines(const Insts &insts, int inst, int l, int xid, int bid) {
+    const InstDev &I = insts[inst];
+    const Lev &L = I.lev[l];
+    level_xb<T>(I, l, xid, bid, x, b);
+    lo = cptr<T>(L.band[DIR == 0 ? BW : BS]);
+    inv = cptr<T>(L.linv[DIR]);
+    cu = cptr<T>(L.lup[DIR]);
+    nx = L.nx; ny = L.ny;
+    om = op = omm = omp = opm = opp = nullptr;
+    if (!ZERO) {
+      om = cptr<T>(L.band[DIR == 0 ? BS : BW]);
+      op = cptr<T>(L.band[DIR == 0 ? BN : BE]);
+      if (NB == 9) {
+        omm = cptr<T>(L.band[BSW]); omp = cptr<T>(L.band[DIR == 0 ? BSE : BNW]);
+        opm = cptr<T>(L.band[DIR == 0 ? BNW : BSE]); opp = cptr<T>(L.band[BNE]);
+      }
+    }
+    st = status_of(insts, inst);
+    pin(x, b, lo, inv, cu, nx, ny, st);
+    if constexpr (!ZERO) pin(om, op);
+    if constexpr (!ZERO && NB == 9) pin(omm, omp, opm, opp);
+  }
+};
+
 // LDS values of a column sweep of L columns in C runs: the composed maps of
 // every wave and column, forward and backward.
 template <int L, int C> constexpr int col_lds() { return 4 * (L * C / 64) * L; }
@@ -33,25 +64,15 @@ template <int L, int C> constexpr int col_lds() { return 4 * (L * C / 64) * L; }
 // as 8 columns x 64 runs of 64 took 94 us, as 4 columns x 128 runs of 32 (16
 // byte pieces of a row) 158.
 template <typename T, int NB, bool ZERO, int L, int C, int K>
-__device__ __forceinline__ void col_sweep(const InstDev &I, const LineGrp gr, int l, int xid,
-                                          int bid, T *lds) {
+__device__ __forceinline__ void col_sweep(const Lines<T, NB, ZERO, 1> &P, const LineGrp gr, T *lds) {
   constexpr int NW = L * C / 64;   // waves
   static_assert(L <= 64 && 64 % L == 0 && (L * C) % 64 == 0, "whole runs per wave");
   T *const s_a = lds, *const s_b = s_a + NW * L, *const r_a = s_b + NW * L, *const r_b = r_a + NW * L;
-  const Lev &Lv = I.lev[l];
-  const int nx = Lv.nx, n = Lv.ny, hx = half_x(nx);
-  T *x; const T *b;
-  level_xb<T>(I, l, xid, bid, x, b);
-  const T *__restrict__ lo = cptr<T>(Lv.band[BS]);
-  const T *__restrict__ inv = cptr<T>(Lv.linv[1]);
-  const T *__restrict__ cu = cptr<T>(Lv.lup[1]);
-  const T *__restrict__ om = cptr<T>(Lv.band[BW]);
-  const T *__restrict__ op = cptr<T>(Lv.band[BE]);
-  const T *omm = nullptr, *omp = nullptr, *opm = nullptr, *opp = nullptr;
-  if (NB == 9) {
-    omm = cptr<T>(Lv.band[BSW]); omp = cptr<T>(Lv.band[BNW]);
-    opm = cptr<T>(Lv.band[BSE]); opp = cptr<T>(Lv.band[BNE]);
-  }
+  const int nx = P.nx, n = P.ny, hx = half_x(nx);
+  T *const x = P.x;
+  const T *const b = P.b, *const lo = P.lo, *const inv = P.inv, *const cu = P.cu;
+  const T *const om = P.om, *const op = P.op;
+  const T *const omm = P.omm, *const omp = P.omp, *const opm = P.opm, *const opp = P.opp;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int k = tid % L, c = tid / L;
   const int kc = (n + C - 1) / C;                  // steps per run (uniform, <= K)
@@ -154,44 +175,44 @@ __device__ __forceinline__ void col_sweep(const InstDev &I, const LineGrp gr, in
 }
 
 template <typename T, int NB, bool ZERO>
-__global__ void __launch_bounds__(kColThreads) k_cols(const InstDev *__restrict__ insts,
+__global__ void __launch_bounds__(kColThreads) k_cols(const Insts insts,
                                                       const LineGrp *__restrict__ map, int l,
                                                       int xid, int bid) {
   __shared__ T lds[col_lds<32, 16>()];
   const LineGrp gr = map[blockIdx.x];
-  const InstDev &I = insts[gr.inst];
-  if (rsc(I)->status != ST_ACTIVE) return;
-  const int n = I.lev[l].ny;
-  if (n <= 64) col_sweep<T, NB, ZERO, 32, 16, 4>(I, gr, l, xid, bid, lds);
-  else if (n <= 128) col_sweep<T, NB, ZERO, 16, 32, 4>(I, gr, l, xid, bid, lds);
-  else if (n <= 256) col_sweep<T, NB, ZERO, 16, 32, 8>(I, gr, l, xid, bid, lds);
-  else if (n <= 384) col_sweep<T, NB, ZERO, 16, 32, 12>(I, gr, l, xid, bid, lds);
-  else col_sweep<T, NB, ZERO, 16, 32, 16>(I, gr, l, xid, bid, lds);
+  const Lines<T, NB, ZERO, 1> P(insts, gr.inst, l, xid, bid);
+  if (P.st != ST_ACTIVE) return;
+  const int n = P.ny;
+  if (n <= 64) col_sweep<T, NB, ZERO, 32, 16, 4>(P, gr, lds);
+  else if (n <= 128) col_sweep<T, NB, ZERO, 16, 32, 4>(P, gr, lds);
+  else if (n <= 256) col_sweep<T, NB, ZERO, 16, 32, 8>(P, gr, lds);
+  else if (n <= 384) col_sweep<T, NB, ZERO, 16, 32, 12>(P, gr, lds);
+  else col_sweep<T, NB, ZERO, 16, 32, 16>(P, gr, lds);
 }
 
 template <typename T, int NB, bool ZERO>
-__global__ void __launch_bounds__(kColThreads) k_cols_long(const InstDev *__restrict__ insts,
+__global__ void __launch_bounds__(kColThreads) k_cols_long(const Insts insts,
                                                            const LineGrp *__restrict__ map, int l,
                                                            int xid, int bid) {
   __shared__ T lds[col_lds<16, 32>()];
   const LineGrp gr = map[blockIdx.x];
-  const InstDev &I = insts[gr.inst];
-  if (rsc(I)->status != ST_ACTIVE) return;
-  const int n = I.lev[l].ny;
+  const Lines<T, NB, ZERO, 1> P(insts, gr.inst, l, xid, bid);
+  if (P.st != ST_ACTIVE) return;
+  const int n = P.ny;
   if constexpr (sizeof(T) == 4) {
-    if (n <= 768) col_sweep<T, NB, ZERO, 16, 32, 24>(I, gr, l, xid, bid, lds);
-    else if (n <= 1024) col_sweep<T, NB, ZERO, 8, 64, 16>(I, gr, l, xid, bid, lds);
-    else if (n <= 2048) col_sweep<T, NB, ZERO, 8, 64, 32>(I, gr, l, xid, bid, lds);
-    else col_sweep<T, NB, ZERO, 8, 64, 64>(I, gr, l, xid, bid, lds);
+    if (n <= 768) col_sweep<T, NB, ZERO, 16, 32, 24>(P, gr, lds);
+    else if (n <= 1024) col_sweep<T, NB, ZERO, 8, 64, 16>(P, gr, lds);
+    else if (n <= 2048) col_sweep<T, NB, ZERO, 8, 64, 32>(P, gr, lds);
+    else col_sweep<T, NB, ZERO, 8, 64, 64>(P, gr, lds);
   } else {
-    if (n <= 1024) col_sweep<T, NB, ZERO, 8, 64, 16>(I, gr, l, xid, bid, lds);
-    else if (n <= 2048) col_sweep<T, NB, ZERO, 4, 128, 16>(I, gr, l, xid, bid, lds);
-    else col_sweep<T, NB, ZERO, 4, 128, 32>(I, gr, l, xid, bid, lds);
+    if (n <= 1024) col_sweep<T, NB, ZERO, 8, 64, 16>(P, gr, lds);
+    else if (n <= 2048) col_sweep<T, NB, ZERO, 4, 128, 16>(P, gr, lds);
+    else col_sweep<T, NB, ZERO, 4, 128, 32>(P, gr, lds);
   }
 }
 
 template <typename T>
-void launch_cols(hipStream_t s, const InstDev *d, const LineGrp *m, int ngroups, int l, bool is_long,
+void launch_cols(hipStream_t s, const Insts &d, const LineGrp *m, int ngroups, int l, bool is_long,
                  bool zero, int xid, int bid) {
   if (!ngroups) return;
 #define SG_COLS(NB, Z)                                                                    \
@@ -203,9 +224,9 @@ void launch_cols(hipStream_t s, const InstDev *d, const LineGrp *m, int ngroups,
   else { if (zero) SG_COLS(5, true); else SG_COLS(5, false); }
 #undef SG_COLS
 }
-template void launch_cols<double>(hipStream_t, const InstDev *, const LineGrp *, int, int, bool,
+template void launch_cols<double>(hipStream_t, const Insts &, const LineGrp *, int, int, bool,
                                   bool, int, int);
-template void launch_cols<float>(hipStream_t, const InstDev *, const LineGrp *, int, int, bool,
+template void launch_cols<float>(hipStream_t, const Insts &, const LineGrp *, int, int, bool,
                                  bool, int, int);
 
 // H consecutive values from slot on, in one load (global loads take any
@@ -242,23 +263,13 @@ __device__ __forceinline__ void stv(T *base, uint32_t slot, const T (&v)[H]) {
 // 2048 x 2048 FP64 12.5 -> 6.6 and 39 -> 27; 4096-step rows 62 -> 45 us (3.0
 // TB/s); a batch of 48 uneven grids 8.9 -> 5.5 and 21 (two launches) -> 11.3.
 template <typename T, int NB, bool ZERO, int K, int WL>
-__device__ __forceinline__ void row_sweep(const InstDev &I, const LineGrp gr, int l, int xid,
-                                          int bid, T *lds) {
+__device__ __forceinline__ void row_sweep(const Lines<T, NB, ZERO, 0> &P, const LineGrp gr, T *lds) {
   constexpr int H = K / 2;
-  const Lev &Lv = I.lev[l];
-  const int n = Lv.nx, ny = Lv.ny, hx = half_x(n);
-  T *x; const T *b;
-  level_xb<T>(I, l, xid, bid, x, b);
-  const T *__restrict__ lo = cptr<T>(Lv.band[BW]);
-  const T *__restrict__ inv = cptr<T>(Lv.linv[0]);
-  const T *__restrict__ cu = cptr<T>(Lv.lup[0]);
-  const T *__restrict__ om = cptr<T>(Lv.band[BS]);
-  const T *__restrict__ op = cptr<T>(Lv.band[BN]);
-  const T *omm = nullptr, *omp = nullptr, *opm = nullptr, *opp = nullptr;
-  if (NB == 9) {
-    omm = cptr<T>(Lv.band[BSW]); omp = cptr<T>(Lv.band[BSE]);
-    opm = cptr<T>(Lv.band[BNW]); opp = cptr<T>(Lv.band[BNE]);
-  }
+  const int n = P.nx, ny = P.ny, hx = half_x(n);
+  T *const x = P.x;
+  const T *const b = P.b, *const lo = P.lo, *const inv = P.inv, *const cu = P.cu;
+  const T *const om = P.om, *const op = P.op;
+  const T *const omm = P.omm, *const omp = P.omp, *const opm = P.opm, *const opp = P.opp;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int W = WL > 1 ? 64 : seg_width((n + K - 1) / K);   // lanes per row in a wave
   const int u = lane & (W - 1);
@@ -380,32 +391,32 @@ __device__ __forceinline__ void row_sweep(const InstDev &I, const LineGrp gr, in
 }
 
 template <typename T, int NB, bool ZERO>
-__global__ void __launch_bounds__(kRowThreads) k_rows(const InstDev *__restrict__ insts,
+__global__ void __launch_bounds__(kRowThreads) k_rows(const Insts insts,
                                                       const LineGrp *__restrict__ map, int l,
                                                       int xid, int bid) {
   __shared__ T lds[16];
   const LineGrp gr = map[blockIdx.x];
-  const InstDev &I = insts[gr.inst];
-  if (rsc(I)->status != ST_ACTIVE) return;
-  const int n = I.lev[l].nx;
-  if (sizeof(T) == 8 && n <= 256) row_sweep<T, NB, ZERO, 4, 1>(I, gr, l, xid, bid, lds);
-  else if (n <= 512) row_sweep<T, NB, ZERO, 8, 1>(I, gr, l, xid, bid, lds);
-  else if (n <= 1024) row_sweep<T, NB, ZERO, 8, 2>(I, gr, l, xid, bid, lds);
-  else row_sweep<T, NB, ZERO, 8, 4>(I, gr, l, xid, bid, lds);
+  const Lines<T, NB, ZERO, 0> P(insts, gr.inst, l, xid, bid);
+  if (P.st != ST_ACTIVE) return;
+  const int n = P.nx;
+  if (sizeof(T) == 8 && n <= 256) row_sweep<T, NB, ZERO, 4, 1>(P, gr, lds);
+  else if (n <= 512) row_sweep<T, NB, ZERO, 8, 1>(P, gr, lds);
+  else if (n <= 1024) row_sweep<T, NB, ZERO, 8, 2>(P, gr, lds);
+  else row_sweep<T, NB, ZERO, 8, 4>(P, gr, lds);
 }
 template <typename T, int NB, bool ZERO>
-__global__ void __launch_bounds__(kRowThreads) k_rows_long(const InstDev *__restrict__ insts,
+__global__ void __launch_bounds__(kRowThreads) k_rows_long(const Insts insts,
                                                            const LineGrp *__restrict__ map, int l,
                                                            int xid, int bid) {
   __shared__ T lds[16];
   const LineGrp gr = map[blockIdx.x];
-  const InstDev &I = insts[gr.inst];
-  if (rsc(I)->status != ST_ACTIVE) return;
-  row_sweep<T, NB, ZERO, 16, 4>(I, gr, l, xid, bid, lds);
+  const Lines<T, NB, ZERO, 0> P(insts, gr.inst, l, xid, bid);
+  if (P.st != ST_ACTIVE) return;
+  row_sweep<T, NB, ZERO, 16, 4>(P, gr, lds);
 }
 
 template <typename T>
-void launch_rows(hipStream_t s, const InstDev *d, const LineGrp *m, int ngroups, int l, bool is_long,
+void launch_rows(hipStream_t s, const Insts &d, const LineGrp *m, int ngroups, int l, bool is_long,
                  bool zero, int xid, int bid) {
   if (!ngroups) return;
 #define SG_ROWS(NB, Z)                                                                    \
@@ -417,9 +428,9 @@ void launch_rows(hipStream_t s, const InstDev *d, const LineGrp *m, int ngroups,
   else { if (zero) SG_ROWS(5, true); else SG_ROWS(5, false); }
 #undef SG_ROWS
 }
-template void launch_rows<double>(hipStream_t, const InstDev *, const LineGrp *, int, int, bool,
+template void launch_rows<double>(hipStream_t, const Insts &, const LineGrp *, int, int, bool,
                                   bool, int, int);
-template void launch_rows<float>(hipStream_t, const InstDev *, const LineGrp *, int, int, bool,
+template void launch_rows<float>(hipStream_t, const Insts &, const LineGrp *, int, int, bool,
                                  bool, int, int);
 
 }  // namespace sg
