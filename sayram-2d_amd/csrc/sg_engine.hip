@@ -158,13 +158,12 @@ struct Slot {
 
 // Setup maps cover every level of every instance (assembly, Galerkin chain,
 // line factors). The cycle maps leave out the levels an instance runs in the
-// fused coarse cycle. The factor maps gfac hold the line groups of both
-// colours (a factorisation does not depend on x, so both colours of a
-// direction and tile shape go in one launch).
+// fused coarse cycle. The factor maps fac hold the line groups of both
+// colours and directions (a factorisation does not depend on x), level by
+// level, those of the 1024-thread tile shape apart ([1]).
 struct Maps {
   std::vector<BlkMap> cmap[kMaxLev], pmap[kMaxLev];
-  std::vector<LineGrp> gfac[kMaxLev][2][kNumTileShapes], gcx[kMaxLev][kNumTileShapes],
-      gcy[kMaxLev][kNumTileShapes];
+  std::vector<FacGrp> fac[2];
   // (the sweep maps sw, swx, swy go by sweep shape, the factor maps by tile shape)
   // cycle: restriction into level l, prolongation into level l, sweeps and
   // coarsest solves, and every instance with a fused coarse cycle
@@ -275,10 +274,8 @@ static void xcd_blocks(std::vector<BlkMap> &v, int unit) {
 struct DevMaps {   // offsets into one device buffer
   const BlkMap *cmap[kMaxLev], *pmap[kMaxLev];
   int ncmap[kMaxLev], npmap[kMaxLev];
-  const LineGrp *gfac[kMaxLev][2][kNumTileShapes], *gcx[kMaxLev][kNumTileShapes],
-      *gcy[kMaxLev][kNumTileShapes];
-  int ngfac[kMaxLev][2][kNumTileShapes], ngcx[kMaxLev][kNumTileShapes],
-      ngcy[kMaxLev][kNumTileShapes];
+  const FacGrp *fac[2];
+  int fac_at[2][kMaxLev + 1];   // the groups of level l: fac_at[l] .. fac_at[l + 1] - 1
   const BlkMap *rmap[kMaxLev], *qmap[kMaxLev];
   int nrmap[kMaxLev], nqmap[kMaxLev];
   const LineGrp *sw[kMaxLev][2][2][kNumSweepShapes], *swx[kMaxLev][kNumSweepShapes],
@@ -813,6 +810,7 @@ void Batch::drop_graphs() {
 int Batch::rebuild() {
   drop_graphs();
   Maps M{};
+  std::vector<LineGrp> gfac[kMaxLev][2][kNumTileShapes];   // lines to factor, by level, direction, shape
   order.clear();
   const bool f64 = opts.precision == SG_FP64;   // FP64 V-cycle
   // the lines the first post-smoothing sweep of level l reads
@@ -853,8 +851,8 @@ int Batch::rebuild() {
       if (coarsest && dense) continue;
       if (coarsest) {
         LineGrp g{c, 0, 1, 1};
-        auto &set = ly == 1 ? M.gcx[l][tile_shape(lim, lx, 0, l, f64)]
-                            : M.gcy[l][tile_shape(lim, ly, 1, l, f64)];
+        auto &set = gfac[l][ly != 1][ly == 1 ? tile_shape(lim, lx, 0, l, f64)
+                                             : tile_shape(lim, ly, 1, l, f64)];
         auto &cyc = ly == 1 ? M.swx[l][sweep_shape(lim, lx, 0, l, f64)]
                             : M.swy[l][sweep_shape(lim, ly, 1, l, f64)];
         set.push_back(g);
@@ -868,7 +866,7 @@ int Batch::rebuild() {
           const int per = tile_lines(sh), sper = sweep_lines(ss, n, f64);
           for (int p = 0; p < 2; ++p) {
             for (int f = p; f < nl; f += 2 * per)
-              M.gfac[l][d][sh].push_back({c, f, std::min(per, (nl - f + 1) / 2), 2});
+              gfac[l][d][sh].push_back({c, f, std::min(per, (nl - f + 1) / 2), 2});
             if (l < lf)
               for (int f = p; f < nl; f += 2 * sper)
                 M.sw[l][d][p][ss].push_back({c, f, std::min(sper, (nl - f + 1) / 2), 2});
@@ -891,12 +889,21 @@ int Batch::rebuild() {
           return d == 0 ? table[g.inst].lev[l].nx : table[g.inst].lev[l].ny;
         };
         for (int p = 0; p < (sh < kNumTileShapes ? 3 : 2); ++p) {
-          auto &w = p < 2 ? M.sw[l][d][p][sh] : M.gfac[l][d][sh];
+          auto &w = p < 2 ? M.sw[l][d][p][sh] : gfac[l][d][sh];
           std::stable_sort(w.begin(), w.end(),
                            [&](const LineGrp &a, const LineGrp &b) { return len(a) > len(b); });
           if (d == 1) xcd_chunks(w);
         }
       }
+  int fac_at[2][kMaxLev + 1] = {};
+  for (int l = 0; l < kMaxLev; ++l) {
+    // columns, then rows; the longest lines of each first
+    for (int d = 1; d >= 0; --d)
+      for (int sh = kNumTileShapes - 1; sh >= 0; --sh)
+        for (const LineGrp &g : gfac[l][d][sh])
+          M.fac[sh == 3].push_back({g.inst, g.first, g.count, g.step, l, d, sh, 0});
+    for (int w = 0; w < 2; ++w) fac_at[w][l + 1] = (int)M.fac[w].size();
+  }
   // merged sweep maps of the 9-point levels (the shapes keep their order:
   // each shape's groups longest first, column groups in XCD chunks, whose
   // members stay on one XCD at any offset in the map)
@@ -933,13 +940,10 @@ int Batch::rebuild() {
   sz(M.fmap.size(), sizeof(FuseMap));
   sz(M.dmap.size(), sizeof(FuseMap));
   sz(M.kmap.size(), sizeof(PackMap));
+  for (int w = 0; w < 2; ++w) sz(M.fac[w].size(), sizeof(FacGrp));
   for (int l = 0; l < kMaxLev; ++l) {
     sz(M.cmap[l].size(), sizeof(BlkMap)); sz(M.pmap[l].size(), sizeof(BlkMap));
     sz(M.rmap[l].size(), sizeof(BlkMap)); sz(M.qmap[l].size(), sizeof(BlkMap));
-    for (int sh = 0; sh < kNumTileShapes; ++sh) {
-      for (int d = 0; d < 2; ++d) sz(M.gfac[l][d][sh].size(), sizeof(LineGrp));
-      sz(M.gcx[l][sh].size(), sizeof(LineGrp)); sz(M.gcy[l][sh].size(), sizeof(LineGrp));
-    }
     for (int sh = 0; sh < kNumSweepShapes; ++sh) {
       for (int d = 0; d < 2; ++d)
         for (int p = 0; p < 2; ++p) sz(M.sw[l][d][p][sh].size(), sizeof(LineGrp));
@@ -970,6 +974,10 @@ int Batch::rebuild() {
   dmn.ndmap = (int)M.dmap.size();
   dmn.kmap = (const PackMap *)put(M.kmap.data(), M.kmap.size(), sizeof(PackMap));
   dmn.nkmap = (int)M.kmap.size();
+  for (int w = 0; w < 2; ++w) {
+    dmn.fac[w] = (const FacGrp *)put(M.fac[w].data(), M.fac[w].size(), sizeof(FacGrp));
+    std::copy(fac_at[w], fac_at[w] + kMaxLev + 1, dmn.fac_at[w]);
+  }
   for (int l = 0; l < kMaxLev; ++l) {
     dmn.cmap[l] = (const BlkMap *)put(M.cmap[l].data(), M.cmap[l].size(), sizeof(BlkMap));
     dmn.ncmap[l] = (int)M.cmap[l].size();
@@ -979,17 +987,6 @@ int Batch::rebuild() {
     dmn.nrmap[l] = (int)M.rmap[l].size();
     dmn.qmap[l] = (const BlkMap *)put(M.qmap[l].data(), M.qmap[l].size(), sizeof(BlkMap));
     dmn.nqmap[l] = (int)M.qmap[l].size();
-    for (int sh = 0; sh < kNumTileShapes; ++sh) {
-      for (int d = 0; d < 2; ++d) {
-        auto &v = M.gfac[l][d][sh];
-        dmn.gfac[l][d][sh] = (const LineGrp *)put(v.data(), v.size(), sizeof(LineGrp));
-        dmn.ngfac[l][d][sh] = (int)v.size();
-      }
-      dmn.gcx[l][sh] = (const LineGrp *)put(M.gcx[l][sh].data(), M.gcx[l][sh].size(), sizeof(LineGrp));
-      dmn.ngcx[l][sh] = (int)M.gcx[l][sh].size();
-      dmn.gcy[l][sh] = (const LineGrp *)put(M.gcy[l][sh].data(), M.gcy[l][sh].size(), sizeof(LineGrp));
-      dmn.ngcy[l][sh] = (int)M.gcy[l][sh].size();
-    }
     for (int sh = 0; sh < kNumSweepShapes; ++sh) {
       for (int d = 0; d < 2; ++d)
         for (int p = 0; p < 2; ++p) {
@@ -1243,17 +1240,12 @@ void Batch::setup_kernels(bool start64) {
   launch_begin(stream, insts(), n, d_part, d_cnt, d_cnt + 1, tol2, opts.rtol * opts.rtol,
                mixed ? opts.max_inner : opts.max_iters, opts.max_iters);
   tbegin(0); launch_assemble(stream, insts(), dm.cmap[0], nb0); tend(0);
-  // LU factors of the line matrices of level l: smoothing lines of both
-  // colours (one launch per direction and tile shape) and the exact solve of
-  // a last level that is a line
-  auto factors = [&](int l, hipStream_t s) {
-    for (int d = 0; d < 2; ++d)
-      for (int sh = 0; sh < kNumTileShapes; ++sh)
-        launch_line_factor(s, insts(), dm.gfac[l][d][sh], dm.ngfac[l][d][sh], l, d, sh, h32);
-    for (int sh = 0; sh < kNumTileShapes; ++sh) {
-      launch_line_factor(s, insts(), dm.gcx[l][sh], dm.ngcx[l][sh], l, 0, sh, h32);
-      launch_line_factor(s, insts(), dm.gcy[l][sh], dm.ngcy[l][sh], l, 1, sh, h32);
-    }
+  // LU factors of the line matrices of levels l0 .. l1 - 1: smoothing lines of
+  // both colours and the exact solve of a last level that is a line
+  auto factors = [&](int l0, int l1, hipStream_t s) {
+    for (int w = 0; w < 2; ++w)
+      launch_line_factor(s, insts(), dm.fac[w] + dm.fac_at[w][l0],
+                         dm.fac_at[w][l1] - dm.fac_at[w][l0], w == 1, h32);
   };
   auto note = [&](hipError_t e) { if (e != hipSuccess && fan_err == hipSuccess) fan_err = e; };
   if (side && time_mask == 0) {
@@ -1270,23 +1262,19 @@ void Batch::setup_kernels(bool start64) {
     }
     for (int l = 0; l < dm.maxlev; ++l) {
       note(hipStreamWaitEvent(side, ev_lev[l], 0));
-      factors(l, side);
+      factors(l, l + 1, side);
     }
     launch_dense_inverse(stream, insts(), dm.dmap, dm.ndmap, h32);
     note(hipEventRecord(ev_join, side));
     note(hipStreamWaitEvent(stream, ev_join, 0));
     launch_coarse_pack(stream, insts(), dm.kmap, dm.nkmap, h32);
   } else {
-    for (int l = 0; l < dm.maxlev; ++l) {
-      tbegin(1);
-      factors(l, stream);
-      if (l + 1 < dm.maxlev) {
-        launch_pweights(stream, insts(), dm.pmap[l], dm.npmap[l], l, h32);
-        launch_rap(stream, insts(), dm.cmap[l + 1], dm.ncmap[l + 1], l, h32);
-      }
-      tend(1);
-    }
     tbegin(1);
+    for (int l = 0; l + 1 < dm.maxlev; ++l) {
+      launch_pweights(stream, insts(), dm.pmap[l], dm.npmap[l], l, h32);
+      launch_rap(stream, insts(), dm.cmap[l + 1], dm.ncmap[l + 1], l, h32);
+    }
+    factors(0, dm.maxlev, stream);
     launch_dense_inverse(stream, insts(), dm.dmap, dm.ndmap, h32);
     launch_coarse_pack(stream, insts(), dm.kmap, dm.nkmap, h32);
     tend(1);

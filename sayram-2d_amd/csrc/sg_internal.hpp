@@ -257,6 +257,8 @@ struct InstDev {
 
 struct BlkMap { int inst; int k0; };      // cell-parallel: 256 cells of one instance
 struct LineGrp { int inst; int first; int count; int step; };   // lines first + k*step, k < count
+// lines first + k * step of one colour and direction of a level, by tile shape
+struct FacGrp { int inst, first, count, step, lev, dir, shape, pad; };
 // The instance table a kernel gets, with the statuses of the instances beside
 // it (KScal::status and ostatus by compact index, mirrored by the kernels that
 // change them): a workgroup reads its status and its instance's pointers in

@@ -9,8 +9,8 @@ void launch_begin(hipStream_t s, const Insts &d, int n, const int *part, int *ac
 void launch_assemble(hipStream_t s, const Insts &d, const BlkMap *m, int nb);
 void launch_pweights(hipStream_t s, const Insts &d, const BlkMap *m, int nb, int l, bool mixed);
 void launch_rap(hipStream_t s, const Insts &d, const BlkMap *m, int nb, int l, bool mixed);
-void launch_line_factor(hipStream_t s, const Insts &d, const LineGrp *m, int ngroups, int l,
-                        int dir, int shape, bool mixed);
+void launch_line_factor(hipStream_t s, const Insts &d, const FacGrp *m, int ngroups, bool sh3,
+                        bool h32);
 // shape: tile shape 0..3 of sg_internal.hpp (lines x steps per workgroup)
 template <typename T>
 void launch_line(hipStream_t s, const Insts &d, const LineGrp *m, int ngroups, int l, int dir,
