@@ -484,7 +484,11 @@ __global__ void __launch_bounds__(kBlock) k_pweights(const Insts insts,
 // The terms of fine row 2 J + fb of the support of coarse point (Ic, J):
 // acc[aj][ai] += P(f, C) A(f, g) P(g, C') for the fine points f of that row
 // inside the grid, their stencil neighbours g inside it and the parents C' of
-// g, in that order.
+// g, in that order. Bound on all but the largest grids: load latency. A point
+// outside the grid is read at the nearest point inside and its factors set to
+// zero, so that a row's loads need no branch and are in flight together
+// (against a branch per point: 20 steps of 90 x 100 FP64 16.0 -> 15.1 ms, 10 of
+// 1021 x 765 PC32 41.1 -> 40.2, of 4096 x 4096 PC32 242.6 -> 240.5).
 template <typename T, int NB>
 __device__ __forceinline__ void rap_row(const Lev &F, const T *const (&pw)[4], int Ic, int J,
                                         int fb, int hxf, double (&acc)[3][3]) {
@@ -492,37 +496,68 @@ __device__ __forceinline__ void rap_row(const Lev &F, const T *const (&pw)[4], i
   constexpr int di_[9] = {0, -1, 1, 0, 0, -1, 1, -1, 1};
   constexpr int dj_[9] = {0, 0, 0, -1, 1, -1, -1, 1, 1};
   const int fx = F.nx, fy = F.ny;
-  const int fj = 2 * J + fb;
-  if (fj < 0 || fj >= fy) return;
+  // slots of the columns 2 Ic - 2 .. 2 Ic + 2, and whether they exist
+  uint32_t sl[5];
+  bool ci[5];
+#pragma unroll
+  for (int k = 0; k < 5; ++k) {
+    const int i = 2 * Ic + k - 2;
+    ci[k] = i >= 0 && i < fx;
+    sl[k] = xslot(min(max(i, 0), fx - 1), hxf);
+  }
+  uint32_t row[3];   // rows 2 J + fb - 1 .. 2 J + fb + 1
+  bool cj[3];
+#pragma unroll
+  for (int k = 0; k < 3; ++k) {
+    const int j = 2 * J + fb + k - 1;
+    cj[k] = j >= 0 && j < fy;
+    row[k] = (uint32_t)(min(max(j, 0), fy - 1) * fx);
+  }
+  double a[3][NB], wf[3];
 #pragma unroll
   for (int fa = -1; fa <= 1; ++fa) {
-    const int fi = 2 * Ic + fa;
-    if (fi < 0 || fi >= fx) continue;
-    const size_t kf = (size_t)fj * fx + xslot(fi, hxf);
+    const uint32_t kf = row[1] + sl[fa + 2];
     // slot of C among the parents of f: (I - (fi >> 1)) + 2 (J - (fj >> 1));
     // an even-even f (fa = fb = 0, slot 0) is injected with weight exactly 1
     const int slot = (fa < 0 ? 1 : 0) + 2 * (fb < 0 ? 1 : 0);
-    const double wf = (fa == 0 && fb == 0) ? 1.0 : (double)gbl(pw[slot])[kf];
+    wf[fa + 1] = (fa == 0 && fb == 0) ? 1.0 : (double)ld32(pw[slot], kf);
+#pragma unroll
+    for (int b = 0; b < NB; ++b) a[fa + 1][b] = ld32(cptr<double>(F.band64[b]), kf);
+  }
+  // Weights P(g, C') of the neighbours g that some f of the row couples to.
+  // The parents at I0 + 1 of an even gi and at J0 + 1 of an even gj (gi, gj have
+  // the parities of ga, gb) have weight zero and an even-even g has the single
+  // weight 1 (k_pweights stores neither).
+  double w[3][5][4];
+#pragma unroll
+  for (int kb = 0; kb < 3; ++kb)
+#pragma unroll
+    for (int ka = 0; ka < 5; ++ka) {
+      if (NB == 5 && kb != 1 && (ka == 0 || ka == 4)) continue;
+      const int ga = ka - 2, gb = fb + kb - 1;
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const bool skip = ((q & 1) && !(ga & 1)) || ((q & 2) && !(gb & 1));
+        const bool unit = !(ga & 1) && !(gb & 1);
+        w[kb][ka][q] = skip ? 0.0 : unit ? 1.0 : (double)ld32(pw[q], row[kb] + sl[ka]);
+      }
+    }
+#pragma unroll
+  for (int fa = -1; fa <= 1; ++fa) {
 #pragma unroll
     for (int b = 0; b < NB; ++b) {
-      const int ga = fa + di_[b], gb = fb + dj_[b];
-      const int gi = 2 * Ic + ga, gj = 2 * J + gb;
-      if (gi < 0 || gi >= fx || gj < 0 || gj >= fy) continue;
-      const double wa = wf * gbl(F.band64[b])[kf];
-      const size_t kg = (size_t)gj * fx + xslot(gi, hxf);
+      const int ga = fa + di_[b], gb = fb + dj_[b], ka = ga + 2, kb = dj_[b] + 1;
+      const bool in = ci[fa + 2] && cj[1] && ci[ka] && cj[kb];
+      const double wa = in ? wf[fa + 1] * a[fa + 1][b] : 0.0;
       const int oi = (ga >= 0 ? ga / 2 : -((1 - ga) / 2)) + 1;   // floor(ga / 2) + 1
       const int oj = (gb >= 0 ? gb / 2 : -((1 - gb) / 2)) + 1;
 #pragma unroll
       for (int q = 0; q < 4; ++q) {
         const int ai = oi + (q & 1), aj = oj + (q >> 1);
         if (ai > 2 || aj > 2) continue;   // such parents carry zero weight
-        // so do the parents at I0 + 1 of an even gi and at J0 + 1 of an even
-        // gj (gi, gj have the parities of ga, gb): k_pweights writes exact
-        // zeros there, and the sum skips them
         if (((q & 1) && !(ga & 1)) || ((q & 2) && !(gb & 1))) continue;
-        // an even-even g has the single weight 1 (q = 0 here)
         const bool unit = !(ga & 1) && !(gb & 1);
-        acc[aj][ai] += wa * (unit ? 1.0 : (double)gbl(pw[q])[kg]);
+        acc[aj][ai] += wa * (unit ? 1.0 : in ? w[kb][ka][q] : 0.0);
       }
     }
   }
@@ -710,9 +745,9 @@ __device__ __forceinline__ void line_factor(const InstDev &I, const FacGrp &gr, 
 // The lines of every level, direction and colour in one launch (SH3: those of
 // the 1024-thread shape): a factorisation reads nothing but its operator, so
 // all of them run side by side once the last operator exists, and the short
-// levels cost nothing beside the longest lines. Measured per step against a
-// launch per level, direction and shape: 90 x 100 FP64 28 us less of 826,
-// 1021 x 765 PC32 54 us less of 2100.
+// levels cost nothing beside the longest lines. Measured against a launch per
+// level, direction and shape: 20 steps of 90 x 100 FP64 16.5 -> 16.0 ms, 10 of
+// 1021 x 765 PC32 42.1 -> 41.0.
 template <typename T, bool SH3>
 __global__ void __launch_bounds__(SH3 ? 1024 : 256) k_line_factor(const Insts insts,
                                                                  const FacGrp *__restrict__ map) {
