@@ -132,9 +132,13 @@ __global__ void __launch_bounds__(kFuseThreads) k_coarse_pack(const Insts insts,
       v[1] = get(L.pw[1]);
       v[2] = get(L.pw[2]);
       v[3] = get(L.pw[3]);
-      if (kind == PK_RES) v[0] = (t & 1) ? v[0] : T(0);
       v[1] = (t & 1) ? v[1] : T(0);
       v[3] = (t & 1) ? v[3] : T(0);
+      if (kind == PK_RES) {
+        v[0] = (t & 1) ? v[0] : T(0);
+        v[2] = T(0);
+        v[3] = get(L.band[BS]);   // the first coupling, as a sweep's v[3]
+      }
     } else {
       v[0] = get(L.band[col ? BS : BW]);
       v[1] = get(L.linv[col]);
@@ -252,58 +256,46 @@ __global__ void __launch_bounds__(kFuseThreads) k_coarse_cycle(const Insts insts
     sb[lf == last ? j * fx + i : kDense + (j + 1) * px + 1 + i] = v;
   }
 
-  // Operands of a task, loaded while the one before runs: K steps of up to 9
-  // arrays (TK_RES: 6 couplings and 2 weights; TK_PRO: 4 weights).
+  // Operands of a task, loaded while the one before runs: K steps of 4 or 9
+  // arrays.
   T v[9][4];
   auto fetch = [&](const CoarseTask &t) __attribute__((always_inline)) {
     if ((tid & ~63) >= t.lanes) return;   // no line in this wave
-    const uint32_t s = t.lanes * t.K, o = t.pack + tid * t.K;
     if (t.K == 4) {
-      if (t.kind == TK_PRO) load_pack<4, 0, 4>(pack, o, s, v);
-      else {
-        if (t.kind != TK_RES) load_pack<4, 0, 3>(pack, o, s, v);
-        else load_pack<4, 0, 2>(pack, t.pack2 + 4 * tid, s, v);
-        if (t.kind != TK_ZERO) load_pack<4, 3, 6>(pack, o + 3 * s, s, v);
-      }
+      const uint32_t s = 4 * t.lanes;
+      load_pack<4, 0, 4>(pack, t.pack + 4 * tid, s, v);
+      if (t.pack2 >= 0) load_pack<4, 4, 5>(pack, t.pack2 + 4 * tid, s, v);
     } else {
-      if (t.kind == TK_PRO) load_pack<1, 0, 4>(pack, o, s, v);
-      else {
-        if (t.kind != TK_RES) load_pack<1, 0, 3>(pack, o, s, v);
-        else load_pack<1, 0, 2>(pack, t.pack2 + tid, s, v);
-        if (t.kind != TK_ZERO) load_pack<1, 3, 6>(pack, o + 3 * s, s, v);
-      }
+      const uint32_t s = t.lanes;
+      load_pack<1, 0, 4>(pack, t.pack + tid, s, v);
+      if (t.pack2 >= 0) load_pack<1, 4, 5>(pack, t.pack2 + tid, s, v);
     }
   };
-  // A task by K steps per lane. The operands' registers are refilled for the
-  // next task as soon as they are used up.
-  auto lines = [&](auto kc, const CoarseTask &t, const CoarseTask &tn) __attribute__((always_inline)) {
+  // A task on lines runs in two parts, K steps per lane, between which the
+  // operands of the next task are loaded into the registers the first part has
+  // used up (one copy of the loads: code run for the first time is slow).
+  T r[4], al[4], up[4];
+  T *x;   // the lane's first step
+  int k;  // its line
+  auto first = [&](auto kc, const CoarseTask &t) __attribute__((always_inline)) {
     constexpr int K = decltype(kc)::value;
-    const int u = tid & ((1 << t.lw) - 1), k = tid >> t.lw;
+    const int u = tid & ((1 << t.lw) - 1);
     const int t0 = min(K * u, t.n);   // lanes past the end of the line stay near it
-    const bool line = k < t.nl;
-    T *const x = sx + t.x0 + 2 * min(k, t.nl - 1) * t.sp + t0 * t.sl;
     const int sl = t.sl, sp_ = t.sp;
+    k = tid >> t.lw;
+    x = sx + t.x0 + 2 * min(k, t.nl - 1) * sp_ + t0 * sl;
     if (t.kind == TK_PRO) {   // odd rows, which alone are read before they are solved
       const T *const c = sx + t.aux + min(k, t.nl - 1) * t.pc + (t0 >> 1);
-      T w[4][K], xo[K], s[3], n[3];
-#pragma unroll
-      for (int a = 0; a < 4; ++a)
-#pragma unroll
-        for (int e = 0; e < K; ++e) w[a][e] = v[a][e];
+      T s[3], n[3];
 #pragma unroll
       for (int e = 0; e < (K == 1 ? 2 : 3); ++e) { s[e] = c[e]; n[e] = c[t.pc + e]; }
 #pragma unroll
-      for (int e = 0; e < K; ++e) xo[e] = x[e];
+      for (int e = 0; e < K; ++e) r[e] = x[e];
 #pragma unroll
       for (int e = 0; e < K; ++e)
-        xo[e] += w[0][e] * s[e / 2] + w[1][e] * s[e / 2 + 1] + w[2][e] * n[e / 2] + w[3][e] * n[e / 2 + 1];
-      fetch(tn);
-#pragma unroll
-      for (int e = 0; e < K; ++e)
-        if (line && K * u + e < t.n) x[e] = xo[e];
+        r[e] += v[0][e] * s[e / 2] + v[1][e] * s[e / 2 + 1] + v[2][e] * n[e / 2] + v[3][e] * n[e / 2 + 1];
       return;
     }
-    T r[K];
     if (t.kind != TK_ZERO) {
       T xm[K + 2], xp[K + 2];
 #pragma unroll
@@ -329,49 +321,60 @@ __global__ void __launch_bounds__(kFuseThreads) k_coarse_cycle(const Insts insts
       // the coarse point at an even column: the odd columns beside it send
       // their weighted residuals (a line's last column sends nothing on: its
       // weight is zero, so the lines of a row need no mask).
-      T *const c = sb + t.aux + min(k, t.nl - 1) * t.pc + (t0 >> 1);
       if constexpr (K == 1) {
-        const T o = dpp0<kRowShr | 1>(v[1][0] * r[0]) + r[0] + dpp0<kRowShl | 1>(v[0][0] * r[0]);
-        fetch(tn);
-        if (line && u < t.n && !(u & 1)) c[0] = o;
+        r[0] = dpp0<kRowShr | 1>(v[1][0] * r[0]) + r[0] + dpp0<kRowShl | 1>(v[0][0] * r[0]);
       } else {
         const T west = dpp0<kRowShr | 1>(v[1][3] * r[3]);
-        const T o0 = west + r[0] + v[0][1] * r[1];
-        const T o1 = v[1][1] * r[1] + r[2] + v[0][3] * r[3];
-        fetch(tn);
-        if (line && K * u < t.n) c[0] = o0;
-        if (line && K * u + 2 < t.n) c[1] = o1;
+        r[0] = west + r[0] + v[0][1] * r[1];
+        r[1] = v[1][1] * r[1] + r[2] + v[0][3] * r[3];
       }
       return;
     }
     // Gauss-Seidel on the lines: d_t = al d_{t-1} + (b_t + r_t) inv_t, then
     // x_t = nup x_{t+1} + d_t
     const T *const b = sb + kDense + (x - sx);
-    T al[K], up[K];
 #pragma unroll
     for (int e = 0; e < K; ++e) {
       al[e] = v[0][e];
       up[e] = v[2][e];
       r[e] = (b[e * sl] + r[e]) * v[1][e];
     }
-    fetch(tn);
-    if constexpr (K == 1) {
-      r[0] = scan_row0<true>(al[0], r[0]);
-      r[0] = scan_row0<false>(up[0], r[0]);
-    } else {
-      T A = T(1), B = T(0);
-#pragma unroll
-      for (int e = 0; e < K; ++e) { B = al[e] * B + r[e]; A = e ? al[e] * A : al[e]; }
-      T d = dpp0<kRowShr | 1>(scan_row0<true>(A, B));
-#pragma unroll
-      for (int e = 0; e < K; ++e) { d = al[e] * d + r[e]; r[e] = d; }
-      B = T(0);
-#pragma unroll
-      for (int e = K - 1; e >= 0; --e) { B = up[e] * B + r[e]; A = e < K - 1 ? up[e] * A : up[e]; }
-      T xv = dpp0<kRowShl | 1>(scan_row0<false>(A, B));
-#pragma unroll
-      for (int e = K - 1; e >= 0; --e) { xv = up[e] * xv + r[e]; r[e] = xv; }
+  };
+  auto second = [&](auto kc, const CoarseTask &t) __attribute__((always_inline)) {
+    constexpr int K = decltype(kc)::value;
+    const int u = tid & ((1 << t.lw) - 1);
+    const int t0 = min(K * u, t.n);
+    const bool line = k < t.nl;
+    if (t.kind == TK_RES) {
+      T *const c = sb + t.aux + min(k, t.nl - 1) * t.pc + (t0 >> 1);
+      if constexpr (K == 1) {
+        if (line && u < t.n && !(u & 1)) c[0] = r[0];
+      } else {
+        if (line && K * u < t.n) c[0] = r[0];
+        if (line && K * u + 2 < t.n) c[1] = r[1];
+      }
+      return;
     }
+    if (t.kind != TK_PRO) {
+      if constexpr (K == 1) {
+        r[0] = scan_row0<true>(al[0], r[0]);
+        r[0] = scan_row0<false>(up[0], r[0]);
+      } else {
+        T A = T(1), B = T(0);
+#pragma unroll
+        for (int e = 0; e < K; ++e) { B = al[e] * B + r[e]; A = e ? al[e] * A : al[e]; }
+        T d = dpp0<kRowShr | 1>(scan_row0<true>(A, B));
+#pragma unroll
+        for (int e = 0; e < K; ++e) { d = al[e] * d + r[e]; r[e] = d; }
+        B = T(0);
+#pragma unroll
+        for (int e = K - 1; e >= 0; --e) { B = up[e] * B + r[e]; A = e < K - 1 ? up[e] * A : up[e]; }
+        T xv = dpp0<kRowShl | 1>(scan_row0<false>(A, B));
+#pragma unroll
+        for (int e = K - 1; e >= 0; --e) { xv = up[e] * xv + r[e]; r[e] = xv; }
+      }
+    }
+    const int sl = t.sl;
 #pragma unroll
     for (int e = 0; e < K; ++e)
       if (line && K * u + e < t.n) x[e * sl] = r[e];
@@ -383,15 +386,16 @@ __global__ void __launch_bounds__(kFuseThreads) k_coarse_cycle(const Insts insts
   for (int it = 1; t.kind != TK_END; ++it) {
     const CoarseTask tn = load_task(tasks, it);
     lds_barrier();   // the task before is done
-    if (t.kind <= TK_RES || t.kind == TK_PRO) {
-      if ((tid & ~63) < t.lanes) {   // the wave has a line
-        if (t.K == 4) lines(std::integral_constant<int, 4>(), t, tn);
-        else lines(std::integral_constant<int, 1>(), t, tn);
-      } else {
-        fetch(tn);
-      }
-    } else {
-      fetch(tn);
+    const bool on = (tid & ~63) < t.lanes;   // the wave has a line (cell tasks: none)
+    if (on) {
+      if (t.K == 4) first(std::integral_constant<int, 4>(), t);
+      else first(std::integral_constant<int, 1>(), t);
+    }
+    fetch(tn);
+    if (on) {
+      if (t.K == 4) second(std::integral_constant<int, 4>(), t);
+      else second(std::integral_constant<int, 1>(), t);
+    } else if (t.lanes == 0) {
       const Lev &L = I.lev[t.lev];
       const int nx = L.nx, ny = L.ny, hx = half_x(nx);
       if (t.kind == TK_DENSE) {

@@ -654,8 +654,9 @@ static std::vector<CoarseTask> coarse_tasks(const InstDev &I, int lf, const sg_o
     t.x0 = col ? place(l, colour, 0) : place(l, 0, colour);
     t.sl = col ? px : 1;
     t.sp = col ? 1 : px;
-    t.pack = pk[l - lf] + pack_offset(nx, ny, kind);
-    t.pack2 = pk[l - lf] + pack_offset(nx, ny, PK_RES);
+    const int own = pk[l - lf] + pack_offset(nx, ny, kind);
+    t.pack = task == TK_RES ? pk[l - lf] + pack_offset(nx, ny, PK_RES) : own;
+    t.pack2 = task == TK_SWEEP || task == TK_RES ? own + 4 * g.lanes * g.K : -1;
     return t;
   };
   auto cells = [&](int task, int l) {

@@ -140,11 +140,13 @@ __host__ __device__ constexpr int fused_pitch(int nx) { return (nx + 2) | 1; }
 // Its operator, packed per step in the order its lanes read it, one group of
 // arrays per level and kind: rows and columns of either colour (9 arrays: -lo
 // inv, inv, -up, and the couplings to the lines beside), the weights of the
-// residual's restriction (2, rows of colour 0) and of the prolongation (4,
-// rows of colour 1). Offsets in values from the level's start.
+// residual's restriction (rows of colour 0; 2 arrays, zeros, and the first of
+// the couplings again) and of the prolongation (4, rows of colour 1). A phase
+// reads the first 4 arrays of one group and, if it has couplings, arrays 4 to 8
+// of a sweep's. Offsets in values from the level's start.
 enum PackKind { PK_ROW0, PK_ROW1, PK_COL0, PK_COL1, PK_RES, PK_PRO, kNumPack };
 __host__ __device__ constexpr int pack_arrays(int kind) {
-  return kind < PK_RES ? 9 : kind == PK_RES ? 2 : 4;
+  return kind < PK_RES ? 9 : 4;
 }
 __host__ __device__ constexpr LineLanes pack_lanes(int nx, int ny, int kind) {
   return kind == PK_COL0 || kind == PK_COL1
@@ -161,8 +163,8 @@ __host__ __device__ constexpr int pack_offset(int nx, int ny, int kind) {
 }
 // One phase of the cycle (built once per instance on the host): what it does,
 // the lanes and lines it takes, and its places in LDS: x0 of the first line's
-// step 0, sl and sp the strides along and across the lines; pack: its arrays;
-// aux, pc: place and pitch in the next level (its b or x).
+// step 0, sl and sp the strides along and across the lines; pack: its first 4
+// arrays, pack2: its next 5 (negative: none); aux, pc: place and pitch in the next level (its b or x).
 enum TaskKind { TK_ZERO, TK_SWEEP, TK_RES, TK_RESTB, TK_DENSE, TK_PRO, TK_PROALL, TK_END };
 struct CoarseTask {
   int kind, K, lw, n, nl, lanes, x0, sl, sp, pack, aux, pc, lev, pack2, pad[2];
