@@ -61,10 +61,10 @@ PREC_NAMES = {"pc32": "FP64 BiCGSTAB with an FP32 multigrid preconditioner",
 HBM_PEAK_GBS = 8000.0
 FAMILY_DESC = {
     "assemble": "k_assemble: operator and right-hand side, FP64",
-    "rap": "set-up: k_pweights, k_rap (Galerkin products), k_line_factor",
-    "line_l0": "k_line<T,5,*,false,*>: level-0 zebra line sweeps",
-    "line_coarse": "k_line<T,9,*,*,*>: line sweeps of the per-level coarse levels (9-point)",
-    "restrict": "k_restrict: restriction of the V-cycle right-hand sides",
+    "rap": "set-up: k_pweights, k_rap (Galerkin products), k_line_factor, k_dense_inverse, k_coarse_pack",
+    "line_l0": "k_rows, k_rows_long, k_cols, k_cols_long <T,5,false>: level-0 zebra line sweeps",
+    "line_coarse": "k_rows, k_rows_long, k_cols, k_cols_long <T,9,*>: line sweeps of the per-level coarse levels (9-point)",
+    "restrict": "k_restrict, k_restrict_residual: restriction of the V-cycle right-hand sides",
     "prolong": "k_prolong: prolongation of the coarse corrections",
     "spmv_v": "k_bicg_v: v = M p-hat and (rh, v)",
     "spmv_t": "k_bicg_t: t = M s-hat, (t, s), (t, t)",

@@ -26,10 +26,11 @@
 //    one base, issued while the phase before runs;
 //  * the hierarchy ends at kDense cells: the four levels that would follow an
 //    8 x 8 level cost 32 phases, the product with its inverse one.
-// Measured per cycle (first level): 90 x 100 FP64 (45 x 50) 32 us and 80 x 80
-// FP32 (40 x 40) 15 us; a version with one thread per line took 69 and 31 from
-// half the sides on, one with every level, direction and colour inlined (60
-// KB of code) 78 and 34 from these.
+//  * the code is small: each piece of it runs a few times only, and cold.
+// Measured per cycle (first level): 90 x 100 FP64 (45 x 50) 28 us, 32 with the
+// operand loads inlined at nine places; a version with one thread per line
+// took 69 from half the sides on, one with every level, direction and colour
+// inlined (60 KB of code) 78.
 #include "sg_device.hpp"
 #include "sg_kernels.hpp"
 #include "sg_scan.hpp"

@@ -1424,11 +1424,11 @@ void Batch::count_bytes(const std::vector<int> &part) {
         t_bytes[4] += vc * (3.0 * T * Nl + T * Nc);
       } else {
         // after an x-line pre-sweep: the even rows' residual formed inside
-        // the restriction (b, the bands, x and 2 stored weights per cell in;
-        // b out); otherwise the residual of every cell (b, the bands, x; r
+        // the restriction (the couplings to the odd rows, 2 or 6, and 2 stored
+        // weights per even-row cell, x of the odd rows in; b out); otherwise the residual of every cell (b, the bands, x; r
         // out) and its restriction (r and 2 weights per cell in; b out)
         if (half_residual(sml))
-          t_bytes[4] += vc * (0.5 * Nl * (nb + 4.0) * T + T * Nc);
+          t_bytes[4] += vc * (0.5 * Nl * (nb == 9.0 ? 9.0 : 5.0) * T + T * Nc);
         else
           t_bytes[4] += vc * (Nl * (nb + 3.0) * T + 3.0 * T * Nl + T * Nc);
       }

@@ -11,12 +11,15 @@ that select how the step is launched, and returns the fastest set:
   eagerly (-1).
 * ``line_tiles``: the line lengths at which the line solves switch tile shape
   (rows: short / medium limits; columns: short / medium limits), and
-  ``coarse_tiles`` the same for the coarser levels.
+  ``coarse_tiles`` the same for the coarser levels. The default lengths of a
+  direction select the sweeps that hold lines of at most 4096 cells in
+  registers; any other lengths select tiles.
 * ``streams``: the tile shapes of a sweep on two HIP streams (2) or one (1).
 * ``group_cells``: the size from which instances are stepped as a second
   group, concurrently with the rest (-1: one group).
 * ``fuse_cells``: the size below which an instance's coarse levels run in the
-  fused one-workgroup cycle (-1: never; above 1024 only with an FP32 V-cycle).
+  fused one-workgroup cycle (-1: never; 1024, the default: any level with sides
+  of at most 64; above 1024 only with an FP32 V-cycle).
 
 ``check_every``, ``use_graph``, ``streams`` and ``group_cells`` never change results: every
 instance's result is bit-identical for all their values. ``line_tiles``,
