@@ -53,7 +53,7 @@ struct Dims { int nx, ny; };
 // exactly by one line solve.
 static std::vector<Dims> level_dims(int nx, int ny) {
   std::vector<Dims> v{{nx, ny}};
-  while (std::min(nx, ny) > 1 && nx * ny > kDense) {
+  while (std::min(nx, ny) > 1 && (long long)nx * ny > kDense) {
     nx = (nx + 1) / 2;
     ny = (ny + 1) / 2;
     v.push_back({nx, ny});

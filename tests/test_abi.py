@@ -92,6 +92,17 @@ def test_instance_bytes_accounting():
     assert b64[-1] / (4096 * 4096) < 300
 
 
+@pytest.mark.parametrize("precision", [sg.SG_FP64, sg.SG_MIXED, sg.SG_PC32])
+def test_instance_bytes_of_grids_of_more_than_2_31_cells(precision):
+    """The sizing call takes any sides: the footprint per cell is that of a
+    large grid (within 1%: the same hierarchy, ratio 4 between its levels) on
+    both sides of 2^31 cells, where the cell count no longer fits an int."""
+    def per_cell(n):
+        return sg.Batch.instance_bytes(n, n, precision) / n ** 2
+    for n in (46340, 46341, 65536, 92682):
+        assert abs(per_cell(n) / per_cell(4096) - 1.0) < 0.01, n
+
+
 def test_seeded_case_is_deterministic_and_well_formed():
     a = sc.seeded_case(37, 21, seed=5, scale=2.0)
     b = sc.seeded_case(37, 21, seed=5, scale=2.0)
