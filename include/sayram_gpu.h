@@ -266,6 +266,10 @@ void sg_batch_destroy(sg_batch *b);
 /* Assembly only: writes the 5 FP64 bands (d|w|e|s|n, K = j*nx+i order) and R
  * of the next step into host buffers, for parity checks of the assembly. */
 int sg_debug_assemble(sg_solver *h, double *bands5, double *R);
+/* The multigrid's dense last level alone: the inverse (row-major, N x N, N =
+ * nx ny <= 64, as stored for the V-cycle of that precision) of the 9-point
+ * operator of bands d|w|e|s|n|sw|se|nw|ne, K = j*nx+i order. */
+int sg_debug_dense_inverse(int nx, int ny, int precision, const double *bands9, double *inverse);
 /* Kernel timing with HIP events around every dispatch of a kernel family, on
  * the stream it runs on (the steps then launch eagerly): kernel_id selects the
  * family (see sg_kernel_name), sg_kernel_count() selects every family, -1

@@ -1624,6 +1624,54 @@ int Batch::debug_assemble(int slot, double *bands, double *R) {
   return SG_OK;
 }
 
+// The inverse of a 9-point operator on at most kDense cells by k_dense_inverse,
+// through an instance whose last level it is.
+static int debug_dense_inverse(int nx, int ny, int precision, const double *bands, double *inv) {
+  if (nx < 1 || ny < 1 || (long long)nx * ny > kDense)
+    return fail(SG_ERR_ARG, "the dense level has 1 to 64 cells");
+  if (precision != SG_FP64 && precision != SG_MIXED && precision != SG_PC32)
+    return fail(SG_ERR_ARG, "precision must be SG_FP64, SG_MIXED or SG_PC32");
+  const bool h32 = precision != SG_FP64;
+  const size_t n = (size_t)nx * ny, T = h32 ? sizeof(float) : sizeof(double);
+  struct Head { InstDev inst; InstStat stat; FuseMap map; };
+  const size_t at = a256(sizeof(Head)), bytes = at + 9 * n * sizeof(double) + n * n * T;
+  std::vector<char> h(bytes, 0);
+  char *d = nullptr;
+  int ndev = 0;
+  if (hipGetDeviceCount(&ndev) != hipSuccess || ndev == 0)
+    return fail(SG_ERR_HIP, "no GPU visible: the PPFV step has no CPU fallback");
+  HIPCHK(hipMalloc((void **)&d, bytes));
+  Head head{};
+  head.inst.nlev = 2;   // a Galerkin level: all nine bands
+  head.map = {0, 1, 1, 0};
+  Lev &L = head.inst.lev[1];
+  L.nx = nx; L.ny = ny;
+  double *const hb = (double *)(h.data() + at);
+  for (int b = 0; b < 9; ++b) {
+    L.band64[b] = (double *)(d + at) + b * n;
+    for (int j = 0; j < ny; ++j)
+      for (int i = 0; i < nx; ++i)
+        hb[b * n + cell_slot(i, j, nx)] = bands[b * n + (size_t)j * nx + i];
+  }
+  L.dinv = d + at + 9 * n * sizeof(double);
+  std::memcpy(h.data(), &head, sizeof(head));
+  hipError_t e = hipMemcpy(d, h.data(), bytes, hipMemcpyHostToDevice);
+  if (e == hipSuccess) {
+    launch_dense_inverse(nullptr, Insts{&((Head *)d)->inst, &((Head *)d)->stat},
+                         &((Head *)d)->map, 1, h32);
+    e = hipGetLastError();
+  }
+  if (e == hipSuccess) e = hipMemcpy(h.data(), d, bytes, hipMemcpyDeviceToHost);
+  (void)hipFree(d);
+  if (e != hipSuccess)
+    return fail(SG_ERR_HIP, std::string("dense inverse failed: ") + hipGetErrorString(e));
+  const char *const out = h.data() + at + 9 * n * sizeof(double);
+  for (size_t r = 0; r < n; ++r)   // entry (r, c) at c n + r
+    for (size_t c = 0; c < n; ++c)
+      inv[r * n + c] = h32 ? ((const float *)out)[c * n + r] : ((const double *)out)[c * n + r];
+  return SG_OK;
+}
+
 }  // namespace sg
 
 // ---------------------------------------------------------------------------
@@ -2036,6 +2084,12 @@ void sg_destroy(sg_solver *h) {
   sg_batch_destroy(h->bt);
   delete h;
 }
+int sg_debug_dense_inverse(int nx, int ny, int precision, const double *bands9, double *inverse) {
+  if (!bands9 || !inverse) return fail(SG_ERR_ARG, "bands9 and inverse must not be null");
+  sg::HostLock lk(sg::g_capture_mu);
+  return sg::debug_dense_inverse(nx, ny, precision, bands9, inverse);
+}
+
 int sg_debug_assemble(sg_solver *h, double *bands5, double *R) {
   if (!h || !bands5 || !R) return fail(SG_ERR_ARG, "null argument");
   sg::HostLock lk(sg::g_capture_mu);
