@@ -49,8 +49,8 @@ static size_t a256(size_t x) { return (x + 255) & ~size_t(255); }
 struct Dims { int nx, ny; };
 
 // Coarsen both directions (ceil halving) until a level has at most kDense cells,
-// which the inverse of its operator solves, or one row or column, solved
-// exactly by one line solve.
+// which the inverse of its operator solves (dense_level), or one row or column,
+// solved exactly by one line solve.
 static std::vector<Dims> level_dims(int nx, int ny) {
   std::vector<Dims> v{{nx, ny}};
   while (std::min(nx, ny) > 1 && (long long)nx * ny > kDense) {
@@ -59,6 +59,14 @@ static std::vector<Dims> level_dims(int nx, int ny) {
     v.push_back({nx, ny});
   }
   return v;
+}
+
+// Whether the last of nlev levels is solved by its dense inverse. A single row or
+// column as the only level is not: its line solve is one launch per V-cycle as
+// the dense cycle is, and its factors cost less than the inverse (64 x 1: a step
+// in FP64 78 against 105 us, in PC32 95 against 129).
+static bool dense_level(int nlev, int nx, int ny) {
+  return (long long)nx * ny <= kDense && (nlev > 1 || std::min(nx, ny) > 1);
 }
 
 // Assigns every device pointer of an instance inside one slab starting at
@@ -128,7 +136,7 @@ static size_t carve(uintptr_t base, int nx, int ny, int prec, InstDev &I) {
     }
     if (l + 1 < I.nlev)
       for (int q = 0; q < 4; ++q) L.pw[q] = take(Nl * T);
-    const bool dense = l + 1 == I.nlev && Nl <= kDense;
+    const bool dense = l + 1 == I.nlev && dense_level(I.nlev, L.nx, L.ny);
     for (int d = 0; d < 2 && !dense; ++d) {
       L.linv[d] = take(Nl * T);
       L.lup[d] = take(Nl * T);
@@ -608,8 +616,7 @@ int Batch::upload_bc(Slot &s, int side, const double *vals) {
 }
 
 static bool dense_last(const InstDev &I) {
-  const Lev &L = I.lev[I.nlev - 1];
-  return L.nx * L.ny <= kDense;
+  return dense_level(I.nlev, I.lev[I.nlev - 1].nx, I.lev[I.nlev - 1].ny);
 }
 
 // First level of an instance's fused coarse cycle: its first level that fits,

@@ -50,3 +50,27 @@ def test_edges_of_the_fused_cycle(gpu_lib, precision, smoother, coarse):
                 assert rel_l2(fused[n][k], per_level[n][k]) <= 1e-11, (SHAPES[k], n)
                 slack = 1 if precision != sg.SG_MIXED else 3   # MIXED counts inner iterations
                 assert abs(its[n][k] - its0[n][k]) <= slack, (SHAPES[k], n, its[n][k], its0[n][k])
+
+
+def _launches(problem, precision, **opts):
+    """Dispatches of the V-cycle's kernel families in one step of a solo batch."""
+    b = sg.Batch(sg.make_opts(precision=precision, **opts))
+    slot = b.add(problem)
+    b.time_kernel("all")
+    b.step(1)
+    n = {k: b.kernel_time(k)[1] for k in ("line_l0", "line_coarse", "restrict", "prolong", "coarse_cycle")}
+    f = b.f(slot)
+    b.close()
+    assert rel_l2(f, orc.step(orc.OracleProblem(problem), problem.f0)) <= 1e-10
+    return n
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("precision", [sg.SG_FP64, sg.SG_MIXED, sg.SG_PC32])
+@pytest.mark.parametrize("shape", [(64, 1), (1, 64), (40, 1), (1, 3), (1, 1), (65, 1), (1, 900)])
+def test_a_single_line_takes_line_solves(gpu_lib, shape, precision):
+    """A grid of one row or column has one level, solved by a line solve per
+    V-cycle whatever its length."""
+    n = _launches(sc.seeded_case(*shape, seed=7), precision)
+    assert n["line_coarse"] > 0
+    assert n["coarse_cycle"] == n["line_l0"] == n["restrict"] == n["prolong"] == 0
