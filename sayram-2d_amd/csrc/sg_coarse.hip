@@ -49,7 +49,7 @@ namespace sg {
 // natural order 7e-5 of it), so that order alone is not safe. It is tried
 // first, every multiplier watched; if one exceeds 64 or is not finite the
 // matrix is read again and inverted with partial pivoting. Measured at 90 x 100
-// in FP64 (42 cells): 18.5 us unwatched, 23.7 watched, 40 with pivoting always
+// in FP64 (42 cells): 18.5 us unwatched, 23.0 watched, 40 with pivoting always
 // (each pivot waits for two more LDS reads and a maximum over the waves). A
 // singular operator gives an infinite inverse, which fails the solve at its first
 // reduction.
@@ -73,6 +73,7 @@ __global__ void __launch_bounds__(1024) k_dense_inverse(const Insts insts,
   __shared__ double s_row[2][16][kDense];   // natural order: row 0; pivoting: the waves' candidates
   __shared__ unsigned s_key[2][16];
   __shared__ int s_at[kDense], s_of[kDense];   // pivot row of a column, column of a pivot row
+  __shared__ int s_bad;
   const InstDev &I = insts[map[blockIdx.x].inst];
   if (ostatus_of(insts, map[blockIdx.x].inst) == ST_IDLE) return;
   const Lev &L = I.lev[I.nlev - 1];
@@ -96,8 +97,10 @@ __global__ void __launch_bounds__(1024) k_dense_inverse(const Insts insts,
       a[r] = (nine || b <= BN) ? gbl(L.band64[b])[j * nx + xslot(i, hx)] : 0.0;
     }
   };
+  T *const out = ptr<T>(L.dinv);
   load();
-  int bad = 0;
+  if (threadIdx.x == 0) s_bad = 0;   // (visible at the first barrier)
+  unsigned long long bad = 0;
 #pragma unroll
   for (int rp = 0; rp < R; ++rp) {
 #pragma unroll 1
@@ -106,62 +109,66 @@ __global__ void __launch_bounds__(1024) k_dense_inverse(const Insts insts,
       if (p >= n) break;   // uniform
       if (wave == w) {
         const double inv = 1.0 / rdlane(a[rp], p);
-        s_row[p & 1][0][lane] = lane == p ? inv : a[rp] * inv;
+        a[rp] = lane == p ? inv : a[rp] * inv;
+        s_row[p & 1][0][lane] = a[rp];
       }
       lds_barrier();
       const double rv = s_row[p & 1][0][lane];
-      unsigned below = 0;   // largest magnitude of the column below the pivot
+      double below = 0.0;   // largest entry of the wave's rows below the pivot, column p
 #pragma unroll
       for (int r = 0; r < R; ++r) {
         const double c = rdlane(a[r], p);
-        const bool own = r == rp && wave == w;
-        if (r > rp || (r == rp && wave > w)) below = max(below, mag_bits(c));
-        a[r] = own ? rv : (lane == p ? 0.0 : a[r]) - c * rv;
+        if (r > rp || (r == rp && wave > w)) below = fmax(below, fabs(c));
+        if (r != rp || wave != w) a[r] = (lane == p ? 0.0 : a[r]) - c * rv;
       }
-      // exponents: |c inv| < 2^(ec + ei - 2044)
-      bad |= (below >> 20) + (mag_bits(rdlane(rv, p)) >> 20) > 2050;
+      bad |= __ballot(!(below * fabs(rv) <= 64.0)) & 1ull << p;   // (lane p of rv: 1 / pivot)
     }
   }
-  if (__syncthreads_or(bad)) {
-    load();
-    // Rows do not move: the pivot of column p is the largest entry of that
-    // column (to 14 bits) in a row that was no pivot yet. Each wave offers its
-    // own candidate with the row scaled by it.
-    unsigned rest = 0;   // bit r: row wave + 16 r was no pivot yet
+  if (lane == 0 && bad) s_bad = 1;
+  lds_barrier();
+  if (!__builtin_amdgcn_readfirstlane(s_bad)) {
 #pragma unroll
-    for (int r = 0; r < R; ++r) rest |= (wave + 16 * r < n ? 1u : 0u) << r;
-#pragma unroll 1
-    for (int p = 0; p < n; ++p) {
-      double c[R], cand = a[0], piv = 1.0;
-      unsigned key = 0;   // rows that were pivots, and rows past the matrix
-#pragma unroll
-      for (int r = 0; r < R; ++r) {
-        c[r] = rdlane(a[r], p);
-        const unsigned k = (rest >> r & 1)
-            ? 0x80000000u | (mag_bits(c[r]) & ~63u) | (63 - (wave + 16 * r)) : 0u;
-        if (k > key) { key = k; cand = a[r]; piv = c[r]; }
-      }
-      const double inv = 1.0 / piv;
-      s_row[p & 1][wave][lane] = lane == p ? inv : cand * inv;
-      if (lane == 0) s_key[p & 1][wave] = key;
-      lds_barrier();
-      const unsigned best = row_max(s_key[p & 1][lane & 15]);
-      const int row = 63 - (int)(__builtin_amdgcn_readfirstlane((int)best) & 63);
-      const double rv = s_row[p & 1][row & 15][lane];
-#pragma unroll
-      for (int r = 0; r < R; ++r) {
-        const bool own = row == wave + 16 * r;
-        a[r] = own ? rv : (lane == p ? 0.0 : a[r]) - c[r] * rv;
-        if (own) rest &= ~(1u << r);
-      }
-      if (threadIdx.x == 0) { s_at[p] = row; s_of[row] = p; }
+    for (int r = 0; r < R; ++r) {
+      const int K = wave + 16 * r;
+      if (K < n && lane < n) st32(out, (uint32_t)(lane * n + K), (T)a[r]);
     }
-  } else if (threadIdx.x < n) {
-    s_at[threadIdx.x] = s_of[threadIdx.x] = threadIdx.x;
+    return;
+  }
+  load();
+  // Rows do not move: the pivot of column p is the largest entry of that column
+  // (to 14 bits) in a row that was no pivot yet. Each wave offers its own
+  // candidate with the row scaled by it.
+  unsigned rest = 0;   // bit r: row wave + 16 r was no pivot yet
+#pragma unroll
+  for (int r = 0; r < R; ++r) rest |= (wave + 16 * r < n ? 1u : 0u) << r;
+#pragma unroll 1
+  for (int p = 0; p < n; ++p) {
+    double c[R], cand = a[0], piv = 1.0;
+    unsigned key = 0;   // rows that were pivots, and rows past the matrix
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+      c[r] = rdlane(a[r], p);
+      const unsigned k = (rest >> r & 1)
+          ? 0x80000000u | (mag_bits(c[r]) & ~63u) | (63 - (wave + 16 * r)) : 0u;
+      if (k > key) { key = k; cand = a[r]; piv = c[r]; }
+    }
+    const double inv = 1.0 / piv;
+    s_row[p & 1][wave][lane] = lane == p ? inv : cand * inv;
+    if (lane == 0) s_key[p & 1][wave] = key;
+    lds_barrier();
+    const unsigned best = row_max(s_key[p & 1][lane & 15]);
+    const int row = 63 - (int)(__builtin_amdgcn_readfirstlane((int)best) & 63);
+    const double rv = s_row[p & 1][row & 15][lane];
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+      const bool own = row == wave + 16 * r;
+      a[r] = own ? rv : (lane == p ? 0.0 : a[r]) - c[r] * rv;
+      if (own) rest &= ~(1u << r);
+    }
+    if (threadIdx.x == 0) { s_at[p] = row; s_of[row] = p; }
   }
   lds_barrier();
   // Row K now is row s_of[K] of the inverse, column p stands for column s_at[p].
-  T *const out = ptr<T>(L.dinv);
 #pragma unroll
   for (int r = 0; r < R; ++r) {
     const int K = wave + 16 * r;
