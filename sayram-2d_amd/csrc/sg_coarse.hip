@@ -1,14 +1,14 @@
 // sg_coarse.hip -- the coarse end of the V-cycle: the dense inverse of the last
 // level and the fused coarse cycle.
 //
-// Fused cycle: the levels of one instance from `lev` (its first level with
-// sides of at most kFuseSide and at most fuse_cells cells) down to its last and
-// back, in one workgroup with LDS barriers between the phases, instead of
-// several launches per level. Per level on the way down an optional
-// pre-smoothing sweep of x-lines and the restriction of the residual (of b
-// itself without pre-smoothing); the last level by the inverse of its
-// operator; then per level the prolongation of the lines the first post-sweep
-// reads and the zebra post-sweeps.
+// Fused cycle: the levels of one instance from `lev` (its first level that fits,
+// fused_fits, and has at most fuse_cells cells) down to its last and back, in one
+// workgroup with LDS barriers between the phases, instead of several launches per
+// level. Per level on the way down an optional pre-smoothing sweep of x-lines and
+// the restriction of the residual (of b itself without pre-smoothing); the last
+// level by the inverse of its operator, or as one line if it is a line of more
+// than kDense cells; then per level the prolongation of the lines the first
+// post-sweep reads and the zebra post-sweeps.
 //
 // Bound: latency of one workgroup, which walks 8 phases per level, each a few
 // LDS accesses and some hundred instructions; bytes do not matter. A wave issues
@@ -16,10 +16,13 @@
 // the first time cost more. Hence:
 //  * x and b of every level stay in LDS for the whole cycle, with a border of
 //    zeros, so that no neighbour needs a test;
-//  * a line is a segment of at most 16 lanes (one step per lane, or four), so
-//    that both Thomas recurrences are scans of affine maps inside one DPP row;
-//    the map at a line's first step has A = 0, which separates the lines of a
-//    row without a mask;
+//  * a line of at most 64 cells is a segment of at most 16 lanes (one step per
+//    lane, or four), so that both Thomas recurrences are scans of affine maps
+//    inside one DPP row; the map at a line's first step has A = 0, which separates
+//    the lines of a row without a mask. Lines of up to 256 cells (levels of at most
+//    1024) take two or four rows, chained through v_readlane: against launches per
+//    level 10 steps of 2048 x 32 FP64 18.8 -> 14.9 ms, of 64 grids of 256 x 4 MIXED
+//    18.7 -> 12.8, a step of 66 x 2 MIXED 536 -> 422 us;
 //  * the phases are one loop over a table built with the instance, and the
 //    operator is packed once per step in the order the lanes read it, zero
 //    where a lane has no cell: a phase's operands are a few vector loads from
@@ -244,27 +247,33 @@ __global__ void __launch_bounds__(kFuseThreads) k_coarse_pack(const Insts insts,
 // Fused coarse cycle
 // ---------------------------------------------------------------------------
 // LDS values of x (and as many of b): the sum over the levels of the bordered
-// arrays, for the largest shapes, and what the lanes past a line's end may
-// reach after the last one.
+// arrays, for the largest shapes, or what the lanes past the end of a level's
+// columns may reach: up to 4 rows past its array.
+constexpr int fused_elems_of(int nx, int ny) {
+  int s = 0, most = 0;
+  for (;; nx = (nx + 1) / 2, ny = (ny + 1) / 2) {
+    const int p = fused_pitch(nx);
+    s += p * (ny + 2);
+    most = s + 4 * p > most ? s + 4 * p : most;
+    if (nx == 1 || ny == 1 || nx * ny <= kDense) return most;
+  }
+}
 constexpr int fused_elems(int cells) {
   int most = 0;
-  for (int fx = 1; fx <= kFuseSide; ++fx)
-    for (int fy = 1; fy <= kFuseSide; ++fy) {
-      if (fx * fy > cells) continue;
-      int s = 0;
-      for (int nx = fx, ny = fy;; nx = (nx + 1) / 2, ny = (ny + 1) / 2) {
-        s += fused_pitch(nx) * (ny + 2);
-        if (nx == 1 || ny == 1 || nx * ny <= kDense) break;
-      }
+  for (int nx = 1; nx <= kFuseLong; ++nx)
+    for (int ny = 1; ny <= kFuseLong && nx * ny <= cells && fused_fits(nx, ny); ++ny) {
+      const int s = fused_elems_of(nx, ny);
       most = s > most ? s : most;
     }
-  return most + 5 * fused_pitch(kFuseSide);
+  return most;
 }
+// (colour 0 has the most lines)
 constexpr bool fused_lanes_fit() {
-  for (int nx = 1; nx <= kFuseSide; ++nx)
-    for (int ny = 1; ny <= kFuseSide; ++ny)
-      for (int k = 0; k < kNumPack; ++k)
-        if (pack_lanes(nx, ny, k).lanes > kFuseThreads && nx * ny > kDense) return false;
+  for (int n = 1; n <= kFuseLong; ++n)
+    for (int np = 1; np <= kFuseLong && fused_fits(n, np); ++np) {
+      const LineLanes g = line_lanes(n, np, 0);
+      if (n * np > kDense && (g.lanes > kFuseThreads || g.lw > 6)) return false;
+    }
   return true;
 }
 
@@ -293,30 +302,28 @@ __device__ __forceinline__ CoarseTask load_task(const CoarseTask *p, int it) {
   return t;
 }
 
-template <typename T, int CAP>
-__global__ void __launch_bounds__(kFuseThreads) k_coarse_cycle(const Insts insts,
-                                                               const FuseMap *__restrict__ map,
-                                                               int xid, int bid) {
-  static_assert(fused_lanes_fit(), "every line of a colour has its lanes");
-  constexpr int XN = fused_elems(CAP), NW = kFuseThreads / 64, DC = kDense / NW;
-  __shared__ T sx[XN];              // x of the levels, bordered
-  __shared__ T sb[kDense + XN];     // the dense level's b, then b in the places of x
-  __shared__ T sp[NW * kDense];
-  const FuseMap fm = map[blockIdx.x];
-  const InstDev &I = insts[fm.inst];
-  const CoarseTask *tasks = I.tasks;
-  const T *pack = cptr<T>(I.pack);
+// What the cycle of an instance reads from its table (pinned: sg_device.hpp).
+template <typename T> struct CycleIn {
+  const CoarseTask *tasks;
+  const T *pack, *bg, *dinv;
+  T *xg;
+  int lf, last, fx, fy, dx, dy;
+};
+
+// sx: x of the levels, bordered (XN values); sb: the dense level's b, then b in the
+// places of x; sp: partial products of the dense level. ROWS: the instance has
+// lines longer than a row of lanes.
+template <typename T, int XN, bool ROWS>
+__device__ __forceinline__ void coarse_cycle(const InstDev &I, const CycleIn<T> &C, T *const sx,
+                                             T *const sb, T *const sp) {
+  constexpr int NW = kFuseThreads / 64, DC = kDense / NW;
+  const CoarseTask *const tasks = C.tasks;
+  const T *const pack = C.pack, *const bg = C.bg, *const dinv = C.dinv;
+  T *const xg = C.xg;
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int lf = fm.lev, last = fm.last;
-  T *xg; const T *bg;
-  level_xb<T>(I, lf, xid, bid, xg, bg);
-  int fx = I.lev[lf].nx, fy = I.lev[lf].ny, dx = I.lev[last].nx, dy = I.lev[last].ny;
-  const T *dinv = cptr<T>(I.lev[last].dinv);
-  int st = status_of(insts, fm.inst);
-  pin(tasks, pack, xg, bg, fx, fy, dx, dy, dinv, st);
-  if (st != ST_ACTIVE) return;
-  const int px = fused_pitch(fx), hxf = half_x(fx), dn = dx * dy;
+  const int lf = C.lf, last = C.last, fx = C.fx, fy = C.fy, dx = C.dx, dy = C.dy;
+  const int px = fused_pitch(fx), hxf = half_x(fx), dn = dinv ? dx * dy : 0;
   // this wave's columns of the last level's inverse, rows on the lanes
   T dv[DC];
 #pragma unroll
@@ -400,7 +407,7 @@ __global__ void __launch_bounds__(kFuseThreads) k_coarse_cycle(const Insts insts
       if constexpr (K == 1) {
         r[0] = dpp0<kRowShr | 1>(v[1][0] * r[0]) + r[0] + dpp0<kRowShl | 1>(v[0][0] * r[0]);
       } else {
-        const T west = dpp0<kRowShr | 1>(v[1][3] * r[3]);
+        const T west = dpp0<ROWS ? kWaveShr1 : kRowShr | 1>(v[1][3] * r[3]);
         r[0] = west + r[0] + v[0][1] * r[1];
         r[1] = v[1][1] * r[1] + r[2] + v[0][3] * r[3];
       }
@@ -439,13 +446,14 @@ __global__ void __launch_bounds__(kFuseThreads) k_coarse_cycle(const Insts insts
         T A = T(1), B = T(0);
 #pragma unroll
         for (int e = 0; e < K; ++e) { B = al[e] * B + r[e]; A = e ? al[e] * A : al[e]; }
-        T d = dpp0<kRowShr | 1>(scan_row0<true>(A, B));
+        const bool rows = ROWS && t.lw > 4;   // uniform
+        T d = rows ? enter_rows0<true>(A, B) : enter_row0<true>(A, B);
 #pragma unroll
         for (int e = 0; e < K; ++e) { d = al[e] * d + r[e]; r[e] = d; }
         B = T(0);
 #pragma unroll
         for (int e = K - 1; e >= 0; --e) { B = up[e] * B + r[e]; A = e < K - 1 ? up[e] * A : up[e]; }
-        T xv = dpp0<kRowShl | 1>(scan_row0<false>(A, B));
+        T xv = rows ? enter_rows0<false>(A, B) : enter_row0<false>(A, B);
 #pragma unroll
         for (int e = K - 1; e >= 0; --e) { xv = up[e] * xv + r[e]; r[e] = xv; }
       }
@@ -532,6 +540,36 @@ __global__ void __launch_bounds__(kFuseThreads) k_coarse_cycle(const Insts insts
     const int j = c / fx, i = xcol(c - j * fx, hxf);
     st32(xg, (uint32_t)c, sx[(j + 1) * px + 1 + i]);
   }
+}
+
+// Instances with long lines run code of their own: with one copy for both the
+// short lines' code is larger, and cold code is time (10 steps of 41 x 33 FP64 4.83
+// ms with one copy, 4.70 with two).
+template <typename T, int CAP>
+__global__ void __launch_bounds__(kFuseThreads) k_coarse_cycle(const Insts insts,
+                                                               const FuseMap *__restrict__ map,
+                                                               int xid, int bid) {
+  static_assert(fused_lanes_fit(), "every line of a colour has its lanes");
+  constexpr int XN = fused_elems(CAP);
+  __shared__ T sx[XN];
+  __shared__ T sb[kDense + XN];
+  __shared__ T sp[kFuseThreads / 64 * kDense];
+  const FuseMap fm = map[blockIdx.x];
+  const InstDev &I = insts[fm.inst];
+  CycleIn<T> C;
+  C.tasks = I.tasks;
+  C.pack = cptr<T>(I.pack);
+  C.lf = fm.lev;
+  C.last = fm.last;
+  level_xb<T>(I, C.lf, xid, bid, C.xg, C.bg);
+  C.fx = I.lev[C.lf].nx; C.fy = I.lev[C.lf].ny;
+  C.dx = I.lev[C.last].nx; C.dy = I.lev[C.last].ny;
+  C.dinv = cptr<T>(I.lev[C.last].dinv);
+  int st = status_of(insts, fm.inst);
+  pin(C.tasks, C.pack, C.xg, C.bg, C.fx, C.fy, C.dx, C.dy, C.dinv, st);
+  if (st != ST_ACTIVE) return;
+  if (__builtin_expect(fm.rows == 0, 1)) coarse_cycle<T, XN, false>(I, C, sx, sb, sp);
+  else coarse_cycle<T, XN, true>(I, C, sx, sb, sp);
 }
 
 void launch_dense_inverse(hipStream_t s, const Insts &d, const FuseMap *m, int n, bool h32) {

@@ -61,12 +61,25 @@ static std::vector<Dims> level_dims(int nx, int ny) {
   return v;
 }
 
+// Packed kind of a last level that is a line.
+static int line_kind(int ny) { return ny == 1 ? PK_ROW0 : PK_COL0; }
+
 // Whether the last of nlev levels is solved by its dense inverse. A single row or
 // column as the only level is not: its line solve is one launch per V-cycle as
 // the dense cycle is, and its factors cost less than the inverse (64 x 1: a step
 // in FP64 78 against 105 us, in PC32 95 against 129).
 static bool dense_level(int nlev, int nx, int ny) {
   return (long long)nx * ny <= kDense && (nlev > 1 || std::min(nx, ny) > 1);
+}
+
+// Values of level l's packed operator in the fused cycle: every kind, of a last
+// level that is a line its one row or column, of a dense one nothing.
+static size_t fused_pack(int nlev, int l, int nx, int ny) {
+  if (l + 1 < nlev) return pack_offset(nx, ny, kNumPack);
+  if (nlev == 1 || dense_level(nlev, nx, ny)) return 0;
+  const int kind = line_kind(ny);
+  const LineLanes g = pack_lanes(nx, ny, kind);
+  return (size_t)pack_arrays(kind) * g.lanes * g.K;
 }
 
 // Assigns every device pointer of an instance inside one slab starting at
@@ -111,9 +124,9 @@ static size_t carve(uintptr_t base, int nx, int ny, int prec, InstDev &I) {
   // first level it may have
   I.tasks = (const CoarseTask *)take(kMaxTasks * sizeof(CoarseTask));
   size_t packed = 0;
-  for (size_t l = 0; l + 1 < dims.size(); ++l)
-    if (std::max(dims[l].nx, dims[l].ny) <= kFuseSide)
-      packed += pack_offset(dims[l].nx, dims[l].ny, kNumPack);
+  for (size_t l = 0; l < dims.size(); ++l)
+    if (fused_fits(dims[l].nx, dims[l].ny))
+      packed += fused_pack(I.nlev, (int)l, dims[l].nx, dims[l].ny);
   I.pack = packed ? take(packed * T) : nullptr;
   for (int l = 0; l < kMaxLev; ++l) {
     Lev &L = I.lev[l];
@@ -381,7 +394,7 @@ struct Batch {
   int rebuild();
   int fuse_level(const InstDev &I) const;
   Insts insts() const { return {d_insts, d_stat}; }
-  // largest fused level: the default takes any with sides of at most kFuseSide
+  // largest fused level: the default takes any that fits
   int fuse_cap() const { return opts.fuse_cells == kFuseCells ? kFuseCells32 : opts.fuse_cells; }
   int step(int nsteps, const int64_t *targets, int ntargets);
   int step_once();
@@ -619,32 +632,33 @@ static bool dense_last(const InstDev &I) {
   return dense_level(I.nlev, I.lev[I.nlev - 1].nx, I.lev[I.nlev - 1].ny);
 }
 
-// First level of an instance's fused coarse cycle: its first level that fits,
-// but only its dense last level when fusion is off or the schedule has a
-// y-line pre-sweep (which the fused cycle does not run); nlev (none) when the
-// last level is a line. It depends only on the instance and the options.
+// First level of an instance's fused coarse cycle: its first level that fits. Only
+// the dense last level, or none (nlev) if the last level is a line, when fusion
+// is off or the schedule has a y-line pre-sweep (which the fused cycle does not
+// run); none when a line would be its only level (one launch either way). It
+// depends only on the instance and the options.
 int Batch::fuse_level(const InstDev &I) const {
-  if (!dense_last(I)) return I.nlev;
+  const int last = I.nlev - 1, end = dense_last(I) ? last : I.nlev;
   if (opts.fuse_cells >= 0 && !((opts.smoother | opts.coarse_smoother) & 2))
-    for (int l = 0; l < I.nlev; ++l)
-      if (std::max(I.lev[l].nx, I.lev[l].ny) <= kFuseSide &&
-          I.lev[l].nx * I.lev[l].ny <= fuse_cap())
+    for (int l = 0; l < last; ++l)
+      if (fused_fits(I.lev[l].nx, I.lev[l].ny) && I.lev[l].nx * I.lev[l].ny <= fuse_cap())
         return l;
-  return I.nlev - 1;
+  return end;
 }
 
 // The phases of an instance's fused coarse cycle from level lf: per level on
 // the way down an x-line pre-sweep and the restriction of its residual (or the
-// restriction of b), the dense solve, per level on the way up the prolongation
-// and the post-sweeps.
+// restriction of b), the dense solve or the line solve of the last level, per
+// level on the way up the prolongation and the post-sweeps.
 static std::vector<CoarseTask> coarse_tasks(const InstDev &I, int lf, const sg_opts &o) {
   const int last = I.nlev - 1;
+  const bool dense = dense_last(I);
   std::vector<CoarseTask> v;
   std::vector<int> xo(1, 0), pk(1, 0);   // by level: places in LDS, packed arrays
   for (int l = lf; l <= last; ++l) {
     const int nx = I.lev[l].nx, ny = I.lev[l].ny;
     xo.push_back(xo.back() + fused_pitch(nx) * (ny + 2));
-    pk.push_back(pk.back() + (l < last ? pack_offset(nx, ny, kNumPack) : 0));
+    pk.push_back(pk.back() + (int)fused_pack(I.nlev, l, nx, ny));
   }
   auto place = [&](int l, int i, int j) {
     return xo[l - lf] + (j + 1) * fused_pitch(I.lev[l].nx) + 1 + i;
@@ -661,7 +675,7 @@ static std::vector<CoarseTask> coarse_tasks(const InstDev &I, int lf, const sg_o
     t.x0 = col ? place(l, colour, 0) : place(l, 0, colour);
     t.sl = col ? px : 1;
     t.sp = col ? 1 : px;
-    const int own = pk[l - lf] + pack_offset(nx, ny, kind);
+    const int own = pk[l - lf] + (l < last ? pack_offset(nx, ny, kind) : 0);
     t.pack = task == TK_RES ? pk[l - lf] + pack_offset(nx, ny, PK_RES) : own;
     t.pack2 = task == TK_SWEEP || task == TK_RES ? own + 4 * g.lanes * g.K : -1;
     return t;
@@ -676,8 +690,9 @@ static std::vector<CoarseTask> coarse_tasks(const InstDev &I, int lf, const sg_o
   for (int l = lf; l < last; ++l) {
     const int s = l == 0 ? o.smoother : o.coarse_smoother;
     // b of the next level: the dense one's in row order, else bordered
-    const int aux = l + 1 == last ? 0 : kDense + place(l + 1, 0, 0);
-    const int pc = l + 1 == last ? I.lev[last].nx : fused_pitch(I.lev[l + 1].nx);
+    const bool rows = dense && l + 1 == last;
+    const int aux = rows ? 0 : kDense + place(l + 1, 0, 0);
+    const int pc = rows ? I.lev[last].nx : fused_pitch(I.lev[l + 1].nx);
     if (s & 1) {
       v.push_back(lines(TK_ZERO, l, PK_ROW0));
       v.push_back(lines(TK_SWEEP, l, PK_ROW1));
@@ -688,7 +703,7 @@ static std::vector<CoarseTask> coarse_tasks(const InstDev &I, int lf, const sg_o
     v.back().aux = aux;
     v.back().pc = pc;
   }
-  v.push_back(cells(TK_DENSE, last));
+  v.push_back(dense ? cells(TK_DENSE, last) : lines(TK_ZERO, last, line_kind(I.lev[last].ny)));
   for (int l = last - 1; l >= lf; --l) {
     const int s = l == 0 ? o.smoother : o.coarse_smoother;
     v.push_back(s & 4 ? lines(TK_PRO, l, PK_PRO) : cells(TK_PROALL, l));
@@ -768,8 +783,8 @@ int Batch::add(const sg_grid *g, const sg_coeffs *c, const sg_bc *bc, const doub
   vertex_weights(g->y_edges, ny, w0, w1);
   (void)hipMemcpy((void *)s.dev.wy0, w0.data(), (ny + 1) * 8, hipMemcpyHostToDevice);
   (void)hipMemcpy((void *)s.dev.wy1, w1.data(), (ny + 1) * 8, hipMemcpyHostToDevice);
-  if (dense_last(s.dev)) {
-    const std::vector<CoarseTask> t = coarse_tasks(s.dev, fuse_level(s.dev), opts);
+  if (const int lf = fuse_level(s.dev); lf < s.dev.nlev) {
+    const std::vector<CoarseTask> t = coarse_tasks(s.dev, lf, opts);
     if (t.size() > (size_t)kMaxTasks ||
         hipMemcpy((void *)s.dev.tasks, t.data(), t.size() * sizeof(CoarseTask),
                   hipMemcpyHostToDevice) != hipSuccess)
@@ -834,13 +849,18 @@ int Batch::rebuild() {
     maxlev = std::max(maxlev, I.nlev);
     const int lf = fuse_level(I);
     slots[k].fuse_lev = lf;
-    if (lf < I.nlev) M.fmap.push_back({c, lf, I.nlev - 1, 0});
+    if (lf < I.nlev)
+      M.fmap.push_back({c, lf, I.nlev - 1, std::max(I.lev[lf].nx, I.lev[lf].ny) > kFuseSide});
     const bool dense = dense_last(I);
     if (dense) M.dmap.push_back({c, I.nlev - 1, I.nlev - 1, 0});
-    for (int l = lf, off = 0; l + 1 < I.nlev; ++l) {
-      for (int kind = 0; kind < kNumPack; ++kind)
-        M.kmap.push_back({c, l, kind, off + pack_offset(I.lev[l].nx, I.lev[l].ny, kind)});
-      off += pack_offset(I.lev[l].nx, I.lev[l].ny, kNumPack);
+    for (int l = lf, off = 0; l < I.nlev; ++l) {
+      const int lx = I.lev[l].nx, ly = I.lev[l].ny;
+      if (l + 1 < I.nlev)
+        for (int kind = 0; kind < kNumPack; ++kind)
+          M.kmap.push_back({c, l, kind, off + pack_offset(lx, ly, kind)});
+      else if (!dense)
+        M.kmap.push_back({c, l, line_kind(ly), off});
+      off += (int)fused_pack(I.nlev, l, lx, ly);
     }
     for (int l = 0; l < I.nlev; ++l) {
       const int lx = I.lev[l].nx, ly = I.lev[l].ny, Nl = lx * ly;

@@ -123,15 +123,37 @@ __host__ __device__ inline size_t cell_slot(int i, int j, int nx) {
   return (size_t)j * nx + xslot(i, half_x(nx));
 }
 
-// band slots; level 0 uses the first five (the operator is 5-point), coarse
-// Galerkin levels use all nine.
-// The fused coarse cycle. The lanes of a sweep colour: a line of n cells is a
-// segment of W lanes (a power of two, at most 16), K steps each; lanes counts
-// whole waves.
+// The coarse end of a V-cycle runs in one workgroup per instance: the fused
+// coarse cycle, from the first level that fits (fused_fits) and has at most
+// fuse_cells cells. Sides of at most kFuseSide make lines of at most 16 lanes; a
+// 64 x 48 level costs the cycle 12 us more and saves some nine launches of 4 us.
+// Levels of at most kFuseLongCells cells may have sides of up to kFuseLong, lines of
+// up to a wave: with a launch per level strips of two cells by 65 to 130 took up to
+// 24% longer than fused, longer ones are no slower.
+constexpr int kFuseCells = 1024;     // default (any level that fits), and the
+                                     // largest other with FP64 V-cycles
+constexpr int kFuseCells32 = 4096;   // the largest with FP32 V-cycles
+constexpr int kFuseSide = 64, kFuseLong = 256, kFuseLongCells = 1024;
+constexpr int kFuseThreads = 512;
+__host__ __device__ constexpr bool fused_fits(int nx, int ny) {
+  const int side = nx > ny ? nx : ny;
+  return side <= kFuseSide || (side <= kFuseLong && nx * ny <= kFuseLongCells);
+}
+// Coarsening ends at the first level of at most kDense cells, which is solved by
+// the inverse of its operator (one wave's lanes are the rows).
+constexpr int kDense = 64;
+
+// The lanes of a sweep colour in the fused cycle: a line of n cells is a segment
+// of W = 1 << lw lanes, K steps each: one step while the line then has at most 16
+// lanes and the colour fits the workgroup, else four. lanes counts whole waves.
 struct LineLanes { int K, lw, nl, lanes; };
 __host__ __device__ constexpr LineLanes line_lanes(int n, int np, int colour) {
-  LineLanes a{n > 16 ? 4 : 1, 0, (np - colour + 1) >> 1, 0};
-  while ((a.K << a.lw) < n) ++a.lw;
+  LineLanes a{1, 0, (np - colour + 1) >> 1, 0};
+  while ((1 << a.lw) < n) ++a.lw;
+  if (a.lw > 4 || (a.nl << a.lw) > kFuseThreads) {
+    a.K = 4;
+    a.lw = a.lw > 2 ? a.lw - 2 : 0;
+  }
   a.lanes = ((a.nl << a.lw) + 63) & ~63;
   return a;
 }
@@ -172,6 +194,8 @@ struct CoarseTask {
 static_assert(sizeof(CoarseTask) == 64, "one scalar load");
 constexpr int kMaxTasks = 64;
 
+// band slots; level 0 uses the first five (the operator is 5-point), coarse
+// Galerkin levels use all nine.
 enum Band { BC = 0, BW = 1, BE = 2, BS = 3, BN = 4, BSW = 5, BSE = 6, BNW = 7, BNE = 8 };
 
 // Krylov vector slots (precision of the Krylov iteration).
@@ -272,22 +296,11 @@ struct Insts {
   __device__ __forceinline__ const InstDev &operator[](int k) const { return t[k]; }
 };
 struct PackMap { int inst, lev, kind, off; };   // off: of the kind's arrays in InstDev::pack
-struct FuseMap { int inst, lev, last, pad; };   // an instance whose levels lev .. last run fused
+// an instance whose levels lev .. last run fused; rows: some of its lines take more
+// than a row of 16 lanes
+struct FuseMap { int inst, lev, last, rows; };
 
-// The coarse end of a V-cycle runs in one workgroup per instance from the
-// first level with at most fuse_cells cells and no side above kFuseSide (a
-// line is then solved by the lanes of one wave): the fused coarse cycle.
-// The default cap takes every level with such sides: a 64 x 48 one costs the
-// cycle 12 us more and saves some nine launches of 4 us.
-constexpr int kFuseCells = 1024;     // default (any level that fits), and the
-                                     // largest other with FP64 V-cycles
-constexpr int kFuseCells32 = 4096;   // the largest with FP32 V-cycles
-constexpr int kFuseSide = 64;
-// Coarsening ends at the first level of at most kDense cells, which is solved by
-// the inverse of its operator (one wave's lanes are the rows).
-constexpr int kDense = 64;
 // Threads of the per-instance finish kernels (sums of the partials).
 constexpr int kFinThreads = 1024;
-constexpr int kFuseThreads = 512;
 
 }  // namespace sg

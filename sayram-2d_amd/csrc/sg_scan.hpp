@@ -40,6 +40,8 @@ __device__ __forceinline__ double rdlane(double v, int l) {
 
 // DPP controls: lane i takes lane i - n / i + n of its row of 16
 constexpr int kRowShr = 0x110, kRowShl = 0x100;
+// lane i takes lane i - 1 of the wave
+constexpr int kWaveShr1 = 0x138;
 
 // Inclusive scan inside the rows: (A, B) of a lane becomes the composition of
 // the maps of its row's (for W < 16: its segment's) lanes up to it, in order
@@ -135,6 +137,31 @@ template <bool FWD, typename T> __device__ __forceinline__ T scan_row0(T A, T B)
   B = A * dpp0<C | 2>(B) + B; A = A * dpp0<C | 2>(A);
   B = A * dpp0<C | 4>(B) + B; A = A * dpp0<C | 4>(A);
   return A * dpp0<C | 8>(B) + B;
+}
+
+// The value entering a lane's map from the lanes before it, for segments of one
+// row of 16 lanes (scan_row0), ...
+template <bool FWD, typename T> __device__ __forceinline__ T enter_row0(T A, T B) {
+  return dpp0<(FWD ? kRowShr : kRowShl) | 1>(scan_row0<FWD>(A, B));
+}
+// ... and of two or four rows: the rows are chained through v_readlane.
+template <bool FWD, typename T> __device__ __forceinline__ T enter_rows0(T A, T B) {
+  constexpr int C = FWD ? kRowShr : kRowShl;
+  B = A * dpp0<C | 1>(B) + B; A = A * dpp<C | 1>(T(1), A);
+  B = A * dpp0<C | 2>(B) + B; A = A * dpp<C | 2>(T(1), A);
+  B = A * dpp0<C | 4>(B) + B; A = A * dpp<C | 4>(T(1), A);
+  B = A * dpp0<C | 8>(B) + B; A = A * dpp<C | 8>(T(1), A);
+  const RowMaps<T> m = row_maps<FWD>(A, B);
+  const int row = (threadIdx.x >> 4) & 3;
+  T v = T(0), w = T(0);   // w enters the next row, v this lane's
+#pragma unroll
+  for (int k = 0; k < 3; ++k) {
+    const int r = FWD ? k : 3 - k;
+    w = m.a[r] * w + m.b[r];
+    v = row == (FWD ? k + 1 : 2 - k) ? w : v;
+  }
+  const T e = dpp0<C | 1>(A * v + B);
+  return (threadIdx.x & 15) == (FWD ? 0 : 15) ? v : e;
 }
 
 // smallest power of two >= n, at most 64

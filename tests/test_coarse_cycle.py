@@ -14,11 +14,19 @@ SHAPES = [(64, 64), (64, 63), (63, 64), (65, 64), (64, 65), (33, 31), (32, 32), 
           (1, 65), (70, 2), (128, 130)]
 
 
-def _run(precision, smoother, coarse, fuse, steps):
+# Long thin levels: lines of two and four rows of 16 lanes, sides and cells at and
+# past what is fused, columns whose lanes fit with four steps each only, last
+# levels that are a line of more than 64 cells, levels fused below others.
+LONG = [(66, 2), (2, 66), (65, 15), (15, 65), (70, 14), (113, 9), (9, 113), (128, 8), (8, 128), (129, 7),
+        (204, 5), (5, 204), (255, 3), (3, 255), (256, 4), (4, 256), (256, 2), (2, 256), (130, 2),
+        (2, 130), (257, 3), (3, 257), (256, 5), (512, 3), (3, 512), (150, 32), (32, 150), (520, 8), (9, 600)]
+
+
+def _run(precision, smoother, coarse, fuse, steps, shapes=SHAPES):
     b = sg.Batch(sg.make_opts(precision=precision, smoother=smoother, coarse_smoother=coarse,
                               fuse_cells=fuse))
     probs = [sc.seeded_case(nx, ny, seed=300 + k, scale=10.0 ** (k % 3 - 1))
-             for k, (nx, ny) in enumerate(SHAPES)]
+             for k, (nx, ny) in enumerate(shapes)]
     slots = [b.add(p) for p in probs]
     out, its = [], []
     for _ in range(steps):
@@ -74,3 +82,34 @@ def test_a_single_line_takes_line_solves(gpu_lib, shape, precision):
     n = _launches(sc.seeded_case(*shape, seed=7), precision)
     assert n["line_coarse"] > 0
     assert n["coarse_cycle"] == n["line_l0"] == n["restrict"] == n["prolong"] == 0
+
+
+# (schedules that smooth along both sides: x-lines alone take 100 iterations on a
+# strip along y, and the solve then ends wherever the stall rule takes it)
+@pytest.mark.gpu
+@pytest.mark.parametrize("precision", [sg.SG_FP64, sg.SG_MIXED, sg.SG_PC32])
+@pytest.mark.parametrize("smoother,coarse", [(0, 0), (13, 13), (12, 12), (9, 8)])
+def test_long_thin_levels(gpu_lib, precision, smoother, coarse):
+    """As test_edges_of_the_fused_cycle, for levels with a side above 64."""
+    probs, per_level, its0 = _run(precision, smoother, coarse, -1, 2, LONG)
+    _, fused, its = _run(precision, smoother, coarse, 0, 2, LONG)
+    for k, p in enumerate(probs):
+        f, op = p.f0, orc.OracleProblem(p)
+        for n in range(2):
+            f = orc.step(op, f)
+            assert rel_l2(fused[n][k], f) <= 1e-10, (LONG[k], n)
+            assert rel_l2(fused[n][k], per_level[n][k]) <= 1e-11, (LONG[k], n)
+            slack = 1 if precision != sg.SG_MIXED else 3
+            assert abs(its[n][k] - its0[n][k]) <= slack, (LONG[k], n, its[n][k], its0[n][k])
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("precision", [sg.SG_FP64, sg.SG_MIXED, sg.SG_PC32])
+@pytest.mark.parametrize("shape", [(66, 2), (2, 66), (130, 3), (130, 2), (2, 130), (256, 4), (4, 256),
+                                   (70, 14), (64, 64), (33, 2)])
+def test_one_launch_per_v_cycle(gpu_lib, shape, precision):
+    """Grids that fit run their whole V-cycle in the fused cycle: no launch per
+    level, whichever of the sides is the long one."""
+    n = _launches(sc.seeded_case(*shape, seed=7), precision)
+    assert n["coarse_cycle"] > 0
+    assert n["line_l0"] == n["line_coarse"] == n["restrict"] == n["prolong"] == 0
