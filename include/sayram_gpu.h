@@ -114,14 +114,14 @@ typedef struct {
                            levels (9-point operators); 0 selects the defaults
                            16, 160, 16, 768. */
   int fuse_cells;       /* the V-cycle levels of an instance from its first level
-                           of at most fuse_cells cells and sides of at most 64
-                           down run in one fused launch per instance (post-
-                           smoothing schedules, with or without an x-line
-                           pre-sweep). 0 or 1024 (default): any level with sides
-                           of at most 64; other values at most 1024 with FP64
-                           V-cycles, 4096 with FP32 ones; -1 disables. Like
-                           line_tiles it changes the rounding of those line
-                           solves. */
+                           that fits and has at most fuse_cells cells down run
+                           in one fused launch per instance (post-smoothing
+                           schedules, with or without an x-line pre-sweep). A
+                           level fits with sides of at most 64, or with at most
+                           1024 cells and sides of at most 256. 0 (default): any
+                           level that fits; 1 to 4096 (FP64 V-cycles: 1024): that
+                           many cells; -1 disables. Like line_tiles it changes
+                           the rounding of those line solves. */
   int streams;          /* 2: the tile shapes of one finest-level line sweep
                            run on two HIP streams (the longest lines beside the
                            rest; a coarser level's shapes share one launch in

@@ -588,7 +588,7 @@ void launch_coarse_cycle(hipStream_t s, const Insts &d, const FuseMap *m, int n,
                          int cap) {
   if (!n) return;
   if (cap <= 1024) k_coarse_cycle<T, 1024><<<n, kFuseThreads, 0, s>>>(d, m, xid, bid);
-  else k_coarse_cycle<T, kFuseCells32><<<n, kFuseThreads, 0, s>>>(d, m, xid, bid);
+  else k_coarse_cycle<T, kFuseCells><<<n, kFuseThreads, 0, s>>>(d, m, xid, bid);
 }
 template void launch_coarse_cycle<double>(hipStream_t, const Insts &, const FuseMap *, int, int,
                                           int, int);

@@ -395,7 +395,7 @@ struct Batch {
   int fuse_level(const InstDev &I) const;
   Insts insts() const { return {d_insts, d_stat}; }
   // largest fused level: the default takes any that fits
-  int fuse_cap() const { return opts.fuse_cells == kFuseCells ? kFuseCells32 : opts.fuse_cells; }
+  int fuse_cap() const { return opts.fuse_cells == 0 ? kFuseCells : opts.fuse_cells; }
   int step(int nsteps, const int64_t *targets, int ntargets);
   int step_once();
   bool graphs_on() const { return opts.use_graph >= 0 && time_mask == 0; }
@@ -459,7 +459,6 @@ static void apply_defaults(sg_opts &o) {
   const bool sm_default = o.smoother <= 0 || o.smoother > 15;
   if (sm_default) o.smoother = 12;
   if (o.coarse_smoother == 0) o.coarse_smoother = sm_default ? 13 : o.smoother;
-  if (o.fuse_cells == 0) o.fuse_cells = kFuseCells;
   if (o.streams == 0) o.streams = 1;
   if (o.group_cells == 0) o.group_cells = 1 << 21;
   if (o.warm_start == 0) o.warm_start = 1;
@@ -474,12 +473,12 @@ int Batch::init(const sg_opts *o, size_t b) {
   if (opts.precision != SG_FP64 && opts.precision != SG_MIXED && opts.precision != SG_PC32)
     return fail(SG_ERR_ARG, "opts.precision must be SG_FP64, SG_MIXED or SG_PC32");
   apply_defaults(opts);
-  if (opts.fuse_cells > (opts.precision == SG_FP64 ? kFuseCells : kFuseCells32))
+  if (opts.fuse_cells > (opts.precision == SG_FP64 ? kFuseLimit64 : kFuseCells))
     return fail(SG_ERR_ARG, opts.precision == SG_FP64
-                                ? "opts.fuse_cells must be at most 1024 with FP64 V-cycles (the fused "
-                                  "cycle keeps a level in LDS)"
-                                : "opts.fuse_cells must be at most 4096 (the fused cycle keeps a level "
-                                  "in LDS)");
+                                ? "opts.fuse_cells must be at most 1024 with FP64 V-cycles (0: no "
+                                  "limit below the largest level that fits)"
+                                : "opts.fuse_cells must be at most 4096, the largest level that fits "
+                                  "the fused cycle");
   if (opts.streams != 1 && opts.streams != 2) return fail(SG_ERR_ARG, "opts.streams must be 0, 1 or 2");
   if (opts.warm_start < -1 || opts.warm_start > 1)
     return fail(SG_ERR_ARG, "opts.warm_start must be -1, 0 or 1");

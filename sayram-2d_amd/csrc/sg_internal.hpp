@@ -130,9 +130,8 @@ __host__ __device__ inline size_t cell_slot(int i, int j, int nx) {
 // Levels of at most kFuseLongCells cells may have sides of up to kFuseLong, lines of
 // up to a wave: with a launch per level strips of two cells by 65 to 130 took up to
 // 24% longer than fused, longer ones are no slower.
-constexpr int kFuseCells = 1024;     // default (any level that fits), and the
-                                     // largest other with FP64 V-cycles
-constexpr int kFuseCells32 = 4096;   // the largest with FP32 V-cycles
+constexpr int kFuseCells = 4096;     // the largest level that fits (the default takes any)
+constexpr int kFuseLimit64 = 1024;   // the largest limit FP64 V-cycles accept
 constexpr int kFuseSide = 64, kFuseLong = 256, kFuseLongCells = 1024;
 constexpr int kFuseThreads = 512;
 __host__ __device__ constexpr bool fused_fits(int nx, int ny) {

@@ -17,9 +17,9 @@ that select how the step is launched, and returns the fastest set:
 * ``streams``: the tile shapes of a sweep on two HIP streams (2) or one (1).
 * ``group_cells``: the size from which instances are stepped as a second
   group, concurrently with the rest (-1: one group).
-* ``fuse_cells``: the size below which an instance's coarse levels run in the
-  fused one-workgroup cycle (-1: never; 1024, the default: any level with sides
-  of at most 64; above 1024 only with an FP32 V-cycle).
+* ``fuse_cells``: the size up to which an instance's coarse levels run in the
+  fused one-workgroup cycle (-1: never; 0, the default: any level that fits;
+  above 1024 only with an FP32 V-cycle).
 
 ``check_every``, ``use_graph``, ``streams`` and ``group_cells`` never change results: every
 instance's result is bit-identical for all their values. ``line_tiles``,
@@ -40,7 +40,7 @@ import sayram_gpu as sg
 
 DEFAULTS = {"check_every": 1, "use_graph": 1, "row_short": 16, "row_mid": 160,
             "col_short": 16, "col_mid": 768, "crow_mid": 160, "ccol_mid": 768, "streams": 1,
-            "fuse_cells": 1024, "group_cells": 1 << 21}
+            "fuse_cells": 0, "group_cells": 1 << 21}
 
 CANDIDATES = {
     "check_every": [1, 2, 3, 4],
@@ -52,7 +52,7 @@ CANDIDATES = {
     "crow_mid": [96, 160, 256],
     "ccol_mid": [128, 256, 768],
     "streams": [1, 2],
-    "fuse_cells": [-1, 256, 1024, 2048, 4096],
+    "fuse_cells": [-1, 256, 1024, 2048, 0],
     "group_cells": [-1, 1 << 18, 1 << 21],
 }
 
@@ -62,7 +62,7 @@ def opts_for(precision: int, p: dict):
                         line_tiles=(p["row_short"], p["row_mid"], p["col_short"], p["col_mid"]),
                         coarse_tiles=(p["row_short"], p.get("crow_mid", 160), p["col_short"],
                                       p.get("ccol_mid", 768)),
-                        streams=p.get("streams", 1), fuse_cells=p.get("fuse_cells", 1024),
+                        streams=p.get("streams", 1), fuse_cells=p.get("fuse_cells", 0),
                         group_cells=p.get("group_cells", 1 << 21))
 
 

@@ -45,7 +45,9 @@ def test_edges_of_the_fused_cycle(gpu_lib, precision, smoother, coarse):
     per-level cycle up to the solve tolerance, and as strong: the two cycles
     are the same operator up to rounding, so they need the same iterations up
     to one."""
-    caps = [0] if precision == sg.SG_FP64 else [0, 4096]
+    # limits that fuse from level 0 of other shapes (above 1024 cells with FP32
+    # V-cycles only; they have a kernel with larger LDS arrays)
+    caps = [0, 1024, 256] if precision == sg.SG_FP64 else [0, 2048, 1024, 256]
     probs, per_level, its0 = _run(precision, smoother, coarse, -1, 3)
     for cap in caps:
         _, fused, its = _run(precision, smoother, coarse, cap, 3)
@@ -101,6 +103,23 @@ def test_long_thin_levels(gpu_lib, precision, smoother, coarse):
             assert rel_l2(fused[n][k], per_level[n][k]) <= 1e-11, (LONG[k], n)
             slack = 1 if precision != sg.SG_MIXED else 3
             assert abs(its[n][k] - its0[n][k]) <= slack, (LONG[k], n, its[n][k], its0[n][k])
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("precision,shape,limit,fused", [
+    (sg.SG_FP64, (64, 48), 0, True), (sg.SG_FP64, (64, 48), 1024, False),
+    (sg.SG_FP64, (45, 22), 990, True), (sg.SG_FP64, (45, 22), 989, False),
+    (sg.SG_FP64, (32, 32), 1023, False), (sg.SG_FP64, (32, 32), 1024, True),
+    (sg.SG_FP64, (33, 32), 1024, False), (sg.SG_FP64, (33, 32), 0, True),
+    (sg.SG_PC32, (64, 48), 0, True), (sg.SG_PC32, (64, 48), 4096, True),
+    (sg.SG_PC32, (64, 48), 3071, False), (sg.SG_PC32, (64, 48), 2048, False),
+    (sg.SG_MIXED, (64, 48), 1024, False), (sg.SG_MIXED, (64, 64), 4095, False),
+    (sg.SG_MIXED, (64, 64), 4096, True), (sg.SG_PC32, (8, 9), 1, False)])
+def test_fuse_cells_is_the_largest_fused_level(gpu_lib, precision, shape, limit, fused):
+    """Every limit means itself: a grid is fused from level 0, with no launch for
+    its own lines, exactly if it has at most that many cells (0: any that fits)."""
+    n = _launches(sc.seeded_case(*shape, seed=7), precision, fuse_cells=limit)
+    assert n["coarse_cycle"] > 0 and (n["line_l0"] == 0) == fused
 
 
 @pytest.mark.gpu

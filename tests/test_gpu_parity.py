@@ -126,10 +126,10 @@ def test_fused_coarse_cycle_matches_per_level_cycle(gpu_lib, precision):
     Shapes cover fusion from level 0 (small grids), from a coarse level, and
     a batch mixing the two."""
     probs = [sc.seeded_case(nx, ny, seed=90 + k, scale=s) for k, (nx, ny, s) in
-             enumerate([(24, 20, 2.0), (70, 45, 0.5), (33, 130, 5.0)])]
+             enumerate([(24, 20, 2.0), (70, 45, 0.5), (33, 130, 5.0), (64, 48, 1.0)])]
     out = {}
-    # FP32 V-cycles also keep levels of up to 2048 and 4096 cells in LDS
-    # (other LDS layouts of the fused kernel)
+    # Limits above 1024 cells (FP32 V-cycles) take a kernel with larger LDS
+    # arrays; the 64 x 48 grid is fused from level 0 with 4096, not with 2048.
     fcs = (0, -1, 300) if precision == 0 else (0, -1, 300, 2048, 4096)
     for fc in fcs:
         b = gpu_lib.Batch(gpu_lib.make_opts(precision=precision, fuse_cells=fc))
