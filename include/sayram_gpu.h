@@ -266,6 +266,9 @@ void sg_batch_destroy(sg_batch *b);
 /* Assembly only: writes the 5 FP64 bands (d|w|e|s|n, K = j*nx+i order) and R
  * of the next step into host buffers, for parity checks of the assembly. */
 int sg_debug_assemble(sg_solver *h, double *bands5, double *R);
+/* Fills every array of an instance that a step writes before it reads with NaN:
+ * a step must not depend on what the memory held. */
+int sg_debug_poison(sg_batch *b, int slot);
 /* The multigrid's dense last level alone: the inverse (row-major, N x N, N =
  * nx ny <= 64, as stored for the V-cycle of that precision) of the 9-point
  * operator of bands d|w|e|s|n|sw|se|nw|ne, K = j*nx+i order. */

@@ -416,6 +416,7 @@ struct Batch {
   int get_f(int slot, double *out);
   int get_f_static(int slot, double *out, double *buf);
   int set_f(int slot, const double *f, int64_t istep);
+  int debug_poison(int slot);
   int debug_assemble(int slot, double *bands, double *R);
   // timing helpers
   void tbegin(int id, hipStream_t s = nullptr);
@@ -1620,6 +1621,22 @@ int Batch::set_f(int slot, const double *f, int64_t istep) {
   return SG_OK;
 }
 
+// NaN into every array of an instance that a step writes before it reads: all
+// of its slab but the inputs, f and df, the geometry and the task table (carve).
+int Batch::debug_poison(int slot) {
+  if (slot < 0 || slot >= (int)slots.size() || !slots[slot].used)
+    return fail(SG_ERR_ARG, "no instance in slot " + std::to_string(slot));
+  const Slot &s = slots[slot];
+  const InstDev &I = s.dev;
+  char *const rest = (char *)I.tasks + kMaxTasks * sizeof(CoarseTask);
+  const std::pair<char *, char *> parts[] = {{(char *)I.R, (char *)I.df},
+                                             {(char *)I.partial, (char *)I.tasks},
+                                             {rest, (char *)s.slab + s.bytes}};
+  for (auto &p : parts) HIPCHK(hipMemsetAsync(p.first, 0xff, p.second - p.first, stream));
+  HIPCHK(hipStreamSynchronize(stream));
+  return SG_OK;
+}
+
 int Batch::debug_assemble(int slot, double *bands, double *R) {
   if (slot < 0 || slot >= (int)slots.size() || !slots[slot].used)
     return fail(SG_ERR_ARG, "no instance in slot " + std::to_string(slot));
@@ -2123,6 +2140,14 @@ int sg_debug_assemble(sg_solver *h, double *bands5, double *R) {
   Batch *G = h->bt->group_of(h->slot, &local);
   if (!G) return fail(SG_ERR_ARG, "no instance");
   return G->debug_assemble(local, bands5, R);
+}
+int sg_debug_poison(sg_batch *b, int slot) {
+  if (!b) return fail(SG_ERR_ARG, "null batch");
+  sg::HostLock lk(sg::g_capture_mu);
+  int local;
+  Batch *G = b->group_of(slot, &local);
+  if (!G) return fail(SG_ERR_ARG, "no instance in slot " + std::to_string(slot));
+  return G->debug_poison(local);
 }
 int sg_solver_batch(sg_solver *h, sg_batch **out) {
   if (!h || !out) return fail(SG_ERR_ARG, "null argument");

@@ -90,6 +90,7 @@ SYMBOLS = [
     ("sg_batch_bytes_in_use", _S, [_V]),
     ("sg_batch_destroy", None, [_V]),
     ("sg_debug_assemble", C.c_int, [_V, _dp, _dp]),
+    ("sg_debug_poison", C.c_int, [_V, C.c_int]),
     ("sg_debug_dense_inverse", C.c_int, [C.c_int, C.c_int, C.c_int, _dp, _dp]),
     ("sg_batch_time_kernel", C.c_int, [_V, C.c_int]),
     ("sg_batch_kernel_time", C.c_int, [_V, C.POINTER(C.c_double), C.POINTER(C.c_int64),
@@ -346,6 +347,10 @@ class Batch:
 
     def bytes_in_use(self):
         return int(lib().sg_batch_bytes_in_use(self.h))
+
+    def debug_poison(self, slot):
+        """NaN into every array that a step writes before it reads."""
+        _check(lib().sg_debug_poison(self.h, int(slot)))
 
     def time_kernel(self, name):
         """Times every dispatch of one kernel family ("all": every family; None: off)."""
