@@ -1451,11 +1451,12 @@ void Batch::count_bytes(const std::vector<int> &part) {
         t_bytes[4] += vc * (3.0 * T * Nl + T * Nc);
       } else {
         // after an x-line pre-sweep: the even rows' residual formed inside
-        // the restriction (the couplings to the odd rows, 2 or 6, and 2 stored
-        // weights per even-row cell, x of the odd rows in; b out); otherwise the residual of every cell (b, the bands, x; r
-        // out) and its restriction (r and 2 weights per cell in; b out)
+        // the restriction (per even-row cell 2 or 6 couplings to the odd rows,
+        // x of an odd row and one stored weight, two at odd columns, in; b
+        // out); otherwise the residual of every cell (b, the bands, x; r out)
+        // and its restriction (r and 2 weights per cell in; b out)
         if (half_residual(sml))
-          t_bytes[4] += vc * (0.5 * Nl * (nb == 9.0 ? 9.0 : 5.0) * T + T * Nc);
+          t_bytes[4] += vc * (0.5 * Nl * (nb == 9.0 ? 8.0 : 4.0) * T + T * Nc);
         else
           t_bytes[4] += vc * (Nl * (nb + 3.0) * T + 3.0 * T * Nl + T * Nc);
       }

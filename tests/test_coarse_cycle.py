@@ -132,3 +132,25 @@ def test_one_launch_per_v_cycle(gpu_lib, shape, precision):
     n = _launches(sc.seeded_case(*shape, seed=7), precision)
     assert n["coarse_cycle"] > 0
     assert n["line_l0"] == n["line_coarse"] == n["restrict"] == n["prolong"] == 0
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("precision,size", [(sg.SG_FP64, 8), (sg.SG_PC32, 4)])
+def test_bytes_of_the_restrictions(gpu_lib, precision, size):
+    """The byte model of the restrictions, per V-cycle: from level 0 b and two
+    weights per cell; below, after the x-line pre-sweep, six couplings, one x and
+    one weight per even-row cell (its odd columns read two weights); and the
+    coarse right-hand side."""
+    b = sg.Batch(sg.make_opts(precision=precision, fuse_cells=-1))
+    b.add(sc.seeded_case(256, 128, seed=3))
+    b.time_kernel("all")
+    b.step(1)
+    n0, levels = 256 * 128, 5   # 256 x 128, .., 16 x 8 (dense: 8 x 4)
+    per_cycle = size * (3 * n0 + n0 / 4)
+    per_cycle += sum(size * (8 * n / 2 + n / 4) for n in (n0 / 4 ** l for l in range(1, levels)))
+    _, launches, nbytes = b.kernel_time("restrict")
+    # V-cycles that ran (those launched after convergence exit and move nothing)
+    cycles = nbytes / per_cycle
+    assert launches % levels == 0 and 1 <= round(cycles) <= launches // levels
+    assert abs(cycles - round(cycles)) < 1e-9, cycles
+    b.close()
