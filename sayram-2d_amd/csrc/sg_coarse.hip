@@ -77,9 +77,9 @@ __global__ void __launch_bounds__(1024) k_dense_inverse(const Insts insts,
   __shared__ unsigned s_key[2][16];
   __shared__ int s_at[kDense], s_of[kDense];   // pivot row of a column, column of a pivot row
   __shared__ int s_bad;
-  const InstDev &I = insts[map[blockIdx.x].inst];
+  CInst &I = insts[map[blockIdx.x].inst];
   if (ostatus_of(insts, map[blockIdx.x].inst) == ST_IDLE) return;
-  const Lev &L = I.lev[I.nlev - 1];
+  CLev &L = I.lev[I.nlev - 1];
   const int nx = L.nx, ny = L.ny, n = nx * ny, hx = half_x(nx);
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const bool nine = I.nlev > 1;
@@ -187,9 +187,9 @@ template <typename T>
 __global__ void __launch_bounds__(kFuseThreads) k_coarse_pack(const Insts insts,
                                                               const PackMap *__restrict__ map) {
   const PackMap pm = map[blockIdx.x];
-  const InstDev &I = insts[pm.inst];
+  CInst &I = insts[pm.inst];
   if (ostatus_of(insts, pm.inst) == ST_IDLE) return;
-  const Lev &L = I.lev[pm.lev];
+  CLev &L = I.lev[pm.lev];
   const int nx = L.nx, ny = L.ny, hx = half_x(nx), kind = pm.kind;
   const LineLanes g = pack_lanes(nx, ny, kind);
   const bool col = kind == PK_COL0 || kind == PK_COL1, nine = pm.lev > 0;
@@ -314,7 +314,7 @@ template <typename T> struct CycleIn {
 // places of x; sp: partial products of the dense level. ROWS: the instance has
 // lines longer than a row of lanes.
 template <typename T, int XN, bool ROWS>
-__device__ __forceinline__ void coarse_cycle(const InstDev &I, const CycleIn<T> &C, T *const sx,
+__device__ __forceinline__ void coarse_cycle(CInst &I, const CycleIn<T> &C, T *const sx,
                                              T *const sb, T *const sp) {
   constexpr int NW = kFuseThreads / 64, DC = kDense / NW;
   const CoarseTask *const tasks = C.tasks;
@@ -480,7 +480,7 @@ __device__ __forceinline__ void coarse_cycle(const InstDev &I, const CycleIn<T> 
       if (t.K == 4) second(std::integral_constant<int, 4>(), t);
       else second(std::integral_constant<int, 1>(), t);
     } else if (t.lanes == 0) {
-      const Lev &L = I.lev[t.lev];
+      CLev &L = I.lev[t.lev];
       const int nx = L.nx, ny = L.ny, hx = half_x(nx);
       if (t.kind == TK_DENSE) {
         T s = T(0);
@@ -555,7 +555,7 @@ __global__ void __launch_bounds__(kFuseThreads) k_coarse_cycle(const Insts insts
   __shared__ T sb[kDense + XN];
   __shared__ T sp[kFuseThreads / 64 * kDense];
   const FuseMap fm = map[blockIdx.x];
-  const InstDev &I = insts[fm.inst];
+  CInst &I = insts[fm.inst];
   CycleIn<T> C;
   C.tasks = I.tasks;
   C.pack = cptr<T>(I.pack);

@@ -56,7 +56,7 @@ template <typename T> __device__ __forceinline__ const T *cptr(const void *p) {
 // space the compiler reads these workgroup-uniform values with scalar loads
 // instead of per-lane loads that every later load waits behind.
 typedef const __attribute__((address_space(4))) KScal ConstKScal;
-__device__ __forceinline__ ConstKScal *rsc(const InstDev &I) { return (ConstKScal *)I.sc; }
+__device__ __forceinline__ ConstKScal *rsc(CInst &I) { return (ConstKScal *)I.sc; }
 
 __device__ __forceinline__ int status_of(const Insts &insts, int k) {
   return ((const __attribute__((address_space(4))) InstStat *)insts.st)[k].status;
@@ -78,12 +78,12 @@ template <typename P> __device__ __forceinline__ void pin1(P &p) { asm volatile(
 template <typename... P> __device__ __forceinline__ void pin(P &...p) { (pin1(p), ...); }
 
 // level-0 vector by id: a Krylov slot (Vec) or an FP32 V-cycle vector (PcVec)
-__device__ __forceinline__ void *vec(const InstDev &I, int id) {
+__device__ __forceinline__ void *vec(CInst &I, int id) {
   return id < kNumVec ? I.kv[id] : (void *)I.pv[id - kNumVec];
 }
 
 template <typename T>
-__device__ __forceinline__ void level_xb(const InstDev &I, int l, int xid, int bid, T *&x,
+__device__ __forceinline__ void level_xb(CInst &I, int l, int xid, int bid, T *&x,
                                          const T *&b) {
   if (l == 0) { x = ptr<T>(vec(I, xid)); b = cptr<T>(vec(I, bid)); }
   else { x = ptr<T>(I.lev[l].x); b = cptr<T>(I.lev[l].b); }

@@ -288,11 +288,15 @@ struct FacGrp { int inst, first, count, step, lev, dir, shape, pad; };
 // it (KScal::status and ostatus by compact index, mirrored by the kernels that
 // change them): a workgroup reads its status and its instance's pointers in
 // the same round trip instead of following the table to the scalars first.
+// No kernel writes the table, so it is read through the constant address space: by
+// scalar loads, also after a kernel's own stores, and free to be issued before them.
 struct InstStat { int status, ostatus, phase, pad; };
+typedef const __attribute__((address_space(4))) InstDev CInst;
+typedef const __attribute__((address_space(4))) Lev CLev;
 struct Insts {
   const InstDev *t;
   InstStat *st;
-  __device__ __forceinline__ const InstDev &operator[](int k) const { return t[k]; }
+  __device__ __forceinline__ CInst &operator[](int k) const { return ((CInst *)t)[k]; }
 };
 struct PackMap { int inst, lev, kind, off; };   // off: of the kind's arrays in InstDev::pack
 // an instance whose levels lev .. last run fused; rows: some of its lines take more

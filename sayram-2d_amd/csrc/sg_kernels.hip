@@ -64,7 +64,7 @@ __device__ __forceinline__ void block_sum(A (&v)[NV]) {
 
 // partial sums of a workgroup (NV values) into slot lblk of the instance
 template <typename A, int NV>
-__device__ __forceinline__ void store_partials(const InstDev &I, int lblk, A (&v)[NV]) {
+__device__ __forceinline__ void store_partials(CInst &I, int lblk, A (&v)[NV]) {
   block_sum<A, NV>(v);
   if (threadIdx.x == 0) {
 #pragma unroll
@@ -115,7 +115,7 @@ __global__ void k_copy_counter(const int *__restrict__ src, int *__restrict__ ds
 // and wxL/wxR = wx0/wx1[vi], wyB/wyT = wy0/wy1[vj]. Dirichlet sides were
 // written in the order XMIN, XMAX, YMIN, YMAX there, so the precedence here
 // is the reverse.
-__device__ __forceinline__ double vertex_value(const InstDev &I, int vi, int vj, double fSW,
+__device__ __forceinline__ double vertex_value(CInst &I, int vi, int vj, double fSW,
                                                double fSE, double fNW, double fNE, double wxL,
                                                double wxR, double wyB, double wyT) {
 #pragma clang fp contract(off)
@@ -247,7 +247,7 @@ __global__ void __launch_bounds__(kBlock) k_assemble(const Insts insts,
                                                     const BlkMap *__restrict__ map) {
 #pragma clang fp contract(off)
   const BlkMap m = map[blockIdx.x];
-  const InstDev &I = insts[m.inst];
+  CInst &I = insts[m.inst];
   if (ostatus_of(insts, m.inst) == ST_IDLE) return;
   const int nx = I.nx, ny = I.ny;
   const int K = m.k0 + threadIdx.x;
@@ -341,7 +341,7 @@ __global__ void __launch_bounds__(kBlock) k_assemble(const Insts insts,
     I.band64[BS][K] = bs;
     I.band64[BN][K] = bn;
     if (I.prec != SG_FP64) {   // FP32 copies for the FP32 V-cycle and Krylov forms
-      const Lev &L0 = I.lev[0];
+      CLev &L0 = I.lev[0];
       ptr<float>(L0.band[BC])[K] = (float)d;
       ptr<float>(L0.band[BW])[K] = (float)bw;
       ptr<float>(L0.band[BE])[K] = (float)be;
@@ -390,7 +390,7 @@ __global__ void __launch_bounds__(kBlock) k_assemble(const Insts insts,
 struct St9 { double c, w, e, s, n, sw, se, nw, ne; };
 
 template <int NB>
-__device__ __forceinline__ St9 load_st(const Lev &L, size_t K) {
+__device__ __forceinline__ St9 load_st(CLev &L, size_t K) {
   St9 a;
   a.c = L.band64[BC][K]; a.w = L.band64[BW][K]; a.e = L.band64[BE][K];
   a.s = L.band64[BS][K]; a.n = L.band64[BN][K];
@@ -410,7 +410,7 @@ __device__ __forceinline__ double safe_den(double d, double c) {
 // x-edge point (i odd, j even): interpolate from west/east coarse points with
 // the stencil collapsed along y.
 template <int NB>
-__device__ __forceinline__ void w_xedge(const Lev &L, size_t K, int i, double &wW, double &wE) {
+__device__ __forceinline__ void w_xedge(CLev &L, size_t K, int i, double &wW, double &wE) {
   const St9 a = load_st<NB>(L, K);
   const double den = safe_den(a.c + a.n + a.s, a.c);
   wW = -(a.w + a.nw + a.sw) / den;
@@ -419,7 +419,7 @@ __device__ __forceinline__ void w_xedge(const Lev &L, size_t K, int i, double &w
 
 // y-edge point (i even, j odd): from south/north, stencil collapsed along x.
 template <int NB>
-__device__ __forceinline__ void w_yedge(const Lev &L, size_t K, int j, double &wS, double &wN) {
+__device__ __forceinline__ void w_yedge(CLev &L, size_t K, int j, double &wS, double &wN) {
   const St9 a = load_st<NB>(L, K);
   const double den = safe_den(a.c + a.w + a.e, a.c);
   wS = -(a.s + a.sw + a.se) / den;
@@ -430,9 +430,9 @@ template <typename T, int NB>
 __global__ void __launch_bounds__(kBlock) k_pweights(const Insts insts,
                                                     const BlkMap *__restrict__ map, int l) {
   const BlkMap m = map[blockIdx.x];
-  const InstDev &I = insts[m.inst];
+  CInst &I = insts[m.inst];
   if (ostatus_of(insts, m.inst) == ST_IDLE) return;
-  const Lev &L = I.lev[l];
+  CLev &L = I.lev[l];
   const int nx = L.nx, ny = L.ny;
   const int K = m.k0 + threadIdx.x;
   if (K >= nx * ny) return;
@@ -490,7 +490,7 @@ __global__ void __launch_bounds__(kBlock) k_pweights(const Insts insts,
 // (against a branch per point: 20 steps of 90 x 100 FP64 16.0 -> 15.1 ms, 10 of
 // 1021 x 765 PC32 41.1 -> 40.2, of 4096 x 4096 PC32 242.6 -> 240.5).
 template <typename T, int NB>
-__device__ __forceinline__ void rap_row(const Lev &F, const T *const (&pw)[4], int Ic, int J,
+__device__ __forceinline__ void rap_row(CLev &F, const T *const (&pw)[4], int Ic, int J,
                                         int fb, int hxf, double (&acc)[3][3]) {
 #pragma clang fp contract(off)
   constexpr int di_[9] = {0, -1, 1, 0, 0, -1, 1, -1, 1};
@@ -567,10 +567,10 @@ template <typename T, int NB, bool COPY>
 __global__ void __launch_bounds__(kBlock) k_rap(const Insts insts,
                                                const BlkMap *__restrict__ map, int l) {
   const BlkMap m = map[blockIdx.x];
-  const InstDev &I = insts[m.inst];
+  CInst &I = insts[m.inst];
   if (ostatus_of(insts, m.inst) == ST_IDLE) return;
-  const Lev &F = I.lev[l];
-  const Lev &Cl = I.lev[l + 1];
+  CLev &F = I.lev[l];
+  CLev &Cl = I.lev[l + 1];
   const int cx = Cl.nx, cy = Cl.ny, fx = F.nx;
   const int KN = m.k0 + threadIdx.x;
   if (KN >= cx * cy) return;
@@ -613,7 +613,7 @@ constexpr int factor_lds(int sh) {
   return 3 * tile_lines(sh) * (tile_steps(sh) + 4) + tile_lines(sh);
 }
 template <typename T, int DIR, int SH>
-__device__ __forceinline__ void line_factor(const InstDev &I, const FacGrp &gr, double *lds) {
+__device__ __forceinline__ void line_factor(CInst &I, const FacGrp &gr, double *lds) {
   constexpr int S = tile_steps(SH), L = tile_lines(SH), NT = tile_threads(SH);
   constexpr int W = NT / L;          // threads per line in the solve, 4 steps each
   constexpr int Q = S * L / NT;      // elements per thread in the loads
@@ -622,7 +622,7 @@ __device__ __forceinline__ void line_factor(const InstDev &I, const FacGrp &gr, 
   double *const s_d = s_lo + L * (S + 4);
   double *const s_up = s_d + L * (S + 4);
   double *const s_c = s_up + L * (S + 4);
-  const Lev &Lv = I.lev[gr.lev];
+  CLev &Lv = I.lev[gr.lev];
   const int nx = Lv.nx, ny = Lv.ny;
   const double *__restrict__ bc = Lv.band64[BC];
   const double *__restrict__ lo = Lv.band64[DIR == 0 ? BW : BS];
@@ -755,7 +755,7 @@ __global__ void __launch_bounds__(SH3 ? 1024 : 256) k_line_factor(const Insts in
   constexpr int E24 = factor_lds(2) > factor_lds(4) ? factor_lds(2) : factor_lds(4);
   __shared__ double lds[SH3 ? factor_lds(3) : E01 > E24 ? E01 : E24];
   const FacGrp gr = map[blockIdx.x];
-  const InstDev &I = insts[gr.inst];
+  CInst &I = insts[gr.inst];
   if (ostatus_of(insts, gr.inst) == ST_IDLE) return;
   if constexpr (SH3) {
     if (gr.dir == 0) line_factor<T, 0, 3>(I, gr, lds);
@@ -817,9 +817,9 @@ __device__ __forceinline__ void line_sweep(const Insts insts, const LineGrp gr,
   T *const s_a = s_rb + KT * TB;
   T *const s_i = s_a + TB;
   T *const s_c = s_i + TB;         // L values
-  const InstDev &I = insts[gr.inst];
+  CInst &I = insts[gr.inst];
   if (status_of(insts, gr.inst) != ST_ACTIVE) return;
-  const Lev &Lv = I.lev[l];
+  CLev &Lv = I.lev[l];
   const int nx = Lv.nx, ny = Lv.ny;
   T *x; const T *b;
   level_xb<T>(I, l, xid, bid, x, b);
@@ -1065,7 +1065,7 @@ k_line_shapes(const Insts insts,
 template <typename T, int NB> struct Sten {
   const T *b[NB];
   int nx, ny;
-  __device__ __forceinline__ Sten(const Lev &L) {
+  __device__ __forceinline__ Sten(CLev &L) {
 #pragma unroll
     for (int k = 0; k < NB; ++k) b[k] = cptr<T>(L.band[k]);
     nx = L.nx; ny = L.ny;
@@ -1121,7 +1121,7 @@ __device__ __forceinline__ T stencil_apply(const Sten<T, NB> &L, size_t K, int i
 struct Sten64 {
   const double *b[5];
   int nx, ny;
-  __device__ __forceinline__ Sten64(const InstDev &I) {
+  __device__ __forceinline__ Sten64(CInst &I) {
 #pragma unroll
     for (int k = 0; k < 5; ++k) b[k] = I.band64[k];
     nx = I.nx; ny = I.ny;
@@ -1161,7 +1161,7 @@ __global__ void __launch_bounds__(kBlock) k_residual(const Insts insts,
                                                     const BlkMap *__restrict__ map, int l,
                                                     int xid, int bid) {
   const BlkMap m = map[blockIdx.x];
-  const InstDev &I = insts[m.inst];
+  CInst &I = insts[m.inst];
   Sten<T, NB> F(I.lev[l]);
   T *x; const T *b;
   level_xb<T>(I, l, xid, bid, x, b);
@@ -1189,7 +1189,7 @@ __global__ void __launch_bounds__(kBlock) k_restrict(const Insts insts,
                                                     const BlkMap *__restrict__ map, int l,
                                                     int xid, int bid) {
   const BlkMap m = map[blockIdx.x];
-  const InstDev &I = insts[m.inst];
+  CInst &I = insts[m.inst];
   T *x; const T *b;
   level_xb<T>(I, l, xid, bid, x, b);
   const T *rp = FROM_B ? b : cptr<T>(I.lev[l].cp);
@@ -1250,8 +1250,8 @@ __global__ void __launch_bounds__(kBlock) k_restrict_residual(const Insts insts,
                                                              const BlkMap *__restrict__ map, int l,
                                                              int xid, int bid) {
   const BlkMap m = map[blockIdx.x];
-  const InstDev &I = insts[m.inst];
-  const Lev &F = I.lev[l];
+  CInst &I = insts[m.inst];
+  CLev &F = I.lev[l];
   T *xp; const T *bp;
   level_xb<T>(I, l, xid, bid, xp, bp);
   const T *s0 = cptr<T>(F.band[BS]), *n0 = cptr<T>(F.band[BN]);
@@ -1343,8 +1343,8 @@ __global__ void __launch_bounds__(kBlock) k_prolong(const Insts insts,
   for (int e = 0; e < kEnt; ++e) m[e] = map[min((int)(kEnt * blockIdx.x) + e, nmap - 1)];
 #pragma unroll
   for (int e = 0; e < kEnt; ++e) {
-    const InstDev &I = insts[m[e].inst];
-    const Lev &F = I.lev[l], &Cl = I.lev[l + 1];
+    CInst &I = insts[m[e].inst];
+    CLev &F = I.lev[l], &Cl = I.lev[l + 1];
     E[e] = {cptr<T>(F.pw[0]), cptr<T>(F.pw[1]), cptr<T>(F.pw[2]), cptr<T>(F.pw[3]), cptr<T>(Cl.x),
             l == 0 ? ptr<T>(vec(I, xid)) : ptr<T>(F.x), F.nx, F.ny, Cl.nx, Cl.ny,
             status_of(insts, m[e].inst), m[e].k0};
@@ -1451,7 +1451,7 @@ __global__ void __launch_bounds__(kBlock) k_bicg_p(const Insts insts,
     const int bi = kLightBlocks * blockIdx.x + e;
     if (bi >= nmap) break;
     const BlkMap m = map[bi];
-    const InstDev &I = insts[m.inst];
+    CInst &I = insts[m.inst];
     if (status_of(insts, m.inst) != ST_ACTIVE) continue;
     const int K = m.k0 + threadIdx.x;
     if (K >= I.nx * I.ny) continue;
@@ -1485,7 +1485,7 @@ __device__ __forceinline__ T krylov_spmv(const M &A, double pcs, int K, const X 
 template <typename T, bool PC> struct KrylovOp { using type = Sten<T, 5>; };
 template <typename T> struct KrylovOp<T, true> { using type = Sten64; };
 template <typename T, bool PC>
-__device__ __forceinline__ typename KrylovOp<T, PC>::type krylov_op(const InstDev &I) {
+__device__ __forceinline__ typename KrylovOp<T, PC>::type krylov_op(CInst &I) {
   if constexpr (PC) return Sten64(I);
   else return Sten<T, 5>(I.lev[0]);
 }
@@ -1506,7 +1506,7 @@ __global__ void __launch_bounds__(kBlock) k_bicg_v(const Insts insts,
                                                   const BlkMap *__restrict__ map) {
   using V32 = typename Pick<PC, T>::type;
   const BlkMap m = map[blockIdx.x];
-  const InstDev &I = insts[m.inst];
+  CInst &I = insts[m.inst];
   auto A = krylov_op<T, PC>(I);
   const V32 *ph = PC ? (const V32 *)I.pv[PV_PH - kNumVec] : (const V32 *)I.kv[VPH];
   const V32 *rhp = PC ? (const V32 *)I.pv[PV_RH - kNumVec] : (const V32 *)I.kv[VRH];
@@ -1538,7 +1538,7 @@ __global__ void __launch_bounds__(kBlock) k_bicg_s(const Insts insts,
     const int bi = kLightBlocks * blockIdx.x + e;
     if (bi >= nmap) break;
     const BlkMap m = map[bi];
-    const InstDev &I = insts[m.inst];
+    CInst &I = insts[m.inst];
     if (status_of(insts, m.inst) != ST_ACTIVE) continue;   // uniform over the workgroup
     const int K = m.k0 + threadIdx.x;
     const int N = I.nx * I.ny;
@@ -1560,7 +1560,7 @@ __global__ void __launch_bounds__(kBlock) k_bicg_t(const Insts insts,
                                                   const BlkMap *__restrict__ map) {
   using V32 = typename Pick<PC, T>::type;
   const BlkMap m = map[blockIdx.x];
-  const InstDev &I = insts[m.inst];
+  CInst &I = insts[m.inst];
   auto A = krylov_op<T, PC>(I);
   const V32 *sh = PC ? (const V32 *)I.pv[PV_SH - kNumVec] : (const V32 *)I.kv[VSH];
   const T *sp = cptr<T>(I.kv[VS]);
@@ -1592,7 +1592,7 @@ __global__ void __launch_bounds__(kBlock) k_bicg_x(const Insts insts,
                                                   const BlkMap *__restrict__ map) {
   using V32 = typename Pick<PC, T>::type;
   const BlkMap m = map[blockIdx.x];
-  const InstDev &I = insts[m.inst];
+  CInst &I = insts[m.inst];
   T *xp = XSTATE ? (T *)I.x : ptr<T>(I.kv[VXK]);
   const V32 *php = PC ? (const V32 *)I.pv[PV_PH - kNumVec] : (const V32 *)I.kv[VPH];
   const V32 *shp = PC ? (const V32 *)I.pv[PV_SH - kNumVec] : (const V32 *)I.kv[VSH];
@@ -1636,7 +1636,7 @@ __global__ void __launch_bounds__(kBlock) k_bicg_x(const Insts insts,
 __global__ void __launch_bounds__(kBlock) k_ir_residual(const Insts insts,
                                                        const BlkMap *__restrict__ map) {
   const BlkMap m = map[blockIdx.x];
-  const InstDev &I = insts[m.inst];
+  CInst &I = insts[m.inst];
   Sten64 M(I);
   int ost = ostatus_of(insts, m.inst);
   M.hold();
@@ -1660,7 +1660,7 @@ __global__ void __launch_bounds__(kBlock) k_ir_residual(const Insts insts,
 __global__ void __launch_bounds__(kBlock) k_ir_inner_init(const Insts insts,
                                                          const BlkMap *__restrict__ map) {
   const BlkMap m = map[blockIdx.x];
-  const InstDev &I = insts[m.inst];
+  CInst &I = insts[m.inst];
   if (ostatus_of(insts, m.inst) != ST_ACTIVE) return;
   const int K = m.k0 + threadIdx.x;
   const int N = I.nx * I.ny;
@@ -1681,7 +1681,7 @@ __global__ void __launch_bounds__(kBlock) k_ir_inner_init(const Insts insts,
 __global__ void __launch_bounds__(kBlock) k_ir_update(const Insts insts,
                                                      const BlkMap *__restrict__ map) {
   const BlkMap m = map[blockIdx.x];
-  const InstDev &I = insts[m.inst];
+  CInst &I = insts[m.inst];
   if (ostatus_of(insts, m.inst) != ST_ACTIVE) return;
   const int K = m.k0 + threadIdx.x;
   if (K >= I.nx * I.ny) return;
@@ -1704,7 +1704,7 @@ __device__ __forceinline__ bool solve_ended(int prec, int status, int ostatus) {
 __global__ void __launch_bounds__(kBlock) k_finalize(const Insts insts,
                                                     const BlkMap *__restrict__ map) {
   const BlkMap m = map[blockIdx.x];
-  const InstDev &I = insts[m.inst];
+  CInst &I = insts[m.inst];
   Sten64 M(I);
   int phase = phase_of(insts, m.inst), st = status_of(insts, m.inst), ost = ostatus_of(insts, m.inst);
   int prec = I.prec;
@@ -1754,7 +1754,7 @@ __global__ void __launch_bounds__(kBlock) k_finalize(const Insts insts,
 __global__ void __launch_bounds__(kBlock) k_commit(const Insts insts,
                                                   const BlkMap *__restrict__ map) {
   const BlkMap m = map[blockIdx.x];
-  const InstDev &I = insts[m.inst];
+  CInst &I = insts[m.inst];
   if (phase_of(insts, m.inst) != 1 || ostatus_of(insts, m.inst) != ST_DONE) return;   // uniform
   const int K = m.k0 + threadIdx.x;
   const bool hist = rsc(I)->hist;   // df holds an earlier increment (uniform)
@@ -1781,7 +1781,7 @@ __global__ void __launch_bounds__(kBlock) k_commit(const Insts insts,
 enum Finish { F_INIT64 = 0, F_V, F_S, F_T, F_X, F_IR_RES, F_INNER_INIT, F_FINALIZE, F_EXTRAP };
 
 template <typename A, int NV>
-__device__ __forceinline__ void sum_partials(const InstDev &I, A (&tot)[NV]) {
+__device__ __forceinline__ void sum_partials(CInst &I, A (&tot)[NV]) {
   // Thread t adds partials t, t + kFinThreads, .. in that order; the loads of
   // 8 of them are issued before they are added, so a large instance (65536
   // partials at 4096^2) costs a few memory latencies, not one per partial.
@@ -1816,7 +1816,7 @@ __global__ void __launch_bounds__(kFinThreads) k_finish(const Insts insts, int n
                                                   int *__restrict__ cnt) {
   const int k = blockIdx.x;
   if (k >= n) return;
-  const InstDev &I = insts[k];
+  CInst &I = insts[k];
   KScal &s = *I.sc;
   const int st = s.status, ost = s.ostatus;
   if (MODE == F_IR_RES || MODE == F_INNER_INIT) {

@@ -23,8 +23,8 @@ template <typename T, int NB, bool ZERO, int DIR> struct Lines {
   const T *b, *lo, *inv, *cu, *om, *op, *omm, *omp, *opm, *opp;
   int nx, ny, st;
   __device__ __forceinline__ Lines(const Insts &insts, int inst, int l, int xid, int bid) {
-    const InstDev &I = insts[inst];
-    const Lev &L = I.lev[l];
+    CInst &I = insts[inst];
+    CLev &L = I.lev[l];
     level_xb<T>(I, l, xid, bid, x, b);
     lo = cptr<T>(L.band[DIR == 0 ? BW : BS]);
     inv = cptr<T>(L.linv[DIR]);
