@@ -60,9 +60,14 @@ template <int L, int C> constexpr int col_lds() { return 4 * (L * C / 64) * L; }
 // grid (FP32) 56 -> 13.4 us, its coarser columns 18.8 -> 7.2; 4096 steps
 // 131 -> 94 us; 2048 steps FP64 106 -> 41 us; the 9-point columns of a batch of
 // 48 uneven grids 14.4 -> 6.8 us, its 5-point ones 34.5 -> 16.5.
-// Run lengths: K steps of three values each must fit the registers; 4096 steps
+// Run lengths: K steps of three values each are held in registers; 4096 steps
 // as 8 columns x 64 runs of 64 took 94 us, as 4 columns x 128 runs of 32 (16
-// byte pieces of a row) 158.
+// byte pieces of a row) 158. A kernel holds every run length of its range in one
+// body and so has the registers of the longest for all of them (9-point, not from
+// zero): k_cols 127 VGPRs in FP32 (4 waves per SIMD) and 234 in FP64 (2, one
+// workgroup per CU), where runs of 8 steps alone need 66 and 98; k_cols_long 256
+// with 25 (FP32) and 32 (FP64) of them spilled to scratch, where no run length
+// alone spills.
 template <typename T, int NB, bool ZERO, int L, int C, int K>
 __device__ __forceinline__ void col_sweep(const Lines<T, NB, ZERO, 1> &P, const LineGrp gr, T *lds) {
   constexpr int NW = L * C / 64;   // waves
